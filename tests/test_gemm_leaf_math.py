@@ -517,3 +517,25 @@ def test_checked_binary16_held_leaves_10bit():
         assert _bits(got) == _bits(ref), (a, b, acc, hs, got, ref)
         checked += 1
     assert checked > 1500 and flagged > 50 and differ_flagged > 0, (checked, flagged, differ_flagged)
+
+
+@pytest.mark.parametrize("neg_form", [False, True])
+def test_rto_pick_is_the_odd_neighbour(neg_form):
+    """Choosing the directed rounding whose pattern is odd (by a mask from one pattern's last
+    bit) gives RTO24's pattern as test_directed_rounding_leaves builds it: the value itself
+    when exact, else the smaller pattern with its last bit set; for an exact zero the form's
+    own zero.  Over adjacent magnitudes of both signs up to infinity, exact values and zeros."""
+    g = np.random.default_rng(77)
+    n = np.concatenate([np.arange(0, 70), 0x7F7FFFFF - np.arange(0, 70),
+                        (np.arange(1, 255)[:, None] * (1 << 23) + np.arange(-3, 3)).ravel(),
+                        g.integers(0, 0x7F7FFFFF, 200000)]).astype(np.uint32)
+    sign = np.uint32(0x80000000)
+    d = np.concatenate([n, sign | (n + 1), n, sign | n, [sign]]).astype(np.uint32)
+    u = np.concatenate([n + 1, sign | n, n, sign | n, [0]]).astype(np.uint32)
+    zero = np.uint32(0) if neg_form else sign          # an exact zero: u, or d
+    ref = np.where(d == u, d, np.minimum(d, u) | np.uint32(1))
+    ref[-1] = zero
+    odd, even = (d, u) if neg_form else (u, d)
+    mask = ((odd << np.uint32(31)).view(np.int32) >> 31).view(np.uint32)
+    got = (odd & mask) | (even & ~mask)
+    assert np.array_equal(got, ref)
