@@ -14,6 +14,7 @@ sizes are kept small so the file runs in seconds."""
 import math
 
 import numpy as np
+import pytest
 
 import oracle
 
