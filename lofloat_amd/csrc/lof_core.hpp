@@ -28,6 +28,14 @@ __host__ __device__ constexpr bool uses_len(int m) {
     return m == SRA || m == SRB || m == SRC || m == SRD;
 }
 
+// Workgroup barrier for LDS data.  The wait for the wave's own LDS stores is written out:
+// hipcc (ROCm 7.2) dropped the one __syncthreads() stands for wherever the barrier heads a loop
+// and the stores end its body -- the assembly had ds_write ... s_barrier with no s_waitcnt
+// between -- so another wave could read the buffer before the last stores had landed.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // Everything a kernel needs for virtual_round(x, FloatingPointParams, ProjSpec),
 // precomputed on the host (make_fmt_dev).
 struct FmtDev {

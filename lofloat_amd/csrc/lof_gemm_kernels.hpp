@@ -346,7 +346,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int tile_m, int til
                 v = gld(g.tb ? g.B + (int64_t)gn * g.ldb + gk : g.B + (int64_t)gk * g.ldb + gn);
             Bs[k * LDB_S + n] = v;
         }
-        __syncthreads();
+        lds_barrier();
         const int kmax = min(BK, g.K - k0);
         for (int kk = 0; kk < kmax; ++kk) {
             float a[TM], b[TN];
@@ -384,7 +384,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int tile_m, int til
                 }
             }
         }
-        __syncthreads();
+        lds_barrier();
     }
     if (in_chunk != 0) {   // short last chunk
         double pd[TM * TN];

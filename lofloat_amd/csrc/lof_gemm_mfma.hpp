@@ -815,7 +815,7 @@ __device__ __forceinline__ void gemm_tile_mfma(const GemmArgs& g, int tile_m, in
     for (int k0 = 0; k0 < g.K; k0 += BK, buf ^= 1) {
         // Slice k0 and its statistics are in LDS buffer `buf`; every wave is done with the
         // other buffer (slice k0 - 32), which the store below refills.
-        __syncthreads();
+        lds_barrier();
         const float* As = smem + buf * (T::BUF_FLOATS + T::STAT_WORDS);
         const float* Bs = As + BK * LDA_S;
         const uint32_t* stat = (const uint32_t*)(Bs + BK * LDB_S);

@@ -145,9 +145,9 @@ __global__ __launch_bounds__(256, C::mfma_wnb == 2 ? 3 : 2) void k_grouped(const
     const int tid = threadIdx.x;
     for (;;) {
         if (tid == 0) s_tile = atomicAdd(&counters[0], 1ull);
-        __syncthreads();
+        lds_barrier();
         const int64_t t = (int64_t)__builtin_amdgcn_readfirstlane((int)(s_tile & 0x7FFFFFFF));
-        __syncthreads();
+        lds_barrier();
         if (t >= total) break;
         int lo = 0, hi = ntasks - 1;
         while (lo < hi) {
@@ -176,7 +176,7 @@ __global__ __launch_bounds__(256, C::mfma_wnb == 2 ? 3 : 2) void k_grouped(const
             else
                 gemm_tile<C::bm, C::bn, C::tm, C::tn, C::bk, false>(
                     T.g, (int)(local / T.tiles_n), (int)(local % T.tiles_n), tid, smem);
-            __syncthreads();  // smem reuse by the next tile
+            lds_barrier();  // smem reuse by the next tile
             break;
         }
     }

@@ -125,7 +125,7 @@ __global__ __launch_bounds__(kPackTPB) void k_pack_encode(PackArgs a) {
             put(q, r);
         }
     }
-    __syncthreads();
+    lds_barrier();
     // Thread t packs slots 32t .. 32t+31 (whole groups: gc divides 32), i.e. words
     // t*n .. t*n+n-1 of the tile.  The bit cursor is the same in every lane, so its branches
     // are scalar.  The words go back into the same LDS (after a barrier), then out coalesced.
@@ -133,7 +133,7 @@ __global__ __launch_bounds__(kPackTPB) void k_pack_encode(PackArgs a) {
     uint4 v[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = reinterpret_cast<const uint4*>(slot_rep)[tid * 4 + i];
-    __syncthreads();
+    lds_barrier();
     uint32_t* wbuf = reinterpret_cast<uint32_t*>(slot_rep);   // 4096 words >= 256 * n
     uint32_t cur = 0u;
     int filled = 0, wo = tid * n;
@@ -151,7 +151,7 @@ __global__ __launch_bounds__(kPackTPB) void k_pack_encode(PackArgs a) {
             cur = rep >> (n - filled);   // the bits of rep past the word's end (0 if none)
         }
     }
-    __syncthreads();
+    lds_barrier();
     const int64_t wbase = (int64_t)blockIdx.x * (kPackTPB * n);
     for (int j = 0; j < n; ++j) {
         const int wl = j * kPackTPB + tid;          // word of the tile
@@ -204,7 +204,7 @@ __global__ __launch_bounds__(kPackTPB) void k_pack_decode(PackArgs a) {
         }
     }
     if (tid == 0) words[kPackTPB * n] = 0u;
-    __syncthreads();
+    lds_barrier();
     const int64_t tbase = (int64_t)blockIdx.x * kTile;
     uint32_t* out = RAW ? a.repsout : reinterpret_cast<uint32_t*>(a.dstf);
     const bool full = a.vec && tbase + kTile <= a.count;

@@ -62,7 +62,7 @@ __global__ __launch_bounds__(kSiluTPB) void k_pwl_silu(SiluArgs a) {
     const int tid = threadIdx.x;
     const int N = a.segments;
     for (int j = tid; j <= N; j += kSiluTPB) tab[j] = a.lut[j];
-    __syncthreads();
+    lds_barrier();
     const T* in = static_cast<const T*>(a.in);
     T* out = static_cast<T*>(a.out);
     constexpr int V = 16 / (int)sizeof(T);         // elements per 16-byte vector
