@@ -113,6 +113,7 @@ LOF_API lof_status lof_conv2d_f32(const lof_conv2d_desc* desc, int32_t config,
     GemmArgs g;
     lof_status s = prepare_gemm(&d, &g);
     if (s != LOF_OK) return s;
+    set_chain(&g, true);
     const int l2 = log2_chunk(g.chunk);
     if (l2 < 0)
         return set_error(LOF_ERR_UNSUPPORTED,
@@ -137,6 +138,7 @@ LOF_API lof_status lof_conv2d_f32(const lof_conv2d_desc* desc, int32_t config,
     // binary16-held / packed binary16 / directed-rounding / mixed-precision FMA leaves off,
     // 0x10000 the bf16 MFMA chunk sums off
     if (config >= 0) {
+        if (config & ~0xFF) g.chain = -1;   // these paths are the tiles' below
         if (config & 0x800) g.sum_off |= 1;
         if (config & 0x1000) g.sum_off |= 2;
         if (config & 0x2000) g.sum_off |= 4;
@@ -189,6 +191,14 @@ LOF_API lof_status lof_conv2d_f32(const lof_conv2d_desc* desc, int32_t config,
         cv.sdb = (int64_t)P * Q * c.K;
         cv.sdm = 1;
         cv.sdpq = c.K;
+    }
+    if (g.chain >= 0) {
+        int t = 1;
+        if (cfg < 0) {
+            t = chain_default_tile(c.K, Ncols);
+            if (t == 4) t = 2;
+        }
+        return launch_chain(g, t, (hipStream_t)stream, "lof_conv2d_f32 launch");
     }
     const int bm = tile ? 128 : 64, bn = 64;
     const dim3 grid((unsigned)((Ncols + bn - 1) / bn), (unsigned)((c.K + bm - 1) / bm));

@@ -10,6 +10,7 @@
 #include <tuple>
 
 #include "lof_gemm.hpp"
+#include "lof_gemm_chain_table.hpp"
 #include "lof_host.hpp"
 
 namespace lofamd {
@@ -26,11 +27,11 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs g) {
 // Occupancy: the 64x64 tile is held to 128 registers (4 waves per SIMD; chunk 1 spills a
 // few), the 64x128 tile to 168 (3 waves): both are latency-bound, and a 4096^2 output's
 // 4096 64x64 tiles then fill 1024 slots in exactly four rounds.
-template <int WMB, int WNB, int CHUNK, bool SUBN, bool DRC = false>
+template <int WMB, int WNB, int CHUNK, bool SUBN>
 __global__ __launch_bounds__(256, (WMB == 1 && WNB == 1) ? 4 : (WMB == 1 && WNB == 2) ? 3 : 1)
 void k_gemm_mfma(GemmArgs g) {
     __shared__ __align__(16) float smem[MfmaTile<WMB, WNB>::SMEM_FLOATS];
-    gemm_tile_mfma<WMB, WNB, CHUNK, SUBN, false, DRC>(g, (int)blockIdx.y, (int)blockIdx.x,
+    gemm_tile_mfma<WMB, WNB, CHUNK, SUBN>(g, (int)blockIdx.y, (int)blockIdx.x,
                                                       (int)threadIdx.x, smem);
 }
 
@@ -41,26 +42,20 @@ struct GemmConfig {
     int bm, bn;
     GemmKernel kernel[2];          // VALU tile, any chunk: [subn]
     GemmKernel mfma[6][2];         // wave tile: [log2(chunk)][subn], chunk in {1, 2, ..., 32}
-    // wave tile with directed-rounding chunk leaves, chunks 8-32: [log2(chunk) - 3] (nullptr
-    // where the tile has none), for the chunk sums of mantissa-only accumulators of 20 or more
-    // bits, which have no other fast leaf.  For narrower accumulators they measured no faster
-    // than the TwoSum round-to-odd leaves (8e7m operands) and 30 % slower on exact sums.
-    GemmKernel drc[3];
 };
 
 #define LOF_GEMM_CFG(BM, BN, TM, TN, BK)                                                    \
     {#BM "x" #BN "/" #TM "x" #TN "/k" #BK, BM, BN,                                           \
-     {k_gemm<BM, BN, TM, TN, BK, false>, k_gemm<BM, BN, TM, TN, BK, true>}, {}, {}}
+     {k_gemm<BM, BN, TM, TN, BK, false>, k_gemm<BM, BN, TM, TN, BK, true>}, {}}
 #define LOF_MFMA_PAIR(WMB, WNB, C) {k_gemm_mfma<WMB, WNB, C, false>, k_gemm_mfma<WMB, WNB, C, true>}
 #define LOF_MFMA_TABLE(WMB, WNB)                                                            \
     {LOF_MFMA_PAIR(WMB, WNB, 1), LOF_MFMA_PAIR(WMB, WNB, 2), LOF_MFMA_PAIR(WMB, WNB, 4),      \
      LOF_MFMA_PAIR(WMB, WNB, 8), LOF_MFMA_PAIR(WMB, WNB, 16), LOF_MFMA_PAIR(WMB, WNB, 32)}
 #define LOF_GEMM_MFMA_CFG(WMB, WNB)                                                         \
-    {"mfma" #WMB #WNB, 64 * WMB, 64 * WNB, {nullptr, nullptr}, LOF_MFMA_TABLE(WMB, WNB), {}}
-#define LOF_GEMM_MFMA_DRC_CFG(WMB, WNB)                                                     \
-    {"mfma" #WMB #WNB, 64 * WMB, 64 * WNB, {nullptr, nullptr}, LOF_MFMA_TABLE(WMB, WNB),      \
-     {k_gemm_mfma<WMB, WNB, 8, false, true>, k_gemm_mfma<WMB, WNB, 16, false, true>,          \
-      k_gemm_mfma<WMB, WNB, 32, false, true>}}
+    {"mfma" #WMB #WNB, 64 * WMB, 64 * WNB, {nullptr, nullptr}, LOF_MFMA_TABLE(WMB, WNB)}
+// a tile of the chunk-sum kernels alone: other products asked to run on it take mfma11
+#define LOF_GEMM_SHORT_CFG(BM, BN)                                                          \
+    {"mfma" #BM "x" #BN, BM, BN, {nullptr, nullptr}, LOF_MFMA_TABLE(1, 1)}
 
 const GemmConfig kConfigs[] = {
     LOF_GEMM_CFG(64, 64, 4, 4, 16),
@@ -70,18 +65,21 @@ const GemmConfig kConfigs[] = {
     LOF_GEMM_CFG(32, 32, 2, 2, 32),
     LOF_GEMM_MFMA_CFG(2, 2),
     LOF_GEMM_MFMA_CFG(2, 1),
-    LOF_GEMM_MFMA_DRC_CFG(1, 1),
-    LOF_GEMM_MFMA_DRC_CFG(1, 2),
+    LOF_GEMM_MFMA_CFG(1, 1),
+    LOF_GEMM_MFMA_CFG(1, 2),
+    LOF_GEMM_SHORT_CFG(32, 32),
+    LOF_GEMM_SHORT_CFG(16, 64),
+    LOF_GEMM_SHORT_CFG(64, 16),
 };
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
-constexpr int kMfma64 = 7, kMfma64x128 = 8;
+constexpr int kFirstMfma = 5, kMfma64 = 7, kMfma64x128 = 8, kFirstShort = 9;
 
 // chunks whose sums can run on MFMA
 bool chunk_fits_mfma(int chunk) { return chunk >= 2 && chunk <= 32 && (32 % chunk) == 0; }
 // chunks the wave tiles (MFMA configs) take: those, and chunk 1 on VALU
 bool chunk_fits_wave_tile(int chunk) { return chunk == 1 || chunk_fits_mfma(chunk); }
 
-bool is_mfma(int config) { return kConfigs[config].kernel[0] == nullptr; }
+bool is_mfma(int config) { return config >= kFirstMfma; }
 
 bool config_valid(int config, int chunk) {
     return config >= 0 && config < kNumConfigs &&
@@ -91,7 +89,6 @@ bool config_valid(int config, int chunk) {
 GemmKernel pick_kernel(const GemmConfig& c, const GemmArgs& g) {
     if (c.kernel[0]) return c.kernel[g.subn ? 1 : 0];
     const int l2 = 31 - __builtin_clz((unsigned)g.chunk);
-    if (l2 >= 3 && c.drc[0] && g.dr_kind == 1 && g.range_f == 0u) return c.drc[l2 - 3];
     return c.mfma[l2][g.subn ? 1 : 0];
 }
 
@@ -132,6 +129,48 @@ int default_config(const lof_gemm_desc& d) {
 }
 
 }  // namespace
+
+void set_chain(GemmArgs* g, bool conv) {
+    g->chain = -1;
+    if (!chunk_fits_mfma(g->chunk) || g->acc_mode != RNE || g->lda > kChainMaxLd ||
+        (!conv && g->ldb > kChainMaxLd))
+        return;
+    if (g->sum_f16) {
+        g->chain = kChainHalf;
+        g->half_top = std::ldexp(1.0f, g->sum_ehi);
+    } else if (g->acc_kind == 0 && g->acc_r < 23) {   // 0 bits: rounding can lose a NaN's sign
+        g->chain = g->acc_r == 0 ? kChainMant23 : kChainMant;
+    }
+}
+
+// Short dimensions take the tile that wastes least of them; else 64x64 from 768 tiles (three a
+// CU) on and 32x32 below, where 64x64 leaves CUs idle or unevenly loaded.  Measured (us, chunk
+// 32 / 8, 23 / 10 bits): 2048x2048x2048, 1024 tiles, 64x64 178 / 364, 32x32 244 / 410;
+// 2048x1024x4096, 512 tiles, 226 / 458 against 241 / 408; 1000x768x3072, 192 tiles, 189 / 322
+// against 98 / 156.  8x4096x4096: 16x64 86 / 151, 32x32 106 / 171.  128x128 ties with 64x64 on the
+// largest products and loses below 1024 tiles of its own.
+int chain_default_tile(int64_t M, int64_t N) {
+    if (M <= 16) return 3;
+    if (N <= 16) return 4;
+    return ((M + 63) / 64) * ((N + 63) / 64) >= 768 ? 1 : 2;
+}
+
+lof_status launch_chain(const GemmArgs& g, int tile, hipStream_t st, const char* what) {
+    const ChainTable& t = g.chain == kChainHalf     ? kChainTableHalf
+                          : g.chain == kChainMant23 ? kChainTableMant23
+                                                    : kChainTableMant;
+    const int l2 = 30 - __builtin_clz((unsigned)g.chunk);   // log2(chunk) - 1
+    ChainKernel k = g.cv.conv ? t.conv[tile][l2] : t.gemm[tile][l2];
+    if (!k) {   // a chunk of 2 on a 16-row block, whose MFMA takes 4 k
+        tile = 1;
+        k = g.cv.conv ? t.conv[tile][l2] : t.gemm[tile][l2];
+    }
+    const ChainDims& d = kChainDims[tile];
+    const int64_t tm = (g.M + d.bm - 1) / d.bm, tn = (g.N + d.bn - 1) / d.bn;
+    if (tm * tn > 0x7FFFFFFF) return set_error(LOF_ERR_UNSUPPORTED, "%s: output too large", what);
+    hipLaunchKernelGGL(k, dim3((unsigned)(tm * tn)), dim3(256), 0, st, g, (unsigned)tm, (unsigned)tn);
+    return check_hip(hipGetLastError(), what);
+}
 
 void set_fast_path(GemmArgs* g, bool on, int m) {
     g->fast = on ? 1 : 0;
@@ -272,6 +311,7 @@ lof_status prepare_gemm(const lof_gemm_desc* d, GemmArgs* g) {
     g->dr_lsb = g->dr_rf > 0 ? 1u : 0u;
     g->dr_mask = ~((1u << g->dr_rf) - 1u);
     g->mfma_bf16 = 1;
+    set_chain(g, false);
     return LOF_OK;
 }
 
@@ -281,7 +321,9 @@ lof_status launch_gemm(const GemmArgs& g, int config, hipStream_t st) {
         return set_error(LOF_ERR_UNSUPPORTED,
                          "lof_gemm_f32: config %d needs a chunk in {1, 2, 4, 8, 16, 32} (got %d)",
                          config, g.chunk);
-    const GemmConfig& c = kConfigs[config];
+    if (is_mfma(config) && g.chain >= 0)
+        return launch_chain(g, kChainTileOf[config - kFirstMfma], st, "lof_gemm_f32 launch");
+    const GemmConfig& c = kConfigs[config >= kFirstShort ? kMfma64 : config];
     dim3 grid((unsigned)((g.N + c.bn - 1) / c.bn), (unsigned)((g.M + c.bm - 1) / c.bm));
     if (grid.y > 65535u) return set_error(LOF_ERR_UNSUPPORTED, "lof_gemm_f32: M too large");
     hipLaunchKernelGGL(pick_kernel(c, g), grid, dim3(256), 0, st, g);
@@ -297,7 +339,9 @@ int resolve_gemm_config(const lof_gemm_desc& d, int config) {
     if (config >= 0) return config;
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tuned.find(tune_key(d));
-    return it != g_tuned.end() ? it->second : default_config(d);
+    if (it != g_tuned.end()) return it->second;
+    return chunk_fits_mfma(d.accum.chunk) ? kChainConfigOf[chain_default_tile(d.M, d.N)]
+                                          : default_config(d);
 }
 
 }  // namespace lofamd
@@ -320,6 +364,8 @@ LOF_API lof_status lof_gemm_f32(const lof_gemm_desc* desc, int32_t config, lof_s
     // exact-sum leaves off, 0x1000 its RTO leaves, 0x2000 its binary16-held chunk-1 leaves,
     // 0x4000 only their packed binary16 form, 0x8000 the directed-rounding chunk-1 leaves,
     // 0x10000 the bf16 MFMA chunk sums (exact chunks of 8 to 32 then use the VALU chain)
+    // -- any of them on the tiles below, which hold those paths, instead of the chunk-sum kernels
+    if (config >= 0 && (config & ~0xFF)) g.chain = -1;
     if (config >= 0 && (config & 0x800)) g.sum_off |= 1;
     if (config >= 0 && (config & 0x1000)) g.sum_off |= 2;
     if (config >= 0 && (config & 0x2000)) g.sum_off |= 4;
@@ -383,6 +429,8 @@ LOF_API lof_status lof_gemm_autotune(const lof_gemm_desc* desc, int32_t iters,
     const bool wave = chunk_fits_wave_tile(g.chunk);
     for (int c = 0; c < kNumConfigs && s == LOF_OK; ++c) {
         if (!config_valid(c, g.chunk) || is_mfma(c) != wave) continue;
+        if (c >= kFirstShort && g.chain < 0) continue;   // would time mfma11 again
+        if (g.chain >= 0 && (c == 6 || c == 8)) continue;
         s = launch_gemm(g, c, st);  // warm-up
         if (s != LOF_OK) break;
         (void)hipEventRecord(e0, st);

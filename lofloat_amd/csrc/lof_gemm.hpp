@@ -11,6 +11,12 @@ namespace lofamd {
 
 lof_status prepare_gemm(const lof_gemm_desc* d, GemmArgs* g);
 void set_fast_path(GemmArgs* g, bool on, int m);
+// Whether the chunk-sum kernels take this product (g->chain); `conv`: B is gathered, not read
+// through ldb.  prepare_gemm calls it for a stored B.
+void set_chain(GemmArgs* g, bool conv);
+// Tile of the chunk-sum kernels for an M x N product, and its launch.
+int chain_default_tile(int64_t M, int64_t N);
+lof_status launch_chain(const GemmArgs& g, int tile, hipStream_t st, const char* what);
 lof_status launch_gemm(const GemmArgs& g, int config, hipStream_t st);
 int resolve_gemm_config(const lof_gemm_desc& d, int config);
 int gemm_num_configs();

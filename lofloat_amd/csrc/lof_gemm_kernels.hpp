@@ -146,6 +146,8 @@ struct GemmArgs {
     int32_t mfma_mode;   // MFMA tile: 0 exactness test, 1 every chunk on the VALU chain,
                          // 2 every chunk on MFMA (testing only: skips the test)
     int32_t mfma_bf16;   // exact chunk sums of bfloat16-valued slices on the bf16 MFMAs
+    int32_t chain;       // ChainKind of the chunk-sum kernels (lof_gemm_chain.hpp), -1: none
+    float half_top;      // kChainHalf: results from here up take the general leaf
     ConvGeom cv;         // wave tiles only: B gathered from an activation (cv.conv != 0)
 };
 
