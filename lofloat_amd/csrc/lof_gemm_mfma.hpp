@@ -58,20 +58,30 @@ __device__ __forceinline__ bf16x8 lds_bf16x8(const float* p, int stride) {
     return __builtin_bit_cast(bf16x8, v);
 }
 
+// Wave reductions on DPP operands (row shifts by 1, 2, 4 and 8, then the row broadcasts of lanes
+// 15 and 31): six VALU instructions with no LDS round trip, the result in lane 63 only.
+// Lanes without a source keep `id`, the operation's identity.
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t v, uint32_t id) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)id, (int)v, CTRL, ROWS, 0xF, false);
+}
+template <class Op>
+__device__ __forceinline__ uint32_t wave_last_u32(uint32_t v, uint32_t id, Op op) {
+    v = op(v, dpp_u32<0x111>(v, id));
+    v = op(v, dpp_u32<0x112>(v, id));
+    v = op(v, dpp_u32<0x114>(v, id));
+    v = op(v, dpp_u32<0x118>(v, id));
+    v = op(v, dpp_u32<0x142, 0xA>(v, id));
+    return op(v, dpp_u32<0x143, 0xC>(v, id));
+}
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, o, 64));
-    return v;
+    return wave_last_u32(v, 0u, [](uint32_t a, uint32_t b) { return max(a, b); });
 }
 __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = min(v, (uint32_t)__shfl_xor((int)v, o, 64));
-    return v;
+    return wave_last_u32(v, ~0u, [](uint32_t a, uint32_t b) { return min(a, b); });
 }
 __device__ __forceinline__ uint32_t wave_or_u32(uint32_t v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v |= (uint32_t)__shfl_xor((int)v, o, 64);
-    return v;
+    return wave_last_u32(v, 0u, [](uint32_t a, uint32_t b) { return a | b; });
 }
 
 // The float leaf's slow path: the exact-zero leaf, else the general leaf (the double fast
@@ -722,7 +732,7 @@ __device__ __forceinline__ void gemm_tile_mfma(const GemmArgs& g, int tile_m, in
             sa.key = wave_min_u32(sa.key);
             sb.key = wave_min_u32(sb.key);
         }
-        if (lane == 0) {
+        if (lane == 63) {   // where the reductions end
             uint32_t* st = stat + wave * 8;
             st[0] = sa.amax; st[1] = sa.mnk; st[2] = sa.orb;
             st[3] = sb.amax; st[4] = sb.mnk; st[5] = sb.orb;
@@ -843,7 +853,9 @@ __device__ __forceinline__ void gemm_tile_mfma(const GemmArgs& g, int tile_m, in
         // round to nearest-even at 11 significant bits):
         //   binary16-shaped format: hs = 0 (its own grid; sum_ehi is 15);
         //   10-bit mantissa-only:   hs = 15 - S, which needs Lf + hs >= -24, i.e.
-        //                           S - Lf <= 39, and b 2^hs FP32-normal for every nonzero b.
+        //                           S - Lf <= 39, and b 2^hs FP32-normal for every nonzero b;
+        //                           the sums need not be exact in FP32 (e5m2 gradients times
+        //                           e4m3 weights are not).
         //
         // When every A value and every scaled B value is a binary16 value as well, the
         // binary16 FMA h <- binary16(-a (b 2^hs) + h) computes the same leaf, two outputs'
@@ -893,16 +905,8 @@ __device__ __forceinline__ void gemm_tile_mfma(const GemmArgs& g, int tile_m, in
             }
             if constexpr (CHUNK == 1) {
               if (try_fast) {
-                if (sum_ok && !(g.sum_off & 4)) {
-                    if (f16) {
-                        h_ok = true;
-                    } else if (g.sum_h10) {
-                        hs = 15 - S;
-                        h_ok = S - Lf <= 39 && bLsb + hs >= -126 && bTop + 1 + hs <= 127;
-                    }
-                    pk_ok = h_ok && a16 && bW <= 11 && bLsb + hs >= -24 && bTop + hs <= 15 &&
-                            !(g.sum_off & 8);
-                }
+                if (sum_ok && f16 && !(g.sum_off & 4)) h_ok = true;
+                pk_ok = h_ok && a16 && bW <= 11 && bLsb >= -24 && bTop <= 15 && !(g.sum_off & 8);
                 // binary16-shaped format on RTO lanes (sums below 2^15, maybe inexact in
                 // FP32): the binary16 FMA rounds the exact sum once, which is what rounding
                 // the reference's RTO24 sum to 11 significant bits gives
@@ -913,7 +917,22 @@ __device__ __forceinline__ void gemm_tile_mfma(const GemmArgs& g, int tile_m, in
                 }
               }
             }
-            dr_ok = try_dr && !sum_ok && !pk_ok && amax <= 0x7F800000u &&
+            // 10-bit mantissa-only: the held leaves need no FP32-exact product or sum, since both
+            // FMAs round the exact h - a b 2^hs once; only that every scaled sum stays on
+            // binary16's 2^-24 grid (S - Lf <= 39) and FP32-normal unscaled (Lf >= -126)
+            if constexpr (CHUNK == 1) {
+                if (sfin && g.sum_h10 && g.range_f != 0u && !(g.sum_off & 4) && S <= g.sum_ehi &&
+                    S - Lf <= 39 && Lf >= -126) {
+                    const int h10 = 15 - S;
+                    if (bLsb + h10 >= -126 && bTop + 1 + h10 <= 127) {
+                        h_ok = true;
+                        hs = h10;
+                        pk_ok = a16 && bW <= 11 && bLsb + hs >= -24 && bTop + hs <= 15 &&
+                                !(g.sum_off & 8);
+                    }
+                }
+            }
+            dr_ok = try_dr && !sum_ok && !pk_ok && !h_ok && amax <= 0x7F800000u &&
                     (g.dr_kind == 1 || S <= g.sum_ehi);
             // chunk 1, binary16-shaped accumulator, every sum below 2^15: the held leaves with
             // the mixed FMA (mix_fnma16) round the exact a b + h once, so they take the lanes
