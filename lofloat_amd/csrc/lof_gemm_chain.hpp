@@ -15,7 +15,7 @@
 //
 // The leaf takes any finite p and acc with no test:
 //   mantissa-only, 1..22 bits   the two directed roundings of p + acc, of which the odd one is
-//                               RTO24's result (rto_pick), then round-to-nearest-even at a fixed
+//                               RTO24's result (rto_fma16), then round-to-nearest-even at a fixed
 //                               bit of the pattern: 7 instructions;
 //   mantissa-only, 23 bits      the odd one is the result: 4 instructions;
 //   binary16-shaped             one mixed-precision FMA, which rounds the exact -acc - p once to
@@ -81,63 +81,84 @@ __device__ __forceinline__ float4 gld4u(const float* p) {
     return make_float4(v.x, v.y, v.z, v.w);
 }
 
-// rd / ru: the two directed roundings of acc[o] + p[o], four outputs, under the same mode switch
-// as fma_down_up16.
-__device__ __forceinline__ void add_down_up4(const float* acc, const float* p, float (&rd)[4],
-                                             float (&ru)[4]) {
+// acc[o] <- RTO24(acc[o] + p[o]) as rto_fma16, for 4 and 8 outputs
+__device__ __forceinline__ void rto_add4(const float* p, float* acc) {
+    float rd[4], mask[4];
     asm volatile(
         "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 2\n\t"
         "s_nop 1\n\t"
-        "v_add_f32 %0, %8, %12\n\t"
-        "v_add_f32 %1, %9, %13\n\t"
-        "v_add_f32 %2, %10, %14\n\t"
-        "v_add_f32 %3, %11, %15\n\t"
+        "v_add_f32 %4, %0, %12\n\t"
+        "v_add_f32 %5, %1, %13\n\t"
+        "v_add_f32 %6, %2, %14\n\t"
+        "v_add_f32 %7, %3, %15\n\t"
         "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 1\n\t"
         "s_nop 1\n\t"
-        "v_add_f32 %4, %8, %12\n\t"
-        "v_add_f32 %5, %9, %13\n\t"
-        "v_add_f32 %6, %10, %14\n\t"
-        "v_add_f32 %7, %11, %15\n\t"
+        "v_add_f32 %0, %0, %12\n\t"
+        "v_add_f32 %1, %1, %13\n\t"
+        "v_add_f32 %2, %2, %14\n\t"
+        "v_add_f32 %3, %3, %15\n\t"
         "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0\n\t"
-        "s_nop 1"
-        : "=&v"(rd[0]), "=&v"(rd[1]), "=&v"(rd[2]), "=&v"(rd[3]),
-          "=&v"(ru[0]), "=&v"(ru[1]), "=&v"(ru[2]), "=&v"(ru[3])
-        : "v"(acc[0]), "v"(acc[1]), "v"(acc[2]), "v"(acc[3]), "v"(p[0]), "v"(p[1]), "v"(p[2]),
-          "v"(p[3]));
+        "v_bfe_i32 %8, %0, 0, 1\n\t"
+        "v_bfe_i32 %9, %1, 0, 1\n\t"
+        "v_bfe_i32 %10, %2, 0, 1\n\t"
+        "v_bfe_i32 %11, %3, 0, 1\n\t"
+        "v_bfi_b32 %0, %8, %0, %4\n\t"
+        "v_bfi_b32 %1, %9, %1, %5\n\t"
+        "v_bfi_b32 %2, %10, %2, %6\n\t"
+        "v_bfi_b32 %3, %11, %3, %7"
+        : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]),
+          "=&v"(rd[0]), "=&v"(rd[1]), "=&v"(rd[2]), "=&v"(rd[3]),
+          "=&v"(mask[0]), "=&v"(mask[1]), "=&v"(mask[2]), "=&v"(mask[3])
+        : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]));
 }
 
-// The same for 8 outputs with one pair of mode switches.
-__device__ __forceinline__ void add_down_up8(const float* acc, const float* p, float (&rd)[8],
-                                             float (&ru)[8]) {
+__device__ __forceinline__ void rto_add8(const float* p, float* acc) {
+    float rd[8], mask[4];
     asm volatile(
         "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 2\n\t"
         "s_nop 1\n\t"
-        "v_add_f32 %0, %16, %24\n\t"
-        "v_add_f32 %1, %17, %25\n\t"
-        "v_add_f32 %2, %18, %26\n\t"
-        "v_add_f32 %3, %19, %27\n\t"
-        "v_add_f32 %4, %20, %28\n\t"
-        "v_add_f32 %5, %21, %29\n\t"
-        "v_add_f32 %6, %22, %30\n\t"
-        "v_add_f32 %7, %23, %31\n\t"
+        "v_add_f32 %8, %0, %20\n\t"
+        "v_add_f32 %9, %1, %21\n\t"
+        "v_add_f32 %10, %2, %22\n\t"
+        "v_add_f32 %11, %3, %23\n\t"
+        "v_add_f32 %12, %4, %24\n\t"
+        "v_add_f32 %13, %5, %25\n\t"
+        "v_add_f32 %14, %6, %26\n\t"
+        "v_add_f32 %15, %7, %27\n\t"
         "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 1\n\t"
         "s_nop 1\n\t"
-        "v_add_f32 %8, %16, %24\n\t"
-        "v_add_f32 %9, %17, %25\n\t"
-        "v_add_f32 %10, %18, %26\n\t"
-        "v_add_f32 %11, %19, %27\n\t"
-        "v_add_f32 %12, %20, %28\n\t"
-        "v_add_f32 %13, %21, %29\n\t"
-        "v_add_f32 %14, %22, %30\n\t"
-        "v_add_f32 %15, %23, %31\n\t"
+        "v_add_f32 %0, %0, %20\n\t"
+        "v_add_f32 %1, %1, %21\n\t"
+        "v_add_f32 %2, %2, %22\n\t"
+        "v_add_f32 %3, %3, %23\n\t"
+        "v_add_f32 %4, %4, %24\n\t"
+        "v_add_f32 %5, %5, %25\n\t"
+        "v_add_f32 %6, %6, %26\n\t"
+        "v_add_f32 %7, %7, %27\n\t"
         "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0\n\t"
-        "s_nop 1"
-        : "=&v"(rd[0]), "=&v"(rd[1]), "=&v"(rd[2]), "=&v"(rd[3]),
+        "v_bfe_i32 %16, %0, 0, 1\n\t"
+        "v_bfe_i32 %17, %1, 0, 1\n\t"
+        "v_bfe_i32 %18, %2, 0, 1\n\t"
+        "v_bfe_i32 %19, %3, 0, 1\n\t"
+        "v_bfi_b32 %0, %16, %0, %8\n\t"
+        "v_bfi_b32 %1, %17, %1, %9\n\t"
+        "v_bfi_b32 %2, %18, %2, %10\n\t"
+        "v_bfi_b32 %3, %19, %3, %11\n\t"
+        "v_bfe_i32 %16, %4, 0, 1\n\t"
+        "v_bfe_i32 %17, %5, 0, 1\n\t"
+        "v_bfe_i32 %18, %6, 0, 1\n\t"
+        "v_bfe_i32 %19, %7, 0, 1\n\t"
+        "v_bfi_b32 %4, %16, %4, %12\n\t"
+        "v_bfi_b32 %5, %17, %5, %13\n\t"
+        "v_bfi_b32 %6, %18, %6, %14\n\t"
+        "v_bfi_b32 %7, %19, %7, %15"
+        : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]),
+          "+v"(acc[4]), "+v"(acc[5]), "+v"(acc[6]), "+v"(acc[7]),
+          "=&v"(rd[0]), "=&v"(rd[1]), "=&v"(rd[2]), "=&v"(rd[3]),
           "=&v"(rd[4]), "=&v"(rd[5]), "=&v"(rd[6]), "=&v"(rd[7]),
-          "=&v"(ru[0]), "=&v"(ru[1]), "=&v"(ru[2]), "=&v"(ru[3]),
-          "=&v"(ru[4]), "=&v"(ru[5]), "=&v"(ru[6]), "=&v"(ru[7])
-        : "v"(acc[0]), "v"(acc[1]), "v"(acc[2]), "v"(acc[3]), "v"(acc[4]), "v"(acc[5]), "v"(acc[6]), "v"(acc[7]),
-          "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "v"(p[4]), "v"(p[5]), "v"(p[6]), "v"(p[7]));
+          "=&v"(mask[0]), "=&v"(mask[1]), "=&v"(mask[2]), "=&v"(mask[3])
+        : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]),
+          "v"(p[4]), "v"(p[5]), "v"(p[6]), "v"(p[7]));
 }
 
 // binary16(na - p), one rounding of the exact difference (see mix_sub16x16), as a float
@@ -194,17 +215,15 @@ __device__ __forceinline__ void chain_leaves(float (&p)[NR], float (&acc)[NR], b
                 for (int o = 0; o < NR; ++o)
                     p[o] = p[o] != p[o] ? __uint_as_float(0x7FC00000u) : p[o];
             }
-        float rd[NR], ru[NR];
-        if constexpr (NR == 8) add_down_up8(acc, p, rd, ru);
-        else add_down_up4(acc, p, rd, ru);
+        if constexpr (NR == 8) rto_add8(p, acc);
+        else rto_add4(p, acc);
+        if constexpr (KIND == kChainMant) {
 #pragma unroll
-        for (int o = 0; o < NR; ++o) {
-            const uint32_t t = rto_pick(__float_as_uint(ru[o]), __float_as_uint(rd[o]));
-            if constexpr (KIND == kChainMant23)
-                acc[o] = __uint_as_float(t);
-            else
+            for (int o = 0; o < NR; ++o) {
+                const uint32_t t = __float_as_uint(acc[o]);
                 acc[o] = __uint_as_float((t + g.dr_half + __builtin_amdgcn_ubfe(t, g.dr_rf, 1u)) &
                                          g.dr_mask);
+            }
         }
     }
 }

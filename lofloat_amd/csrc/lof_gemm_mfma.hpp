@@ -290,109 +290,125 @@ __device__ __forceinline__ void exact_sub16x16(const f32x16& p, float (&na)[16])
         : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "v"(p[4]), "v"(p[5]), "v"(p[6]), "v"(p[7]), "v"(p[8]), "v"(p[9]), "v"(p[10]), "v"(p[11]), "v"(p[12]), "v"(p[13]), "v"(p[14]), "v"(p[15]));
 }
 
-// RD / RU: a[o] * b + c[o] rounded down and up, for 16 outputs.  The wave's FP32 rounding
-// mode (MODE.FP_ROUND[1:0]: 2 toward -inf, 1 toward +inf, 0 nearest even) is switched only
-// inside this one asm block, which ends in round-to-nearest-even again, so no FP operation
-// the compiler schedules ever runs under a directed mode.  The FMA is correctly rounded in
-// every mode, FP32 subnormals included (denormals are not flushed), so rd / ru are the two
-// directed roundings of the exact a * b + c.
-__device__ __forceinline__ void fma_down_up16(const float (&a)[16], float b, const float (&c)[16],
-                                              float (&rd)[16], float (&ru)[16]) {
+// acc[o] <- RTO24(a[o] * b + acc[o]), the reference's round-to-odd sum (cutlass_gemms.cuh:74-80:
+// the truncation rz = (rd >= 0 ? rd : ru) of the directed roundings rd / ru, with its last bit set
+// when rd != ru), for any operands, the product exact or not.  rd and ru are the FMA under
+// round-down and round-up: the wave's FP32 rounding mode (MODE.FP_ROUND[1:0]: 2 toward -inf, 1
+// toward +inf, 0 nearest even) is switched only inside this one asm block, so no FP operation
+// the compiler schedules runs under a directed mode.  When rd != ru they are adjacent floats of
+// one sign (FP32 subnormals are kept; FLT_MAX and inf are adjacent patterns too), so the
+// truncation with its last bit set is the odd pattern of the two: ru where ru is odd, else rd
+// -- by ru's last bit as a mask (v_bfe_i32) and a bitwise select.  An exact sum has
+// rd == ru; an exact zero keeps rd's sign, roundTowardNegative's ((+0) + (+0) = +0, any other
+// exact zero -0).  Four instructions a leaf; comparing rd with ru and or-ing the smaller
+// pattern's last bit took six.
+__device__ __forceinline__ void rto_fma16(const float* a, float b, float* acc) {
+    float rd[16], mask[4];
     asm volatile(
         "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 2\n\t"
         "s_nop 1\n\t"
-        "v_fma_f32 %0, %32, %48, %49\n\t"
-        "v_fma_f32 %1, %33, %48, %50\n\t"
-        "v_fma_f32 %2, %34, %48, %51\n\t"
-        "v_fma_f32 %3, %35, %48, %52\n\t"
-        "v_fma_f32 %4, %36, %48, %53\n\t"
-        "v_fma_f32 %5, %37, %48, %54\n\t"
-        "v_fma_f32 %6, %38, %48, %55\n\t"
-        "v_fma_f32 %7, %39, %48, %56\n\t"
-        "v_fma_f32 %8, %40, %48, %57\n\t"
-        "v_fma_f32 %9, %41, %48, %58\n\t"
-        "v_fma_f32 %10, %42, %48, %59\n\t"
-        "v_fma_f32 %11, %43, %48, %60\n\t"
-        "v_fma_f32 %12, %44, %48, %61\n\t"
-        "v_fma_f32 %13, %45, %48, %62\n\t"
-        "v_fma_f32 %14, %46, %48, %63\n\t"
-        "v_fma_f32 %15, %47, %48, %64\n\t"
+        "v_fma_f32 %16, %36, %52, %0\n\t"
+        "v_fma_f32 %17, %37, %52, %1\n\t"
+        "v_fma_f32 %18, %38, %52, %2\n\t"
+        "v_fma_f32 %19, %39, %52, %3\n\t"
+        "v_fma_f32 %20, %40, %52, %4\n\t"
+        "v_fma_f32 %21, %41, %52, %5\n\t"
+        "v_fma_f32 %22, %42, %52, %6\n\t"
+        "v_fma_f32 %23, %43, %52, %7\n\t"
+        "v_fma_f32 %24, %44, %52, %8\n\t"
+        "v_fma_f32 %25, %45, %52, %9\n\t"
+        "v_fma_f32 %26, %46, %52, %10\n\t"
+        "v_fma_f32 %27, %47, %52, %11\n\t"
+        "v_fma_f32 %28, %48, %52, %12\n\t"
+        "v_fma_f32 %29, %49, %52, %13\n\t"
+        "v_fma_f32 %30, %50, %52, %14\n\t"
+        "v_fma_f32 %31, %51, %52, %15\n\t"
         "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 1\n\t"
         "s_nop 1\n\t"
-        "v_fma_f32 %16, %32, %48, %49\n\t"
-        "v_fma_f32 %17, %33, %48, %50\n\t"
-        "v_fma_f32 %18, %34, %48, %51\n\t"
-        "v_fma_f32 %19, %35, %48, %52\n\t"
-        "v_fma_f32 %20, %36, %48, %53\n\t"
-        "v_fma_f32 %21, %37, %48, %54\n\t"
-        "v_fma_f32 %22, %38, %48, %55\n\t"
-        "v_fma_f32 %23, %39, %48, %56\n\t"
-        "v_fma_f32 %24, %40, %48, %57\n\t"
-        "v_fma_f32 %25, %41, %48, %58\n\t"
-        "v_fma_f32 %26, %42, %48, %59\n\t"
-        "v_fma_f32 %27, %43, %48, %60\n\t"
-        "v_fma_f32 %28, %44, %48, %61\n\t"
-        "v_fma_f32 %29, %45, %48, %62\n\t"
-        "v_fma_f32 %30, %46, %48, %63\n\t"
-        "v_fma_f32 %31, %47, %48, %64\n\t"
+        "v_fma_f32 %0, %36, %52, %0\n\t"
+        "v_fma_f32 %1, %37, %52, %1\n\t"
+        "v_fma_f32 %2, %38, %52, %2\n\t"
+        "v_fma_f32 %3, %39, %52, %3\n\t"
+        "v_fma_f32 %4, %40, %52, %4\n\t"
+        "v_fma_f32 %5, %41, %52, %5\n\t"
+        "v_fma_f32 %6, %42, %52, %6\n\t"
+        "v_fma_f32 %7, %43, %52, %7\n\t"
+        "v_fma_f32 %8, %44, %52, %8\n\t"
+        "v_fma_f32 %9, %45, %52, %9\n\t"
+        "v_fma_f32 %10, %46, %52, %10\n\t"
+        "v_fma_f32 %11, %47, %52, %11\n\t"
+        "v_fma_f32 %12, %48, %52, %12\n\t"
+        "v_fma_f32 %13, %49, %52, %13\n\t"
+        "v_fma_f32 %14, %50, %52, %14\n\t"
+        "v_fma_f32 %15, %51, %52, %15\n\t"
         "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0\n\t"
-        "s_nop 1"
-        : "=&v"(rd[0]), "=&v"(rd[1]), "=&v"(rd[2]), "=&v"(rd[3]), "=&v"(rd[4]), "=&v"(rd[5]),
-          "=&v"(rd[6]), "=&v"(rd[7]), "=&v"(rd[8]), "=&v"(rd[9]), "=&v"(rd[10]), "=&v"(rd[11]),
+        "v_bfe_i32 %32, %0, 0, 1\n\t"
+        "v_bfe_i32 %33, %1, 0, 1\n\t"
+        "v_bfe_i32 %34, %2, 0, 1\n\t"
+        "v_bfe_i32 %35, %3, 0, 1\n\t"
+        "v_bfi_b32 %0, %32, %0, %16\n\t"
+        "v_bfi_b32 %1, %33, %1, %17\n\t"
+        "v_bfi_b32 %2, %34, %2, %18\n\t"
+        "v_bfi_b32 %3, %35, %3, %19\n\t"
+        "v_bfe_i32 %32, %4, 0, 1\n\t"
+        "v_bfe_i32 %33, %5, 0, 1\n\t"
+        "v_bfe_i32 %34, %6, 0, 1\n\t"
+        "v_bfe_i32 %35, %7, 0, 1\n\t"
+        "v_bfi_b32 %4, %32, %4, %20\n\t"
+        "v_bfi_b32 %5, %33, %5, %21\n\t"
+        "v_bfi_b32 %6, %34, %6, %22\n\t"
+        "v_bfi_b32 %7, %35, %7, %23\n\t"
+        "v_bfe_i32 %32, %8, 0, 1\n\t"
+        "v_bfe_i32 %33, %9, 0, 1\n\t"
+        "v_bfe_i32 %34, %10, 0, 1\n\t"
+        "v_bfe_i32 %35, %11, 0, 1\n\t"
+        "v_bfi_b32 %8, %32, %8, %24\n\t"
+        "v_bfi_b32 %9, %33, %9, %25\n\t"
+        "v_bfi_b32 %10, %34, %10, %26\n\t"
+        "v_bfi_b32 %11, %35, %11, %27\n\t"
+        "v_bfe_i32 %32, %12, 0, 1\n\t"
+        "v_bfe_i32 %33, %13, 0, 1\n\t"
+        "v_bfe_i32 %34, %14, 0, 1\n\t"
+        "v_bfe_i32 %35, %15, 0, 1\n\t"
+        "v_bfi_b32 %12, %32, %12, %28\n\t"
+        "v_bfi_b32 %13, %33, %13, %29\n\t"
+        "v_bfi_b32 %14, %34, %14, %30\n\t"
+        "v_bfi_b32 %15, %35, %15, %31"
+        : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]),
+          "+v"(acc[4]), "+v"(acc[5]), "+v"(acc[6]), "+v"(acc[7]),
+          "+v"(acc[8]), "+v"(acc[9]), "+v"(acc[10]), "+v"(acc[11]),
+          "+v"(acc[12]), "+v"(acc[13]), "+v"(acc[14]), "+v"(acc[15]),
+          "=&v"(rd[0]), "=&v"(rd[1]), "=&v"(rd[2]), "=&v"(rd[3]),
+          "=&v"(rd[4]), "=&v"(rd[5]), "=&v"(rd[6]), "=&v"(rd[7]),
+          "=&v"(rd[8]), "=&v"(rd[9]), "=&v"(rd[10]), "=&v"(rd[11]),
           "=&v"(rd[12]), "=&v"(rd[13]), "=&v"(rd[14]), "=&v"(rd[15]),
-          "=&v"(ru[0]), "=&v"(ru[1]), "=&v"(ru[2]), "=&v"(ru[3]), "=&v"(ru[4]), "=&v"(ru[5]),
-          "=&v"(ru[6]), "=&v"(ru[7]), "=&v"(ru[8]), "=&v"(ru[9]), "=&v"(ru[10]), "=&v"(ru[11]),
-          "=&v"(ru[12]), "=&v"(ru[13]), "=&v"(ru[14]), "=&v"(ru[15])
-        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]),
-          "v"(a[7]), "v"(a[8]), "v"(a[9]), "v"(a[10]), "v"(a[11]), "v"(a[12]), "v"(a[13]),
-          "v"(a[14]), "v"(a[15]), "v"(b),
-          "v"(c[0]), "v"(c[1]), "v"(c[2]), "v"(c[3]), "v"(c[4]), "v"(c[5]), "v"(c[6]),
-          "v"(c[7]), "v"(c[8]), "v"(c[9]), "v"(c[10]), "v"(c[11]), "v"(c[12]), "v"(c[13]),
-          "v"(c[14]), "v"(c[15]));
+          "=&v"(mask[0]), "=&v"(mask[1]), "=&v"(mask[2]), "=&v"(mask[3])
+        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]),
+          "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]),
+          "v"(a[8]), "v"(a[9]), "v"(a[10]), "v"(a[11]),
+          "v"(a[12]), "v"(a[13]), "v"(a[14]), "v"(a[15]), "v"(b));
 }
 
-// RTO24 from the two directed roundings of x (bit patterns, equal when x is a float): the
-// neighbour with the odd significand, so the pattern of the pair whose last bit is set.  An
-// exact x has equal patterns and keeps them, an exact zero the even one's sign (`even`), and
-// overflow the odd FLT_MAX over the even infinity.  Two instructions: `odd`'s last bit as a mask
-// (an asm statement, since the compiler turns the plain expression into an and, a compare and a
-// select) and a bitwise select; testing rd == ru and or-ing the smaller pattern's last bit
-// takes four.
-__device__ __forceinline__ uint32_t rto_pick(uint32_t odd, uint32_t even) {
-    uint32_t mask;
-    asm("v_bfe_i32 %0, %1, 0, 1" : "=v"(mask) : "v"(odd));
-    return (odd & mask) | (even & ~mask);
-}
-
-// Directed-rounding leaves of 16 outputs: acc[o] <- round(RTO24(a[o] * b + acc[o])) for any
-// operands, the products exact or not.  This is round_to_odd_fma's construction
-// (cutlass_gemms.cuh:74-80) from the directed roundings rd / ru of x = a * b + acc: the
-// truncation rz = (rd >= 0 ? rd : ru) with its last bit set when rd != ru.  So an exact x is
-// rd, an exact zero with roundTowardNegative's sign ((+0) + (+0) = +0, any other exact zero
-// -0), and an overflowing x gives FLT_MAX | 1 with its sign.  When rd != ru they are adjacent
-// floats of the same sign bit (FP32 subnormals are kept, so only an exact zero straddles it;
-// FLT_MAX and inf are adjacent patterns too), and the truncation with its last bit set is the
-// odd one of the two: rto_pick.
-// round() is round-to-nearest-even at bit dr_rf of the pattern (a mantissa-only accumulator:
-// bitwise virtual_round, lo_float.h:2716-2756) or, F16, the binary16 conversion (a
-// binary16-shaped format, for sums the caller has bounded below 2^15).  M23: a 23-bit
-// accumulator, whose round() keeps every float: RTO24 alone, 4 instructions a leaf against 7.
-// (Forward and both gradients of a 2048 x 1024 -> 4096 layer on FP32 operands: 6.66 -> 3.94 ms.)
+// Directed-rounding leaves of 16 outputs: acc[o] <- round(RTO24(a[o] * b + acc[o])).  round() is
+// round-to-nearest-even at bit dr_rf of the pattern (a mantissa-only accumulator: bitwise
+// virtual_round, lo_float.h:2716-2756) or, F16, the binary16 conversion (a binary16-shaped
+// format, for sums the caller has bounded below 2^15).  M23: a 23-bit accumulator, whose round()
+// keeps every float: RTO24 alone, 4 instructions a leaf against 7.
+// (Forward and both gradients of a 2048 x 1024 -> 4096 layer on FP32 operands: 6.64 -> 3.26 ms.)
 template <bool F16, bool M23 = false>
 __device__ __forceinline__ void leaves_dr16(const float (&a)[16], float b, float (&acc)[16],
                                             const GemmArgs& g) {
-    float rd[16], ru[16];
-    fma_down_up16(a, b, acc, rd, ru);
+    rto_fma16(a, b, acc);
+    if constexpr (!M23) {
 #pragma unroll
-    for (int o = 0; o < 16; ++o) {
-        const uint32_t t = rto_pick(__float_as_uint(ru[o]), __float_as_uint(rd[o]));
-        if constexpr (F16)
-            acc[o] = (float)(_Float16)__uint_as_float(t);
-        else if constexpr (M23)
-            acc[o] = __uint_as_float(t);
-        else   // round to nearest even at bit dr_rf: the kept lsb (none when dr_rf is 0)
-            acc[o] = __uint_as_float((t + g.dr_half + __builtin_amdgcn_ubfe(t, g.dr_rf, g.dr_lsb)) &
-                                     g.dr_mask);
+        for (int o = 0; o < 16; ++o) {
+            const uint32_t t = __float_as_uint(acc[o]);
+            if constexpr (F16)
+                acc[o] = (float)(_Float16)acc[o];
+            else   // round to nearest even at bit dr_rf: the kept lsb (none when dr_rf is 0)
+                acc[o] = __uint_as_float((t + g.dr_half + __builtin_amdgcn_ubfe(t, g.dr_rf, g.dr_lsb)) &
+                                         g.dr_mask);
+        }
     }
 }
 
