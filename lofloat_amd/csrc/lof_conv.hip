@@ -14,6 +14,7 @@
 #include <cstdint>
 
 #include "lof_gemm.hpp"
+#include "lof_gemm_chain.hpp"
 #include "lof_host.hpp"
 
 namespace lofamd {
@@ -192,7 +193,7 @@ LOF_API lof_status lof_conv2d_f32(const lof_conv2d_desc* desc, int32_t config,
         cv.sdm = 1;
         cv.sdpq = c.K;
     }
-    if (g.chain >= 0) {
+    if (g.chain >= 0 && (g.chunk > 1 || g.chain != kChainMant)) {
         int t = 1;
         if (cfg < 0) {
             t = chain_default_tile(c.K, Ncols);

@@ -73,6 +73,8 @@ const GemmConfig kConfigs[] = {
 };
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
 constexpr int kFirstMfma = 5, kMfma64 = 7, kMfma64x128 = 8, kFirstShort = 9;
+constexpr bool kShortTile[kChainTiles] = {false, false, true, true, true};
+constexpr int kShortMantTiles = 64;
 
 // chunks whose sums can run on MFMA
 bool chunk_fits_mfma(int chunk) { return chunk >= 2 && chunk <= 32 && (32 % chunk) == 0; }
@@ -84,6 +86,13 @@ bool is_mfma(int config) { return config >= kFirstMfma; }
 bool config_valid(int config, int chunk) {
     return config >= 0 && config < kNumConfigs &&
            (!is_mfma(config) || chunk_fits_wave_tile(chunk));
+}
+
+// Whether the chunk-sum kernels run this product on a wave-tile config.  At chunk 1 the mantissa-
+// only accumulators of 1 to 22 bits, 10 aside, keep the wave tile's exact-sum and held leaves (a third to
+// an eighth of the directed leaf's instructions) and take the short tiles only.
+bool chain_takes(const GemmArgs& g, int config) {
+    return g.chain >= 0 && (g.chunk > 1 || g.chain != kChainMant || config >= kFirstShort);
 }
 
 GemmKernel pick_kernel(const GemmConfig& c, const GemmArgs& g) {
@@ -112,17 +121,23 @@ TuneKey tune_key(const lof_gemm_desc& d) {
                    d.accum.chunk};
 }
 
-// Untuned choice, from measurements at M = N = K = 4096 and on conv-shaped GEMMs
-// (M = 64..512, e4m3 / 8e7m inputs): wave tiles for the chunks they take, 64x128 (each
-// lane's A values serve two B columns) where that still gives enough tiles -- >= 384 (1.5
-// per CU) for chunks 2..32 (+18-22 % over 64x64 at chunks 2 and 4), >= 768 for chunk 1,
-// whose exact-sum leaves are LDS-bound (e4m3 +10-15 %, 8e7m on the RTO leaves -4-9 %) --
-// else 64x64; the 32x64 VALU tile for other chunks; the 32x32 VALU tile when there are too
-// few tiles to fill the chip.
+// Untuned choice: the chunk-sum kernels' tile (chain_default_tile) where they run; at chunk 1 with
+// another accumulator 64x128 (each lane's A values serve two B columns) from 768 such tiles on
+// (4096^3: e4m3 +10-15 % over 64x64, 8e7m on the RTO leaves -4-9 %), else 64x64; the 32x64 VALU
+// tile for other chunks, the 32x32 one when there are too few tiles to fill the chip.
 int default_config(const lof_gemm_desc& d) {
     if (chunk_fits_wave_tile(d.accum.chunk)) {
+        const int t = chain_default_tile(d.M, d.N);
+        const lof_accum& ac = d.accum;
+        const bool mant = ac.kind == LOF_ACCUM_MANTISSA;
+        const bool half = !mant && ac.fmt.mantissa_bits == 10 && ac.fmt.bias == 15;
+        if (ac.spec.mode == RNE && (half || (mant && (ac.chunk > 1 || ac.mant_bits == 23 || ac.mant_bits == 10))))
+            return kChainConfigOf[t];
+        if (ac.spec.mode == RNE && mant && kShortTile[t] &&
+            (int64_t)((d.M + 63) / 64) * ((d.N + 63) / 64) < kShortMantTiles)
+            return kChainConfigOf[t];
         const int64_t tiles_64x128 = (int64_t)((d.M + 63) / 64) * ((d.N + 127) / 128);
-        return tiles_64x128 >= (d.accum.chunk == 1 ? 768 : 384) ? kMfma64x128 : kMfma64;
+        return tiles_64x128 >= 768 ? kMfma64x128 : kMfma64;
     }
     if ((int64_t)((d.M + 31) / 32) * ((d.N + 63) / 64) >= 1024) return 3;
     return 4;
@@ -132,14 +147,18 @@ int default_config(const lof_gemm_desc& d) {
 
 void set_chain(GemmArgs* g, bool conv) {
     g->chain = -1;
-    if (!chunk_fits_mfma(g->chunk) || g->acc_mode != RNE || g->lda > kChainMaxLd ||
+    if (!chunk_fits_wave_tile(g->chunk) || g->acc_mode != RNE || g->lda > kChainMaxLd ||
         (!conv && g->ldb > kChainMaxLd))
         return;
     if (g->sum_f16) {
+        // chunk 1 holds the accumulator as binary16, whose top binade the format must reach
+        if (g->chunk == 1 && g->sum_ehi < 15) return;
         g->chain = kChainHalf;
         g->half_top = std::ldexp(1.0f, g->sum_ehi);
     } else if (g->acc_kind == 0 && g->acc_r < 23) {   // 0 bits: rounding can lose a NaN's sign
-        g->chain = g->acc_r == 0 ? kChainMant23 : kChainMant;
+        g->chain = g->acc_r == 0                       ? kChainMant23
+                   : g->acc_r == 13 && g->chunk == 1 ? kChainMant10
+                                                     : kChainMant;
     }
 }
 
@@ -158,10 +177,11 @@ int chain_default_tile(int64_t M, int64_t N) {
 lof_status launch_chain(const GemmArgs& g, int tile, hipStream_t st, const char* what) {
     const ChainTable& t = g.chain == kChainHalf     ? kChainTableHalf
                           : g.chain == kChainMant23 ? kChainTableMant23
+                          : g.chain == kChainMant10 ? kChainTableMant10
                                                     : kChainTableMant;
-    const int l2 = 30 - __builtin_clz((unsigned)g.chunk);   // log2(chunk) - 1
+    const int l2 = 31 - __builtin_clz((unsigned)g.chunk);
     ChainKernel k = g.cv.conv ? t.conv[tile][l2] : t.gemm[tile][l2];
-    if (!k) {   // a chunk of 2 on a 16-row block, whose MFMA takes 4 k
+    if (!k) {   // chunk 2 on a 16-row block (its MFMA takes 4 k), chunk 1 on the widest tile
         tile = 1;
         k = g.cv.conv ? t.conv[tile][l2] : t.gemm[tile][l2];
     }
@@ -321,7 +341,7 @@ lof_status launch_gemm(const GemmArgs& g, int config, hipStream_t st) {
         return set_error(LOF_ERR_UNSUPPORTED,
                          "lof_gemm_f32: config %d needs a chunk in {1, 2, 4, 8, 16, 32} (got %d)",
                          config, g.chunk);
-    if (is_mfma(config) && g.chain >= 0)
+    if (is_mfma(config) && chain_takes(g, config))
         return launch_chain(g, kChainTileOf[config - kFirstMfma], st, "lof_gemm_f32 launch");
     const GemmConfig& c = kConfigs[config >= kFirstShort ? kMfma64 : config];
     dim3 grid((unsigned)((g.N + c.bn - 1) / c.bn), (unsigned)((g.M + c.bm - 1) / c.bm));
@@ -339,9 +359,7 @@ int resolve_gemm_config(const lof_gemm_desc& d, int config) {
     if (config >= 0) return config;
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tuned.find(tune_key(d));
-    if (it != g_tuned.end()) return it->second;
-    return chunk_fits_mfma(d.accum.chunk) ? kChainConfigOf[chain_default_tile(d.M, d.N)]
-                                          : default_config(d);
+    return it != g_tuned.end() ? it->second : default_config(d);
 }
 
 }  // namespace lofamd
@@ -429,8 +447,9 @@ LOF_API lof_status lof_gemm_autotune(const lof_gemm_desc* desc, int32_t iters,
     const bool wave = chunk_fits_wave_tile(g.chunk);
     for (int c = 0; c < kNumConfigs && s == LOF_OK; ++c) {
         if (!config_valid(c, g.chunk) || is_mfma(c) != wave) continue;
-        if (c >= kFirstShort && g.chain < 0) continue;   // would time mfma11 again
-        if (g.chain >= 0 && (c == 6 || c == 8)) continue;
+        if (c >= kFirstShort && !chain_takes(g, c)) continue;   // would time mfma11 again
+        if ((c == 6 || c == 8) && chain_takes(g, c)) continue;
+        if (c == 5 && g.chunk == 1 && chain_takes(g, c)) continue;
         s = launch_gemm(g, c, st);  // warm-up
         if (s != LOF_OK) break;
         (void)hipEventRecord(e0, st);

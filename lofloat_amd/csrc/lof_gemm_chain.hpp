@@ -42,7 +42,7 @@ namespace lofamd {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // Accumulators the tile's leaf takes (ChainArgs-free: the constants are GemmArgs').
-enum ChainKind : int { kChainMant = 0, kChainMant23 = 1, kChainHalf = 2 };
+enum ChainKind : int { kChainMant = 0, kChainMant23 = 1, kChainHalf = 2, kChainMant10 = 3 };
 
 // An operand slice in LDS: R rows (A's m, B's n) by BK k, k-major in groups of four k that
 // start PAD floats apart, the row swizzled by k.  An MFMA operand read takes KI consecutive k of
@@ -68,7 +68,7 @@ struct ChainTile {
     static constexpr int NR = BS * BS / 64;        // outputs per lane and block
     static constexpr int KI = BS == 32 ? 2 : 4;    // k per MFMA
     static constexpr int BUF_FLOATS = ChainLds<BM, BK, KI>::FLOATS + ChainLds<BN, BK, KI>::FLOATS;
-    static constexpr int SMEM_FLOATS = 2 * BUF_FLOATS + 4;   // + 3 non-finite flags
+    static constexpr int SMEM_FLOATS = 2 * BUF_FLOATS + 40;   // + 3 flags, statistics, 3 flags
     static constexpr int NA4 = BM * BK / 1024, NB4 = BN * BK / 1024;   // float4 per thread
     static_assert(NA4 * 1024 == BM * BK && NB4 * 1024 == BN * BK, "whole float4s per thread");
 };
@@ -228,6 +228,218 @@ __device__ __forceinline__ void chain_leaves(float (&p)[NR], float (&acc)[NR], b
     }
 }
 
+// Chunk 1, on the negated accumulator: na[o] <- -RTO24(a[o] * b + acc[o]), na = -acc.  Round-to-odd
+// and both roundings after it are odd functions, so rto_fma16's construction applied to
+// y = na - a b gives the negated result; only an exact zero changes: -(RTO24's zero of the sum)
+// is roundTowardPositive's zero of y, so the pick is by rd's last bit and falls to ru.
+__device__ __forceinline__ void rto_fnma16(const float* a, float b, float* na) {
+    float rd[16], mask[4];
+    asm volatile(
+        "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 2\n\t"
+        "s_nop 1\n\t"
+        "v_fma_f32 %16, -%36, %52, %0\n\t"
+        "v_fma_f32 %17, -%37, %52, %1\n\t"
+        "v_fma_f32 %18, -%38, %52, %2\n\t"
+        "v_fma_f32 %19, -%39, %52, %3\n\t"
+        "v_fma_f32 %20, -%40, %52, %4\n\t"
+        "v_fma_f32 %21, -%41, %52, %5\n\t"
+        "v_fma_f32 %22, -%42, %52, %6\n\t"
+        "v_fma_f32 %23, -%43, %52, %7\n\t"
+        "v_fma_f32 %24, -%44, %52, %8\n\t"
+        "v_fma_f32 %25, -%45, %52, %9\n\t"
+        "v_fma_f32 %26, -%46, %52, %10\n\t"
+        "v_fma_f32 %27, -%47, %52, %11\n\t"
+        "v_fma_f32 %28, -%48, %52, %12\n\t"
+        "v_fma_f32 %29, -%49, %52, %13\n\t"
+        "v_fma_f32 %30, -%50, %52, %14\n\t"
+        "v_fma_f32 %31, -%51, %52, %15\n\t"
+        "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 1\n\t"
+        "s_nop 1\n\t"
+        "v_fma_f32 %0, -%36, %52, %0\n\t"
+        "v_fma_f32 %1, -%37, %52, %1\n\t"
+        "v_fma_f32 %2, -%38, %52, %2\n\t"
+        "v_fma_f32 %3, -%39, %52, %3\n\t"
+        "v_fma_f32 %4, -%40, %52, %4\n\t"
+        "v_fma_f32 %5, -%41, %52, %5\n\t"
+        "v_fma_f32 %6, -%42, %52, %6\n\t"
+        "v_fma_f32 %7, -%43, %52, %7\n\t"
+        "v_fma_f32 %8, -%44, %52, %8\n\t"
+        "v_fma_f32 %9, -%45, %52, %9\n\t"
+        "v_fma_f32 %10, -%46, %52, %10\n\t"
+        "v_fma_f32 %11, -%47, %52, %11\n\t"
+        "v_fma_f32 %12, -%48, %52, %12\n\t"
+        "v_fma_f32 %13, -%49, %52, %13\n\t"
+        "v_fma_f32 %14, -%50, %52, %14\n\t"
+        "v_fma_f32 %15, -%51, %52, %15\n\t"
+        "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0\n\t"
+        "v_bfe_i32 %32, %16, 0, 1\n\t"
+        "v_bfe_i32 %33, %17, 0, 1\n\t"
+        "v_bfe_i32 %34, %18, 0, 1\n\t"
+        "v_bfe_i32 %35, %19, 0, 1\n\t"
+        "v_bfi_b32 %0, %32, %16, %0\n\t"
+        "v_bfi_b32 %1, %33, %17, %1\n\t"
+        "v_bfi_b32 %2, %34, %18, %2\n\t"
+        "v_bfi_b32 %3, %35, %19, %3\n\t"
+        "v_bfe_i32 %32, %20, 0, 1\n\t"
+        "v_bfe_i32 %33, %21, 0, 1\n\t"
+        "v_bfe_i32 %34, %22, 0, 1\n\t"
+        "v_bfe_i32 %35, %23, 0, 1\n\t"
+        "v_bfi_b32 %4, %32, %20, %4\n\t"
+        "v_bfi_b32 %5, %33, %21, %5\n\t"
+        "v_bfi_b32 %6, %34, %22, %6\n\t"
+        "v_bfi_b32 %7, %35, %23, %7\n\t"
+        "v_bfe_i32 %32, %24, 0, 1\n\t"
+        "v_bfe_i32 %33, %25, 0, 1\n\t"
+        "v_bfe_i32 %34, %26, 0, 1\n\t"
+        "v_bfe_i32 %35, %27, 0, 1\n\t"
+        "v_bfi_b32 %8, %32, %24, %8\n\t"
+        "v_bfi_b32 %9, %33, %25, %9\n\t"
+        "v_bfi_b32 %10, %34, %26, %10\n\t"
+        "v_bfi_b32 %11, %35, %27, %11\n\t"
+        "v_bfe_i32 %32, %28, 0, 1\n\t"
+        "v_bfe_i32 %33, %29, 0, 1\n\t"
+        "v_bfe_i32 %34, %30, 0, 1\n\t"
+        "v_bfe_i32 %35, %31, 0, 1\n\t"
+        "v_bfi_b32 %12, %32, %28, %12\n\t"
+        "v_bfi_b32 %13, %33, %29, %13\n\t"
+        "v_bfi_b32 %14, %34, %30, %14\n\t"
+        "v_bfi_b32 %15, %35, %31, %15\n\t"
+        "s_nop 1"
+        : "+v"(na[0]), "+v"(na[1]), "+v"(na[2]), "+v"(na[3]),
+          "+v"(na[4]), "+v"(na[5]), "+v"(na[6]), "+v"(na[7]),
+          "+v"(na[8]), "+v"(na[9]), "+v"(na[10]), "+v"(na[11]),
+          "+v"(na[12]), "+v"(na[13]), "+v"(na[14]), "+v"(na[15]),
+          "=&v"(rd[0]), "=&v"(rd[1]), "=&v"(rd[2]), "=&v"(rd[3]),
+          "=&v"(rd[4]), "=&v"(rd[5]), "=&v"(rd[6]), "=&v"(rd[7]),
+          "=&v"(rd[8]), "=&v"(rd[9]), "=&v"(rd[10]), "=&v"(rd[11]),
+          "=&v"(rd[12]), "=&v"(rd[13]), "=&v"(rd[14]), "=&v"(rd[15]),
+          "=&v"(mask[0]), "=&v"(mask[1]), "=&v"(mask[2]), "=&v"(mask[3])
+        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]),
+          "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]),
+          "v"(a[8]), "v"(a[9]), "v"(a[10]), "v"(a[11]),
+          "v"(a[12]), "v"(a[13]), "v"(a[14]), "v"(a[15]), "v"(b));
+}
+
+__device__ __forceinline__ void rto_fnma4(const float* a, float b, float* na) {
+    float rd[4], mask[4];
+    asm volatile(
+        "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 2\n\t"
+        "s_nop 1\n\t"
+        "v_fma_f32 %4, -%12, %16, %0\n\t"
+        "v_fma_f32 %5, -%13, %16, %1\n\t"
+        "v_fma_f32 %6, -%14, %16, %2\n\t"
+        "v_fma_f32 %7, -%15, %16, %3\n\t"
+        "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 1\n\t"
+        "s_nop 1\n\t"
+        "v_fma_f32 %0, -%12, %16, %0\n\t"
+        "v_fma_f32 %1, -%13, %16, %1\n\t"
+        "v_fma_f32 %2, -%14, %16, %2\n\t"
+        "v_fma_f32 %3, -%15, %16, %3\n\t"
+        "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0\n\t"
+        "v_bfe_i32 %8, %4, 0, 1\n\t"
+        "v_bfe_i32 %9, %5, 0, 1\n\t"
+        "v_bfe_i32 %10, %6, 0, 1\n\t"
+        "v_bfe_i32 %11, %7, 0, 1\n\t"
+        "v_bfi_b32 %0, %8, %4, %0\n\t"
+        "v_bfi_b32 %1, %9, %5, %1\n\t"
+        "v_bfi_b32 %2, %10, %6, %2\n\t"
+        "v_bfi_b32 %3, %11, %7, %3\n\t"
+        "s_nop 1"
+        : "+v"(na[0]), "+v"(na[1]), "+v"(na[2]), "+v"(na[3]),
+          "=&v"(rd[0]), "=&v"(rd[1]), "=&v"(rd[2]), "=&v"(rd[3]),
+          "=&v"(mask[0]), "=&v"(mask[1]), "=&v"(mask[2]), "=&v"(mask[3])
+        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b));
+}
+
+// h <- binary16(h - a b), one rounding of the exact difference (see mix_fnma16), for the
+// binary16 pairs h[i] = (h[2 i], h[2 i + 1]); the low halves first, so that no instruction follows
+// the one that wrote half of its register.
+__device__ __forceinline__ void mix_fnma_pairs16(const float* a, float b, uint32_t* h) {
+    asm volatile(
+        "v_fma_mixlo_f16 %0, -%8, %24, %0 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %1, -%10, %24, %1 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %2, -%12, %24, %2 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %3, -%14, %24, %3 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %4, -%16, %24, %4 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %5, -%18, %24, %5 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %6, -%20, %24, %6 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %7, -%22, %24, %7 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %0, -%9, %24, %0 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %1, -%11, %24, %1 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %2, -%13, %24, %2 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %3, -%15, %24, %3 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %4, -%17, %24, %4 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %5, -%19, %24, %5 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %6, -%21, %24, %6 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %7, -%23, %24, %7 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "s_nop 1"
+        : "+v"(h[0]), "+v"(h[1]), "+v"(h[2]), "+v"(h[3]),
+          "+v"(h[4]), "+v"(h[5]), "+v"(h[6]), "+v"(h[7])
+        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]),
+          "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]),
+          "v"(a[8]), "v"(a[9]), "v"(a[10]), "v"(a[11]),
+          "v"(a[12]), "v"(a[13]), "v"(a[14]), "v"(a[15]), "v"(b));
+}
+
+__device__ __forceinline__ void mix_fnma_pairs4(const float* a, float b, uint32_t* h) {
+    asm volatile(
+        "v_fma_mixlo_f16 %0, -%2, %6, %0 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %1, -%4, %6, %1 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %0, -%3, %6, %0 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %1, -%5, %6, %1 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "s_nop 1"
+        : "+v"(h[0]), "+v"(h[1])
+        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b));
+}
+
+// The same, with the least magnitude of every result so far in `least`'s low half.
+__device__ __forceinline__ void mix_fnma_pairs16(const float* a, float b, uint32_t* h, uint32_t& least) {
+    asm volatile(
+        "v_fma_mixlo_f16 %0, -%9, %25, %0 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %1, -%11, %25, %1 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %2, -%13, %25, %2 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %3, -%15, %25, %3 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %4, -%17, %25, %4 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %5, -%19, %25, %5 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %6, -%21, %25, %6 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %7, -%23, %25, %7 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %0, -%10, %25, %0 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %1, -%12, %25, %1 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %2, -%14, %25, %2 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %3, -%16, %25, %3 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %4, -%18, %25, %4 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %5, -%20, %25, %5 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %6, -%22, %25, %6 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %7, -%24, %25, %7 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_min3_f16 %8, %8, |%0|, |%0| op_sel:[0,0,1,0]\n\t"
+        "v_min3_f16 %8, %8, |%1|, |%1| op_sel:[0,0,1,0]\n\t"
+        "v_min3_f16 %8, %8, |%2|, |%2| op_sel:[0,0,1,0]\n\t"
+        "v_min3_f16 %8, %8, |%3|, |%3| op_sel:[0,0,1,0]\n\t"
+        "v_min3_f16 %8, %8, |%4|, |%4| op_sel:[0,0,1,0]\n\t"
+        "v_min3_f16 %8, %8, |%5|, |%5| op_sel:[0,0,1,0]\n\t"
+        "v_min3_f16 %8, %8, |%6|, |%6| op_sel:[0,0,1,0]\n\t"
+        "v_min3_f16 %8, %8, |%7|, |%7| op_sel:[0,0,1,0]"
+        : "+v"(h[0]), "+v"(h[1]), "+v"(h[2]), "+v"(h[3]),
+          "+v"(h[4]), "+v"(h[5]), "+v"(h[6]), "+v"(h[7]), "+v"(least)
+        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]),
+          "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]),
+          "v"(a[8]), "v"(a[9]), "v"(a[10]), "v"(a[11]),
+          "v"(a[12]), "v"(a[13]), "v"(a[14]), "v"(a[15]), "v"(b));
+}
+
+__device__ __forceinline__ void mix_fnma_pairs4(const float* a, float b, uint32_t* h, uint32_t& least) {
+    asm volatile(
+        "v_fma_mixlo_f16 %0, -%3, %7, %0 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %1, -%5, %7, %1 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %0, -%4, %7, %0 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %1, -%6, %7, %1 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "s_nop 0\n\t"
+        "v_min3_f16 %2, %2, |%0|, |%0| op_sel:[0,0,1,0]\n\t"
+        "v_min3_f16 %2, %2, |%1|, |%1| op_sel:[0,0,1,0]"
+        : "+v"(h[0]), "+v"(h[1]), "+v"(least)
+        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b));
+}
+
 // B of an implicit-GEMM convolution: a thread's four columns n = n0 + 4 * (tid % (BN / 4)) + j are
 // the same in every slice (256 is a multiple of BN / 4); their output image, first input row
 // and column and base offset are computed once.  A column past N gets a row that puts every
@@ -278,6 +490,18 @@ struct ConvCols {
 // One BM x BN output tile of chunk sums of CHUNK (2..32) products; g.lda, g.ldb <= kChainMaxLd.
 constexpr int64_t kChainMaxLd = 1 << 22;   // a tile's offsets from its corner fit 32 bits
 
+// Statistics of an operand slice (chunk 1, 23 bits): the largest magnitude and a lower bound on
+// the exponent of every value's lowest set bit, as SliceStat's amax and key.
+struct SliceKey {
+    uint32_t amax = 0u, key = 0xFFFFFFFFu;
+    __device__ __forceinline__ void add(float v) {
+        const uint32_t b = __float_as_uint(v), sh = b << 1;
+        amax = max(amax, sh);
+        key = min(key, ((sh - 1u) >> 24) + min((uint32_t)__builtin_ctz(b | 0x80000000u), 24u));
+    }
+    __device__ __forceinline__ void add(const float4& v) { add(v.x); add(v.y); add(v.z); add(v.w); }
+};
+
 template <class T, int CHUNK, int KIND, bool CONV>
 __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, int tile_n, int tid,
                                                 float* smem) {
@@ -286,8 +510,17 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
     using LA = ChainLds<BM, BK, KI>;
     using LB = ChainLds<BN, BK, KI>;
     constexpr int NA4 = T::NA4, NB4 = T::NB4;
-    constexpr bool kFlag = KIND == kChainMant;
-    static_assert(CHUNK >= KI && BK % CHUNK == 0, "whole MFMAs per chunk, whole chunks per slice");
+    // per-slice flags: an infinity or NaN among the operands (kChainMant, and any kind's chunk 1
+    // but binary16's); a value that binary16 does not hold (binary16, chunk 1)
+    constexpr bool kStep = CHUNK == 1;
+    constexpr bool kF16Flag = kStep && KIND == kChainHalf;
+    constexpr bool kFlag = KIND == kChainMant || kStep;
+    // operand statistics: exact sums (23 bits), binary16's grid (10 bits)
+    constexpr bool kStat = kStep && (KIND == kChainMant23 || KIND == kChainMant10);
+    constexpr bool kWide = kStep && KIND == kChainMant10;   // a second flag: not binary16 operands
+    static_assert(kStep || (CHUNK >= KI && BK % CHUNK == 0),
+                  "whole MFMAs per chunk, whole chunks per slice");
+    constexpr float kPadA = kStep ? 0.0f : -0.0f;   // k past K, see the head comment
     using vec = typename std::conditional<BS == 32, f32x16, f32x4>::type;
 
     const int lane = tid & 63, wave = tid >> 6;
@@ -295,6 +528,7 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
     const int m0 = tile_m * BM, n0 = tile_n * BN;
     const int am0 = (wave / T::WC) * BS * WMB, bn0 = (wave % T::WC) * BS * WNB;
     uint32_t* flags = (uint32_t*)(smem + 2 * T::BUF_FLOATS);
+    uint32_t* stats = flags + 4;   // [buffer][wave][amax A, key A, amax B, key B]
 
     // Element mapping: float4 f = tid + 256 * it of the A slice is row m = f / (BK / 4),
     // k = 4 * (f % (BK / 4)) .. + 3 of a row-major A, or k = f / (BM / 4), m = 4 * (f % (BM / 4))
@@ -360,7 +594,7 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
     auto load_slice = [&](int k0) {
         const int kl = g.K - k0;
         load_op(va, std::integral_constant<int, BM>{}, A0 + (g.ta ? (int64_t)k0 * g.lda : (int64_t)k0),
-                g.ta != 0, g.lda, g.M - m0, kl, -0.0f);
+                g.ta != 0, g.lda, g.M - m0, kl, kPadA);
         if constexpr (CONV) {
             const int t = otid();
 #pragma unroll
@@ -376,6 +610,8 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
     auto store_slice = [&](int buf, int fl) {
         float* As = smem + buf * T::BUF_FLOATS;
         float z = 0.0f;   // 0 * v summed: NaN as soon as one v is not finite
+        bool wide = false;
+        SliceKey ka, kb;
         auto put = [&](float* S, auto lds, auto rows, const auto& v, bool kmaj) {
             using L = decltype(lds);
             constexpr int R = decltype(rows)::value, NV = R * BK / 1024;
@@ -395,7 +631,12 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
                     d[3 * R + (r ^ L::swz(3))] = v[it].w;
                 }
             }
-            if constexpr (kFlag) {
+            if constexpr (kF16Flag) {
+                auto w = [](float x) { return (float)(_Float16)x != x; };
+#pragma unroll
+                for (int it = 0; it < NV; ++it)
+                    wide |= w(v[it].x) | w(v[it].y) | w(v[it].z) | w(v[it].w);
+            } else if constexpr (kFlag) {
 #pragma unroll
                 for (int it = 0; it < NV; ++it) {
                     z = __builtin_fmaf(v[it].x, 0.0f, z);
@@ -408,23 +649,47 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
         put(As, LA{}, std::integral_constant<int, BM>{}, va, g.ta != 0);
         put(As + LA::FLOATS, LB{}, std::integral_constant<int, BN>{}, vb, CONV || g.tb == 0);
         if constexpr (kFlag)
-            if (z != 0.0f) flags[fl] = 1u;   // z is +-0 or NaN
+            if (wide || z != 0.0f) flags[fl] = 1u;   // z is +-0 or NaN
+        if constexpr (kWide) {   // A binary16 values, B of at most 11 significant bits
+            uint32_t low = 0u;
+#pragma unroll
+            for (int it = 0; it < NA4; ++it) {
+                auto w = [](float x) { return (float)(_Float16)x != x; };
+                wide |= w(va[it].x) | w(va[it].y) | w(va[it].z) | w(va[it].w);
+            }
+#pragma unroll
+            for (int it = 0; it < NB4; ++it)
+                low |= __float_as_uint(vb[it].x) | __float_as_uint(vb[it].y) |
+                       __float_as_uint(vb[it].z) | __float_as_uint(vb[it].w);
+            if (wide || (low & 0x1FFFu) != 0u) flags[fl + 36] = 1u;
+        }
+        if constexpr (kStat) {
+#pragma unroll
+            for (int it = 0; it < NA4; ++it) ka.add(va[it]);
+#pragma unroll
+            for (int it = 0; it < NB4; ++it) kb.add(vb[it]);
+            const uint4 w = make_uint4(wave_max_u32(ka.amax), wave_min_u32(ka.key),
+                                       wave_max_u32(kb.amax), wave_min_u32(kb.key));
+            if (lane == 63) *(uint4*)(stats + buf * 16 + wave * 4) = w;
+        }
     };
 
-    float acc[WMB][WNB][NR];   // kChainHalf: -acc, from -0
+    // the accumulators; kNeg: negated, from -0 (binary16, and every kind's chunk 1)
+    constexpr bool kNeg = KIND == kChainHalf || kStep;
+    float acc[WMB][WNB][NR];
 #pragma unroll
     for (int bi = 0; bi < WMB; ++bi)
 #pragma unroll
         for (int bj = 0; bj < WNB; ++bj)
 #pragma unroll
-            for (int r = 0; r < NR; ++r) acc[bi][bj][r] = KIND == kChainHalf ? -0.0f : 0.0f;
+            for (int r = 0; r < NR; ++r) acc[bi][bj][r] = kNeg ? -0.0f : 0.0f;
 
     // Leaves in pieces of PN outputs.  PIPE: a chunk's leaves run between the next chunk's
     // MFMAs, from its second step on (the first piece still waits for the sums to settle), so
     // one wave keeps both the matrix cores and the VALU busy; the leaf before the first chunk
     // works on zero sums, which leave zero accumulators as they are.  The wide tile (64 sums a
     // wave) has no registers for a second set.
-    constexpr int STEPS = CHUNK / KI;
+    constexpr int STEPS = kStep ? 1 : CHUNK / KI;
     constexpr int PN = NR == 4 ? 4 : 8, PIECES = WMB * WNB * NR / PN;
     constexpr bool PIPE = STEPS >= 2 && WMB * WNB * NR <= 32;
     constexpr int FIRST = STEPS >= 4 ? 1 : 0;
@@ -467,30 +732,421 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
     for (int bj = 0; bj < WNB; ++bj)
         rb[bj] = lhi * BN + ((bn0 + bj * BS + lcol) ^ LB::swz(lhi));
 
+    // ---- chunk 1: every k's leaf, on the negated accumulators
+    // Row quads of a lane's outputs (rows 8 rq + 4 lhi .. + 3 of a block) and its column, at the
+    // swizzle of k's place in its group of four.
+    auto a_quad = [&](const float* As, int k, int bi, int rq) -> float4 {
+        return *(const float4*)&As[LA::row(k) + ((am0 + bi * BS + rq * 8 + lhi * 4) ^ LA::swz(k))];
+    };
+    auto b_col = [&](const float* Bs, int k, int bj) -> float {
+        return Bs[LB::row(k) + ((bn0 + bj * BS + lcol) ^ LB::swz(k))];
+    };
+    // leaf(bi, bj, a, b) for every k < kmax, in groups of four k (those past K add -0): a group's
+    // next k is read while the current one computes
+    auto for_k = [&](const float* As, const float* Bs, int kmax, auto leaf) {
+        float a[2][WMB][NR], b[2][WNB];
+        auto fetch = [&](int set, const float* Ap, const float* Bp, int k) {
+#pragma unroll
+            for (int bi = 0; bi < WMB; ++bi)
+#pragma unroll
+                for (int rq = 0; rq < NR / 4; ++rq) {
+                    const float4 v = a_quad(Ap, k, bi, rq);
+                    a[set][bi][4 * rq + 0] = v.x;
+                    a[set][bi][4 * rq + 1] = v.y;
+                    a[set][bi][4 * rq + 2] = v.z;
+                    a[set][bi][4 * rq + 3] = v.w;
+                }
+#pragma unroll
+            for (int bj = 0; bj < WNB; ++bj) b[set][bj] = b_col(Bp, k, bj);
+        };
+        constexpr bool kAhead = NR == 4;
+        if constexpr (kAhead) fetch(0, As, Bs, 0);
+        const int ng = (kmax + 3) / 4;
+        for (int q = 0; q < ng; ++q) {
+            const float* Aq = As + q * LA::GROUP;
+            const float* Bq = Bs + q * LB::GROUP;
+            const int adv = q + 1 < ng ? 1 : 0;   // the last group reads its own first k again
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if constexpr (!kAhead) fetch(j & 1, Aq, Bq, j);
+                else if (j < 3) fetch((j + 1) & 1, Aq, Bq, j + 1);
+                else fetch(0, Aq + adv * LA::GROUP, Bq + adv * LB::GROUP, 0);
+#pragma unroll
+                for (int bi = 0; bi < WMB; ++bi)
+#pragma unroll
+                    for (int bj = 0; bj < WNB; ++bj) leaf(bi, bj, a[j & 1][bi], b[j & 1][bj]);
+            }
+        }
+    };
+    // The general leaf over a slice, out of line per leaf: slices with an infinity or a NaN, and
+    // binary16 sums that reach 65520 (or held values that are not binary16).
+    auto general_slice = [&](const float* As, const float* Bs, int kmax) {
+        const LeafGen L = leaf_gen(g);
+        for (int k = 0; k < kmax; ++k)
+#pragma unroll
+            for (int bi = 0; bi < WMB; ++bi)
+#pragma unroll
+                for (int bj = 0; bj < WNB; ++bj) {
+                    const float b = b_col(Bs, k, bj);
+#pragma unroll
+                    for (int rq = 0; rq < NR / 4; ++rq) {
+                        const float4 a4 = a_quad(As, k, bi, rq);
+                        const float av[4] = {a4.x, a4.y, a4.z, a4.w};
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) {
+                            float& na = acc[bi][bj][4 * rq + x];
+                            na = -(float)leaf_slow<LeafGen>((double)av[x] * (double)b, -(double)na, L);
+                        }
+                    }
+                }
+    };
+    uint32_t h[WMB][WNB][NR / 2];   // the accumulators as binary16 pairs while `held`
+    bool held = false;
+    int accL = 1000;   // 23 bits: every accumulator of the wave is a multiple of 2^accL
+    // to and from binary16 pairs scaled by 2^hs (exact both ways where they are used)
+    int hs = 0;
+    auto hold = [&](int to) {
+        hs = to;
+#pragma unroll
+        for (int bi = 0; bi < WMB; ++bi)
+#pragma unroll
+            for (int bj = 0; bj < WNB; ++bj)
+#pragma unroll
+                for (int r = 0; r < NR / 2; ++r)
+                    h[bi][bj][r] = __builtin_bit_cast(
+                        uint32_t, f16x2{(_Float16)__builtin_ldexpf(acc[bi][bj][2 * r], hs),
+                                        (_Float16)__builtin_ldexpf(acc[bi][bj][2 * r + 1], hs)});
+    };
+    auto unhold = [&]() {
+#pragma unroll
+        for (int bi = 0; bi < WMB; ++bi)
+#pragma unroll
+            for (int bj = 0; bj < WNB; ++bj)
+#pragma unroll
+                for (int r = 0; r < NR / 2; ++r) {
+                    const f16x2 v = __builtin_bit_cast(f16x2, h[bi][bj][r]);
+                    acc[bi][bj][2 * r] = __builtin_ldexpf((float)v.x, -hs);
+                    acc[bi][bj][2 * r + 1] = __builtin_ldexpf((float)v.y, -hs);
+                }
+    };
+    // every leaf by directed roundings
+    auto directed = [&](const float* As, const float* Bs, int kmax) {
+        for_k(As, Bs, kmax, [&](int bi, int bj, const float* a, float b) {
+            float (&x)[NR] = acc[bi][bj];
+            if constexpr (NR == 16) rto_fnma16(a, b, x);
+            else rto_fnma4(a, b, x);
+            if constexpr (KIND != kChainMant23)
+#pragma unroll
+                for (int r = 0; r < NR; ++r) {
+                    const uint32_t t = __float_as_uint(x[r]);
+                    x[r] = __uint_as_float((t + g.dr_half + __builtin_amdgcn_ubfe(t, g.dr_rf, 1u)) &
+                                           g.dr_mask);
+                }
+        });
+    };
+    auto step_slice = [&](const float* As, const float* Bs, int kmax, bool special, bool wide16,
+                          int buf) {
+        if constexpr (KIND == kChainHalf) {
+            // Held as binary16 pairs while every accumulator is a binary16 value below 2^15 at a
+            // slice's start.  The binary16 FMA (operands binary16 too: packed, two leaves an
+            // instruction) and the mixed one round the exact h - a b once, which is the leaf as long
+            // as no result passes 65504; an infinity or NaN stays one, so one look at the slice's
+            // end finds it, and the slice is redone from its start values.
+            if (!held) {
+                bool ok = true;
+#pragma unroll
+                for (int bi = 0; bi < WMB; ++bi)
+#pragma unroll
+                    for (int bj = 0; bj < WNB; ++bj)
+#pragma unroll
+                        for (int r = 0; r < NR; ++r) {
+                            const float x = acc[bi][bj][r];
+                            ok &= (float)(_Float16)x == x && fabsf(x) < 32768.0f;
+                        }
+                held = __all(ok);
+                if (held) hold(0);
+            }
+            if (held) {
+                uint32_t h0[WMB][WNB][NR / 2];
+#pragma unroll
+                for (int bi = 0; bi < WMB; ++bi)
+#pragma unroll
+                    for (int bj = 0; bj < WNB; ++bj)
+#pragma unroll
+                        for (int r = 0; r < NR / 2; ++r) h0[bi][bj][r] = h[bi][bj][r];
+                if (!special) {
+                    for_k(As, Bs, kmax, [&](int bi, int bj, const float* a, float b) {
+                        const _Float16 bv = (_Float16)b;
+#pragma unroll
+                        for (int r = 0; r < NR / 2; ++r) {
+                            const f16x2 av = {(_Float16)a[2 * r], (_Float16)a[2 * r + 1]};
+                            h[bi][bj][r] = __builtin_bit_cast(
+                                uint32_t, __builtin_elementwise_fma(
+                                              -av, f16x2{bv, bv},
+                                              __builtin_bit_cast(f16x2, h[bi][bj][r])));
+                        }
+                    });
+                } else {
+                    for_k(As, Bs, kmax, [&](int bi, int bj, const float* a, float b) {
+                        if constexpr (NR == 16) mix_fnma_pairs16(a, b, h[bi][bj]);
+                        else mix_fnma_pairs4(a, b, h[bi][bj]);
+                    });
+                }
+                bool over = false;
+#pragma unroll
+                for (int bi = 0; bi < WMB; ++bi)
+#pragma unroll
+                    for (int bj = 0; bj < WNB; ++bj)
+#pragma unroll
+                        for (int r = 0; r < NR / 2; ++r) {
+                            const uint32_t e = ~h[bi][bj][r];   // exponent all ones: inf or NaN
+                            over |= (e & 0x7C00u) == 0u || (e & 0x7C000000u) == 0u;
+                        }
+                const bool redo = __any(over);
+                if (redo) {
+#pragma unroll
+                    for (int bi = 0; bi < WMB; ++bi)
+#pragma unroll
+                        for (int bj = 0; bj < WNB; ++bj)
+#pragma unroll
+                            for (int r = 0; r < NR / 2; ++r) h[bi][bj][r] = h0[bi][bj][r];
+                    unhold();
+                }
+                held = !redo;
+            }
+            if (__builtin_expect(!held, 0)) general_slice(As, Bs, kmax);
+        } else {
+            if (__builtin_expect(special, 0)) {
+                general_slice(As, Bs, kmax);
+                accL = -1000;
+                return;
+            }
+            if constexpr (KIND == kChainMant23) {
+                // Exact sums: when every sum of 32 consecutive k is exact in FP32, each leaf is the
+                // plain FMA (RTO24 and the rounding keep an exact sum), and 32 of them are 32 / KI
+                // steps of the f32 MFMA on the negated accumulator, whose round-to-nearest zeros
+                // are the negated RTO24 zeros.  All sums are multiples of 2^L, L the lower of the
+                // products' lowest bit (from the slice's statistics) and the accumulators', and
+                // below 2^S with 2^S > |acc| + 33 amax_A amax_B: exact when S <= L + 24.
+                uint32_t amA = 0u, amB = 0u, kyA = ~0u, kyB = ~0u;
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    const uint4 v = *(const uint4*)(stats + buf * 16 + w * 4);
+                    amA = max(amA, v.x); kyA = min(kyA, v.y);
+                    amB = max(amB, v.z); kyB = min(kyB, v.w);
+                }
+                const int sL = amA == 0u || amB == 0u ? 1000 : (int)kyA + (int)kyB - 300;
+                // an upper bound on a product's magnitude, at least 2^-126
+                const float pm = fmaxf(__uint_as_float(amA >> 1) * __uint_as_float(amB >> 1), 0x1p-126f) *
+                                 1.0000152587890625f;
+                for (int kq = 0; kq < kmax; kq += 32) {
+                    float am = 0.0f;
+#pragma unroll
+                    for (int bi = 0; bi < WMB; ++bi)
+#pragma unroll
+                        for (int bj = 0; bj < WNB; ++bj)
+#pragma unroll
+                            for (int r = 0; r < NR; ++r) am = fmaxf(am, fabsf(acc[bi][bj][r]));
+                    const float bnd = __builtin_fmaf(33.0f, pm, am) * 1.0000152587890625f;
+                    const int S = (int)(__float_as_uint(bnd) >> 23) - 126;
+                    bool ok = S <= 127 && sL >= -149 && __all(S <= sL + 24);
+                    if (ok && accL < sL) {   // unknown or finer: the accumulators' own lowest bit
+                        if (accL == -1000) {
+                            uint32_t key = ~0u;
+#pragma unroll
+                            for (int bi = 0; bi < WMB; ++bi)
+#pragma unroll
+                                for (int bj = 0; bj < WNB; ++bj)
+#pragma unroll
+                                    for (int r = 0; r < NR; ++r) {
+                                        const uint32_t x = __float_as_uint(acc[bi][bj][r]);
+                                        key = min(key, (((x << 1) - 1u) >> 24) +
+                                                           min((uint32_t)__builtin_ctz(x | 0x80000000u), 24u));
+                                    }
+                            key = wave_min_u32(key);
+                            accL = (int)__builtin_amdgcn_readlane((int)key, 63) - 150;   // 129 for zeros
+                        }
+                        ok = accL >= -149 && __all(S <= min(sL, accL) + 24);
+                    }
+                    const float* Aq = As + kq / 4 * LA::GROUP;
+                    const float* Bq = Bs + kq / 4 * LB::GROUP;
+                    if (ok) {
+                        accL = min(accL, sL);
+                        vec c[WMB][WNB];
+#pragma unroll
+                        for (int bi = 0; bi < WMB; ++bi)
+#pragma unroll
+                            for (int bj = 0; bj < WNB; ++bj)
+#pragma unroll
+                                for (int r = 0; r < NR; ++r) c[bi][bj][r] = acc[bi][bj][r];
+#pragma unroll
+                        for (int i = 0; i < 32 / KI; ++i) {
+                            float a[WMB], b[WNB];
+#pragma unroll
+                            for (int bi = 0; bi < WMB; ++bi) a[bi] = -Aq[LA::row(KI * i) + ra[bi]];
+#pragma unroll
+                            for (int bj = 0; bj < WNB; ++bj) b[bj] = Bq[LB::row(KI * i) + rb[bj]];
+#pragma unroll
+                            for (int bi = 0; bi < WMB; ++bi)
+#pragma unroll
+                                for (int bj = 0; bj < WNB; ++bj) {
+                                    if constexpr (BS == 32)
+                                        c[bi][bj] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                                            a[bi], b[bj], c[bi][bj], 0, 0, 0);
+                                    else
+                                        c[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                                            a[bi], b[bj], c[bi][bj], 0, 0, 0);
+                                }
+                        }
+                        settle(c);
+#pragma unroll
+                        for (int bi = 0; bi < WMB; ++bi)
+#pragma unroll
+                            for (int bj = 0; bj < WNB; ++bj)
+#pragma unroll
+                                for (int r = 0; r < NR; ++r) acc[bi][bj][r] = c[bi][bj][r];
+                    } else {
+                        accL = -1000;
+                        directed(Aq, Bq, min(32, kmax - kq));
+                    }
+                }
+            } else if constexpr (KIND == kChainMant10) {
+                // 10 bits: binary16's significand, any exponent.  Held for 32 k as binary16 pairs
+                // scaled by 2^hs, hs the same for the wave: below 2^15, and from 2^-14 up, binary16 rounds a
+                // sum as the accumulator does.  Below 2^-14 it does too where every sum is a
+                // multiple of 2^-24 scaled (then it has at most 10 bits there); elsewhere the least
+                // result tells: above 2^-14, no sum was below.  Bounds per 32 k, for the wave: sums
+                // are below 2^S > (1 + 2^-11)^32 (|acc| + 33 amax_A amax_B), and multiples of 2^L as
+                // for exact sums (a rounding keeps a coarser or equal grid).
+                uint32_t amA = 0u, amB = 0u, kyA = ~0u, kyB = ~0u;
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    const uint4 v = *(const uint4*)(stats + buf * 16 + w * 4);
+                    amA = max(amA, v.x); kyA = min(kyA, v.y);
+                    amB = max(amB, v.z); kyB = min(kyB, v.w);
+                }
+                const bool zero = amA == 0u || amB == 0u;
+                const int sL = zero ? 1000 : (int)kyA + (int)kyB - 300;
+                const int bLsb = amB == 0u ? 1000 : (int)kyB - 150;
+                const int bTop = amB == 0u ? -1000 : (int)(amB >> 24) - 127;
+                const float pm = fmaxf(__uint_as_float(amA >> 1) * __uint_as_float(amB >> 1), 0x1p-126f) *
+                                 1.0000152587890625f;
+                for (int kq = 0; kq < kmax; kq += 32) {
+                    const float* Aq = As + kq / 4 * LA::GROUP;
+                    const float* Bq = Bs + kq / 4 * LB::GROUP;
+                    const int kn = min(32, kmax - kq);
+                    // the wave's largest and smallest accumulator magnitudes
+                    float hi_f = 0.0f, lo_f = 0x1.fffffep+127f;
+#pragma unroll
+                    for (int bi = 0; bi < WMB; ++bi)
+#pragma unroll
+                        for (int bj = 0; bj < WNB; ++bj)
+#pragma unroll
+                            for (int r = 0; r < NR; ++r) {
+                                hi_f = fmaxf(hi_f, fabsf(acc[bi][bj][r]));
+                                lo_f = fminf(lo_f, fabsf(acc[bi][bj][r]));
+                            }
+                    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane(
+                        (int)wave_max_u32(__float_as_uint(hi_f)), 63);
+                    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane(
+                        (int)wave_min_u32(__float_as_uint(lo_f)), 63);
+                    const float bnd = __builtin_fmaf(33.0f, pm, __uint_as_float(hi)) * 1.0158f;   // 1.015749...
+                    const int S = (int)(__float_as_uint(bnd) >> 23) - 126;
+                    const bool in = S <= 127;   // finite, and no overflow rule
+                    bool grid = in && !wide16 && sL >= -126 && S - sL <= 39;
+                    if (grid && accL == -1000) {   // unknown: the accumulators' own lowest bit
+                        uint32_t key = ~0u;
+#pragma unroll
+                        for (int bi = 0; bi < WMB; ++bi)
+#pragma unroll
+                            for (int bj = 0; bj < WNB; ++bj)
+#pragma unroll
+                                for (int r = 0; r < NR; ++r) {
+                                    const uint32_t x = __float_as_uint(acc[bi][bj][r]);
+                                    key = min(key, (((x << 1) - 1u) >> 24) +
+                                                       min((uint32_t)__builtin_ctz(x | 0x80000000u), 24u));
+                                }
+                        accL = __builtin_amdgcn_readlane((int)wave_min_u32(key), 63) - 150;   // 129 for zeros
+                    }
+                    const int L = min(sL, accL);
+                    // hs for the grid: 2^L to 2^-24 or above, 2^S to 2^15 or below, B within binary16
+                    const int gLo = max(-24 - L, -24 - bLsb), gHi = min(15 - S, 15 - bTop);
+                    grid = grid && L >= -126 && gLo <= gHi;
+                    if (grid) {
+                        accL = L;
+                        hold(gHi);
+                        for_k(Aq, Bq, kn, [&](int bi, int bj, const float* a, float b) {
+                            const _Float16 bv = (_Float16)__builtin_ldexpf(b, hs);
+#pragma unroll
+                            for (int r = 0; r < NR / 2; ++r) {
+                                const f16x2 av = {(_Float16)a[2 * r], (_Float16)a[2 * r + 1]};
+                                h[bi][bj][r] = __builtin_bit_cast(
+                                    uint32_t, __builtin_elementwise_fma(
+                                                  -av, f16x2{bv, bv},
+                                                  __builtin_bit_cast(f16x2, h[bi][bj][r])));
+                            }
+                        });
+                        unhold();
+                        continue;
+                    }
+                    accL = -1000;
+                    // checked: the smallest start value at 2^-14 or above scaled (so that all convert),
+                    // sums below 2^-126 seen too (hs <= 112), b 2^hs FP32-normal
+                    const int eLo = (int)(lo >> 23) - 127;
+                    const int cLo = max(-14 - eLo, -126 - bLsb), cHi = min(min(15 - S, 112), 126 - bTop);
+                    if (in && lo != 0u && cLo <= cHi) {
+                        hold(cHi);
+                        uint32_t least = 0x7BFFu;
+                        for_k(Aq, Bq, kn, [&](int bi, int bj, const float* a, float b) {
+                            const float bs = __builtin_ldexpf(b, hs);
+                            if constexpr (NR == 16) mix_fnma_pairs16(a, bs, h[bi][bj], least);
+                            else mix_fnma_pairs4(a, bs, h[bi][bj], least);
+                        });
+                        if (__all((least & 0xFFFFu) > 0x0400u)) {   // 2^-14
+                            unhold();
+                            continue;
+                        }
+                    }
+                    directed(Aq, Bq, kn);
+                }
+            } else {
+                directed(As, Bs, kmax);
+            }
+        }
+    };
+
     // Non-finite flags, three in turn: slice s reads flag s % 3 between its barrier and the next;
     // meanwhile the store of slice s + 1 sets flag (s + 1) % 3 and flag (s + 2) % 3 (read last by
     // slice s - 1, before this slice's barrier) is cleared for slice s + 2.
     if constexpr (kFlag) {
-        if (tid < 3) flags[tid] = 0u;
+        if (tid < 3) flags[tid] = flags[tid + 36] = 0u;
         lds_barrier();
     }
     int fs = 0, buf = 1;
     for (int k0 = -BK; k0 < g.K; k0 += BK) {   // the first pass only loads slice 0
-        bool special = false;
+        bool special = false, wide16 = false;
         if (k0 >= 0) lds_barrier();   // slice k0 is in buffer buf; the other one is free
         const int fn = k0 < 0 ? 0 : fs == 2 ? 0 : fs + 1;
         if constexpr (kFlag) {
             if (k0 >= 0) {
                 special = __builtin_amdgcn_readfirstlane((int)flags[fs]) != 0;
-                if (tid == 0) flags[fn == 2 ? 0 : fn + 1] = 0u;
+                if constexpr (kWide) wide16 = __builtin_amdgcn_readfirstlane((int)flags[fs + 36]) != 0;
+                if (tid == 0) {
+                    const int fc = fn == 2 ? 0 : fn + 1;
+                    flags[fc] = 0u;
+                    if constexpr (kWide) flags[fc + 36] = 0u;
+                }
             }
         }
         const bool has_next = k0 + BK < g.K;
         if (has_next) load_slice(k0 + BK);   // in flight while this slice computes
         const float* As = smem + buf * T::BUF_FLOATS;
         const float* Bs = As + LA::FLOATS;
+        if constexpr (kStep) {
+            if (k0 >= 0) step_slice(As, Bs, min(BK, g.K - k0), special, wide16, buf);
+        }
         // chunks that hold a k < K (none in the first pass)
-        const int nq = k0 < 0 ? 0 : min(BK, g.K - k0 + CHUNK - 1) / CHUNK;
+        const int nq = kStep || k0 < 0 ? 0 : min(BK, g.K - k0 + CHUNK - 1) / CHUNK;
         for (int q = 0; q < nq; ++q) {
             const int kb = q * CHUNK;
             // The chunk's k in groups of G MFMA steps (64 cycles of the matrix cores each group):
@@ -570,6 +1226,8 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
         for (int n = 0; n < PIECES; ++n) piece(prev, n, sprev);
     }
 
+    if constexpr (kStep && KIND == kChainHalf)
+        if (held) unhold();
     // epilogue (cutlass LinearCombination): D = alpha * acc, or fma(alpha, acc, beta * C);
     // a convolution's D(m, n) / C(m, n) sit at b * sdb + m * sdm + (p * Q + q) * sdpq
 #pragma unroll
@@ -587,7 +1245,7 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
             for (int r = 0; r < NR; ++r) {
                 const int gm = m0 + am0 + bi * BS + (r >> 2) * 8 + lhi * 4 + (r & 3);
                 if (gm >= g.M || gn >= g.N) continue;
-                const float a = KIND == kChainHalf ? -acc[bi][bj][r] : acc[bi][bj][r];
+                const float a = kNeg ? -acc[bi][bj][r] : acc[bi][bj][r];
                 float d;
                 if (g.beta != 0.0f)
                     d = __builtin_fmaf(g.alpha, a, g.beta * gld(g.C + (int64_t)gm * row_stride_c + col));

@@ -52,22 +52,23 @@ __global__ __launch_bounds__(256, kChainWaves<T>) void k_gemm_chain(GemmArgs g, 
 
 using ChainKernel = void (*)(GemmArgs, unsigned, unsigned);
 
-// [tile][log2(chunk) - 1]; nullptr where a chunk of 2 is shorter than the block's MFMA
+// [tile][log2(chunk)]; nullptr where a chunk of 2 is shorter than the block's MFMA, and for chunk
+// 1 on the widest tile
 struct ChainTable {
-    ChainKernel gemm[kChainTiles][5];
-    ChainKernel conv[kChainTiles][5];
+    ChainKernel gemm[kChainTiles][6];
+    ChainKernel conv[kChainTiles][6];
 };
 
 template <class T, int CHUNK, int KIND, bool CONV>
 constexpr ChainKernel chain_kernel() {
-    if constexpr (CHUNK >= T::KI) return k_gemm_chain<T, CHUNK, KIND, CONV>;
+    if constexpr (CHUNK == 1 ? T::WMB == 1 : CHUNK >= T::KI) return k_gemm_chain<T, CHUNK, KIND, CONV>;
     else return nullptr;
 }
 
 #define LOF_CHAIN_ROW(T, KIND, CONV)                                                        \
-    {chain_kernel<T, 2, KIND, CONV>(), chain_kernel<T, 4, KIND, CONV>(),                     \
-     chain_kernel<T, 8, KIND, CONV>(), chain_kernel<T, 16, KIND, CONV>(),                    \
-     chain_kernel<T, 32, KIND, CONV>()}
+    {chain_kernel<T, 1, KIND, CONV>(), chain_kernel<T, 2, KIND, CONV>(),                     \
+     chain_kernel<T, 4, KIND, CONV>(), chain_kernel<T, 8, KIND, CONV>(),                     \
+     chain_kernel<T, 16, KIND, CONV>(), chain_kernel<T, 32, KIND, CONV>()}
 // the convolution gathers its B slice, which costs the wide tiles more than it gives
 #define LOF_CHAIN_TABLE(KIND)                                                               \
     {{LOF_CHAIN_ROW(ChainT0, KIND, false), LOF_CHAIN_ROW(ChainT1, KIND, false),              \
@@ -76,7 +77,15 @@ constexpr ChainKernel chain_kernel() {
      {{}, LOF_CHAIN_ROW(ChainT1, KIND, true), LOF_CHAIN_ROW(ChainT2, KIND, true),            \
       LOF_CHAIN_ROW(ChainT3, KIND, true), {}}}
 
-extern const ChainTable kChainTableMant, kChainTableMant23, kChainTableHalf;
+// chunk 1 alone (longer chunks of a 10-bit accumulator are kChainMant's)
+#define LOF_CHAIN_ROW1(T, KIND, CONV) {chain_kernel<T, 1, KIND, CONV>(), {}, {}, {}, {}, {}}
+#define LOF_CHAIN_TABLE1(KIND)                                                              \
+    {{{}, LOF_CHAIN_ROW1(ChainT1, KIND, false), LOF_CHAIN_ROW1(ChainT2, KIND, false),        \
+      LOF_CHAIN_ROW1(ChainT3, KIND, false), LOF_CHAIN_ROW1(ChainT4, KIND, false)},           \
+     {{}, LOF_CHAIN_ROW1(ChainT1, KIND, true), LOF_CHAIN_ROW1(ChainT2, KIND, true),          \
+      LOF_CHAIN_ROW1(ChainT3, KIND, true), {}}}
+
+extern const ChainTable kChainTableMant, kChainTableMant10, kChainTableMant23, kChainTableHalf;
 
 // The dimensions of tile t.
 struct ChainDims { int bm, bn; };

@@ -1,6 +1,7 @@
-"""GPU parity of the chunk-sum kernels (chunks 2 to 32, every chunk sum an f32 MFMA chain): every
-tile, at the edges of tiles and slices, in all operand layouts and with odd leading dimensions,
-against the oracle bit for bit; and the f32 MFMA against the VALU fmaf chain."""
+"""GPU parity of the chunk-sum kernels (chunks 2 to 32, every chunk sum an f32 MFMA chain) and of
+their chunk-1 form (directed, binary16-held and exact-sum leaves): every tile, at the edges of
+tiles and slices, in all operand layouts and with odd leading dimensions, against the oracle bit
+for bit; and the f32 MFMA against the VALU fmaf chain."""
 import numpy as np
 import pytest
 import torch
@@ -67,7 +68,7 @@ def test_accumulators_and_values(dev, kind, values):
     import lofloat_amd as lof
     M, N, K = 33, 70, 131
     A, B = _operands(M, N, K, values, seed=11)
-    for chunk in (2, 4, 8, 16, 32):
+    for chunk in (1, 2, 4, 8, 16, 32):
         acc, oacc = _accums(lof, kind, chunk)
         ref = oracle.gemm(A, B, oacc, alpha=0.75)
         for cfg in CONFIGS:
@@ -83,7 +84,7 @@ def test_edges_and_layouts(dev, shape, odd):
     import lofloat_amd as lof
     M, N, K = shape
     A, B = _operands(M, N, K, "uniform", seed=M + N + K)
-    for kind, chunk in ((10, 8), (HALF, 32), (23, 4)):
+    for kind, chunk in ((10, 8), (HALF, 32), (23, 4), (7, 1), (HALF, 1), (23, 1)):
         acc, oacc = _accums(lof, kind, chunk)
         ref = oracle.gemm(A, B, oacc, alpha=0.75)
         for ta, tb in ((0, 0), (0, 1), (1, 0), (1, 1)):
@@ -92,7 +93,7 @@ def test_edges_and_layouts(dev, shape, odd):
                             f"{shape} {kind} chunk {chunk} ta {ta} tb {tb} config {cfg}")
 
 
-@pytest.mark.parametrize("chunk", [8, 32])
+@pytest.mark.parametrize("chunk", [1, 8, 32])
 @pytest.mark.parametrize("case", [(3, 20, 9, 9, 3, 1, 1), (2, 5, 13, 70, 3, 2, 1),
                                   (1, 33, 17, 130, 1, 1, 0), (2, 3, 20, 24, 7, 2, 3)], ids=str)
 def test_conv(dev, case, chunk):
@@ -108,6 +109,43 @@ def test_conv(dev, case, chunk):
             y = lof.conv2d(torch.from_numpy(x).to(dev), torch.from_numpy(w).to(dev), acc,
                            stride=stride, padding=pad, config=cfg).cpu().numpy()
             assert_bits(y, ref, f"conv {case} {kind} chunk {chunk} config {cfg}")
+
+
+@pytest.mark.parametrize("bits", [10, 23])
+@pytest.mark.parametrize("case", ["grows", "mixed", "zeros", "one_bit", "columns", "zero_a"])
+def test_chunk_1_leaf_changes(dev, case, bits):
+    """Chunk 1, 23 bits: slices whose sums are all exact run on the MFMA, the others leaf by leaf,
+    and a wave goes from one to the other as its accumulators grow (24 bits are passed about
+    half way), as columns of 24-bit values come in, over zero sums of both signs, and with one
+    inexact term in an otherwise exact product.  10 bits: from the packed binary16 leaves on the
+    grid to the checked and the directed ones and back, with columns 2^40 apart in a wave and a
+    zero operand slice beside large values."""
+    import lofloat_amd as lof
+    M, N, K = 70, 66, 520
+    g = np.random.default_rng(31)
+    A, B = (oracle.virtual_round(g.standard_normal(s).astype(np.float32).ravel(),
+                                 (8, 3, 7, 1, 0, 0)).reshape(s) for s in ((M, K), (K, N)))
+    if case == "grows":
+        A, B = np.abs(A) * 8, np.abs(B) * 8 + np.float32(2.0 ** -9)
+    elif case == "mixed":
+        A[:, 200:230] = g.standard_normal((M, 30)).astype(np.float32)
+    elif case == "zeros":
+        A[:, 1::2] = -A[:, ::2]
+        B[1::2] = B[::2]
+        A[3] = -0.0
+    elif case == "columns":
+        A = g.uniform(-1, 1, (M, K)).astype(np.float32)
+        B[:, ::7] *= np.float32(2.0 ** 40)
+    elif case == "zero_a":
+        A[:, 64:192] = 0.0
+        B[64:192] *= np.float32(2.0 ** 30)
+    else:
+        A[5, 300] = np.float32(1 + 2.0 ** -23)
+    acc, oacc = _accums(lof, bits, 1)
+    ref = oracle.gemm(A, B, oacc, alpha=0.75)
+    for cfg in CONFIGS:
+        for ta, tb in ((0, 1), (1, 0)):
+            assert_bits(_run(lof, A, B, acc, dev, ta, tb, cfg, False), ref, f"{case} config {cfg}")
 
 
 @pytest.mark.parametrize("scale", [0, 20, 60, 110, -60, -75])
