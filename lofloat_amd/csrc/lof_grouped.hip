@@ -2,14 +2,14 @@
 //
 // The plan uploads one GroupTask per job and the first tile index of each job (jobs are
 // ordered GEMMs first, largest first, then rounding jobs, largest first).  GEMMs with
-// k-chunk 8, 16 or 32 use the config's MFMA chunk-sum tile (64 x 64, 128 x 64 or 64 x 128),
-// the others the config's VALU tile.  The kernel is held to two workgroups per CU (launch
+// k-chunk 8, 16 or 32 use the config's MFMA chunk-sum tile (64 x 64, 128 x 64 or 64 x 128, or the
+// chunk-sum kernels' 32 x 32, which takes chunk 1 too), the others the config's VALU tile.  The kernel is held to two workgroups per CU (launch
 // bounds), which the 128 x 64 MFMA tile would otherwise drop to one, and the configs with
 // the 64 x 128 tile to three, as its single-GEMM kernel (measured 11.9 against 12.9 ms on
 // the 64-job benchmark mix, although the bound costs spills).  A fixed grid of
-// workgroups (as many as fit on the device at once) repeatedly claims the next tile with
-// an atomic counter, finds its job by binary search over the start indices, and runs the
-// job's tile routine: the same device routines as the single-job kernels, dispatched once
+// workgroups (as many as fit on the device at once) takes its first tiles by workgroup index and
+// repeatedly claims the next one with an atomic counter, finds its job among the start
+// indices, and runs the job's tile routine: the same device routines as the single-job kernels, dispatched once
 // per tile on the job's rounding mode.  The last workgroup to finish resets the counters,
 // so a replayed launch (e.g. from a HIP graph) needs no memset and no host work.
 #include <hip/hip_runtime.h>
@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "lof_gemm.hpp"
+#include "lof_gemm_chain_table.hpp"
 #include "lof_host.hpp"
 #include "lof_round_kernels.hpp"
 
@@ -59,7 +60,22 @@ struct GroupedCfg {
     static constexpr int bm = BM, bn = BN, tm = TM, tn = TN, bk = BK, sub = SUB;
     static constexpr int mfma_wmb = WMB;   // MFMA GEMM tile: (64 * WMB) x (64 * WNB)
     static constexpr int mfma_wnb = WNB;
+    static constexpr bool chain = false;
+    static constexpr int mfma_smem = MfmaTile<WMB, WNB>::SMEM_FLOATS;
+    static constexpr int per_cu = WNB == 2 ? 3 : 2;   // workgroups per CU the kernel is held to
     // floats per rounding / MX tile: SUB sub-tiles of 2048 floats
+    static constexpr int64_t round_tile_elems = (int64_t)SUB * kMxTileElems;
+};
+
+// The configs above inline the wave tile, whose 64 rows leave most CUs idle on small GEMMs.  This
+// one takes the 32 x 32 tile of the chunk-sum kernels for every GEMM they run at chunks 1, 8, 16 and
+// 32 (a 256^3 GEMM is 64 tiles of 4 slices instead of 8 tiles of 8), the VALU tile for the others.
+template <int SUB>
+struct GroupedChainCfg {
+    static constexpr int bm = 32, bn = 64, tm = 2, tn = 4, bk = 32, sub = SUB;
+    static constexpr bool chain = true;
+    static constexpr int mfma_smem = ChainT2::SMEM_FLOATS;
+    static constexpr int per_cu = 3;
     static constexpr int64_t round_tile_elems = (int64_t)SUB * kMxTileElems;
 };
 
@@ -134,25 +150,42 @@ __device__ __forceinline__ void grouped_mfma(const GemmArgs& g, int tm, int tn, 
 #undef LOF_GM
 }
 
+// The chunk-sum kernels' 32 x 32 tile by accumulator kind and chunk, on a copy of the arguments: read
+// through the task table they would be loaded again after every barrier.
+__device__ __forceinline__ void grouped_chain(const GemmArgs& task, int tm, int tn, int tid,
+                                              float* smem) {
+    const GemmArgs g = task;
+#define LOF_GK(C, KIND)                                                        \
+    if (g.chunk == C && g.chain == KIND) {                                     \
+        gemm_tile_chain<ChainT2, C, KIND, false>(g, tm, tn, tid, smem);        \
+        return;                                                                \
+    }
+#define LOF_GKC(KIND) LOF_GK(1, KIND) LOF_GK(8, KIND) LOF_GK(16, KIND) LOF_GK(32, KIND)
+    LOF_GKC(kChainHalf) LOF_GKC(kChainMant23) LOF_GKC(kChainMant) LOF_GK(1, kChainMant10)
+#undef LOF_GKC
+#undef LOF_GK
+}
+
 template <class C>
-__global__ __launch_bounds__(256, C::mfma_wnb == 2 ? 3 : 2) void k_grouped(const GroupTask* __restrict__ tasks,
+__global__ __launch_bounds__(256, C::per_cu) void k_grouped(const GroupTask* __restrict__ tasks,
                                                  const int64_t* __restrict__ starts, int ntasks,
                                                  int64_t total, unsigned long long* counters) {
     constexpr int kValuSmem = gemm_smem_floats<C::bm, C::bn, C::bk>();
-    constexpr int kMfmaSmem = MfmaTile<C::mfma_wmb, C::mfma_wnb>::SMEM_FLOATS;
+    constexpr int kMfmaSmem = C::mfma_smem;
     __shared__ __align__(16) float smem[kValuSmem > kMfmaSmem ? kValuSmem : kMfmaSmem];
     __shared__ unsigned long long s_tile;
     const int tid = threadIdx.x;
-    for (;;) {
-        if (tid == 0) s_tile = atomicAdd(&counters[0], 1ull);
-        lds_barrier();
-        const int64_t t = (int64_t)__builtin_amdgcn_readfirstlane((int)(s_tile & 0x7FFFFFFF));
-        lds_barrier();
-        if (t >= total) break;
-        int lo = 0, hi = ntasks - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (starts[mid] <= t) lo = mid; else hi = mid - 1;
+    // The first tile is the workgroup's own index (the grid is at most one workgroup per tile), the
+    // others come off the counter; a plan that fits the grid never touches it.
+    for (int64_t t = blockIdx.x;;) {
+        // the job of tile t: the starts at or below t, counted 64 at a time by the wave's lanes (one
+        // load for up to 64 jobs; a binary search is one dependent load per halving)
+        int lo = -1;
+        for (int b = 0; b < ntasks; b += 64) {
+            const int i = b + (tid & 63);
+            const uint64_t le = __builtin_amdgcn_ballot_w64(i < ntasks && starts[i] <= t);
+            lo += __popcll(le);
+            if (le != ~0ull) break;
         }
         const GroupTask& T = tasks[lo];
         const int64_t local = t - starts[lo];
@@ -167,10 +200,11 @@ __global__ __launch_bounds__(256, C::mfma_wnb == 2 ? 3 : 2) void k_grouped(const
             grouped_mx(T.x, T.mode, T.rsrc, local, C::sub, tid);
             break;
         default:
-            if (T.mfma)
-                grouped_mfma<C::mfma_wmb, C::mfma_wnb>(T.g, (int)(local / T.tiles_n), (int)(local % T.tiles_n),
-                                          tid, smem);
-            else if (T.g.subn)
+            if (T.mfma) {
+                const int tm = (int)(local / T.tiles_n), tn = (int)(local % T.tiles_n);
+                if constexpr (C::chain) grouped_chain(T.g, tm, tn, tid, smem);
+                else grouped_mfma<C::mfma_wmb, C::mfma_wnb>(T.g, tm, tn, tid, smem);
+            } else if (T.g.subn)
                 gemm_tile<C::bm, C::bn, C::tm, C::tn, C::bk, true>(
                     T.g, (int)(local / T.tiles_n), (int)(local % T.tiles_n), tid, smem);
             else
@@ -179,6 +213,12 @@ __global__ __launch_bounds__(256, C::mfma_wnb == 2 ? 3 : 2) void k_grouped(const
             lds_barrier();  // smem reuse by the next tile
             break;
         }
+        if (total <= (int64_t)gridDim.x) break;
+        if (tid == 0) s_tile = atomicAdd(&counters[0], 1ull) + gridDim.x;
+        lds_barrier();
+        t = (int64_t)__builtin_amdgcn_readfirstlane((int)(s_tile & 0x7FFFFFFF));
+        lds_barrier();
+        if (t >= total) break;
     }
     if (tid == 0) {
         __threadfence();
@@ -193,14 +233,15 @@ __global__ __launch_bounds__(256, C::mfma_wnb == 2 ? 3 : 2) void k_grouped(const
 struct GroupedConfig {
     const char* name;
     int bm, bn;
-    int mfma_bm, mfma_bn;   // MFMA GEMM tile (64 x 64, 128 x 64 or 64 x 128)
+    int mfma_bm, mfma_bn;   // MFMA GEMM tile (64 x 64, 128 x 64 or 64 x 128; 32 x 32)
+    bool chain;             // the MFMA GEMM tile is the chunk-sum kernels'
     int64_t round_tile_elems;
     void (*kernel)(const GroupTask*, const int64_t*, int, int64_t, unsigned long long*);
 };
 
 #define LOF_GCFG(BM, BN, TM, TN, BK, SUB, WMB, WNB)                                        \
     {#BM "x" #BN "/" #TM "x" #TN " r" #SUB " mfma" #WMB #WNB, BM, BN, 64 * WMB, 64 * WNB,   \
-     GroupedCfg<BM, BN, TM, TN, BK, SUB, WMB, WNB>::round_tile_elems,                     \
+     false, GroupedCfg<BM, BN, TM, TN, BK, SUB, WMB, WNB>::round_tile_elems,                     \
      k_grouped<GroupedCfg<BM, BN, TM, TN, BK, SUB, WMB, WNB>>}
 
 const GroupedConfig kGConfigs[] = {
@@ -212,9 +253,13 @@ const GroupedConfig kGConfigs[] = {
     LOF_GCFG(64, 64, 4, 4, 16, 8, 2, 1),
     LOF_GCFG(64, 64, 4, 4, 16, 4, 1, 2),
     LOF_GCFG(64, 64, 4, 4, 16, 8, 1, 2),
+    {"32x64/2x4 r4 mfma32x32", 32, 64, 32, 32, true, GroupedChainCfg<4>::round_tile_elems,
+     k_grouped<GroupedChainCfg<4>>},
 };
 constexpr int kNumGConfigs = sizeof(kGConfigs) / sizeof(kGConfigs[0]);
-int g_default_gconfig = 4;   // 64 x 64 VALU, 128 x 64 MFMA, 4 rounding sub-tiles
+constexpr int kChainGConfig = kNumGConfigs - 1;
+constexpr int kWaveGConfig = 4;   // 64 x 64 VALU, 128 x 64 MFMA, 4 rounding sub-tiles
+int g_default_gconfig = -1;       // the tuned config, -1: none yet
 std::mutex g_gmu;
 
 // Fixed device workspace of lof_grouped_run_noalloc: the work-queue counters, the job
@@ -260,6 +305,11 @@ struct lof_graph {
 
 namespace {
 
+bool grouped_mfma_chunk(int chunk) { return chunk == 8 || chunk == 16 || chunk == 32; }
+bool grouped_on_chain(const GemmArgs& g) {
+    return g.chain >= 0 && (g.chunk == 1 || grouped_mfma_chunk(g.chunk));
+}
+
 lof_status build_task(const lof_group_item& it, const GroupedConfig& cfg, GroupTask* t,
                       int64_t* tiles) {
     *t = GroupTask{};
@@ -286,8 +336,8 @@ lof_status build_task(const lof_group_item& it, const GroupedConfig& cfg, GroupT
     case LOF_ITEM_GEMM:
         s = prepare_gemm(&it.gemm, &t->g);
         if (s != LOF_OK) return s;
-        t->mfma = (it.gemm.accum.chunk == 8 || it.gemm.accum.chunk == 16 ||
-                   it.gemm.accum.chunk == 32) ? 1 : 0;
+        t->mfma = grouped_mfma_chunk(it.gemm.accum.chunk) ? 1 : 0;
+        if (cfg.chain) t->mfma = grouped_on_chain(t->g) ? 1 : 0;
         {
             const int bm = t->mfma ? cfg.mfma_bm : cfg.bm;
             const int bn = t->mfma ? cfg.mfma_bn : cfg.bn;
@@ -317,10 +367,21 @@ lof_status free_plan(lof_grouped* p) {
 }
 
 
-int resolve_gconfig(int config) {
+// The config asked for, else the tuned one, else the chunk-sum kernels' tile unless a GEMM of
+// chunk 8 to 32 has an accumulator they do not take (the wave tile then runs its chunk sums on MFMA;
+// here it would take the VALU tile).  An item that cannot be prepared is reported by build_task.
+int resolve_gconfig(int config, const lof_group_item* items, int count) {
     if (config >= 0) return config;
-    std::lock_guard<std::mutex> lk(g_gmu);
-    return g_default_gconfig;
+    {
+        std::lock_guard<std::mutex> lk(g_gmu);
+        if (g_default_gconfig >= 0) return g_default_gconfig;
+    }
+    for (int i = 0; i < count; ++i) {
+        if (items[i].kind != LOF_ITEM_GEMM || !grouped_mfma_chunk(items[i].gemm.accum.chunk)) continue;
+        GemmArgs g;
+        if (prepare_gemm(&items[i].gemm, &g) == LOF_OK && !grouped_on_chain(g)) return kWaveGConfig;
+    }
+    return kChainGConfig;
 }
 
 // Validates every item and lays the jobs out in queue order: GEMMs first, largest first,
@@ -394,6 +455,8 @@ lof_status launch_alone(const GroupTask& t, hipStream_t st) {
         d.trans_a = t.g.ta; d.trans_b = t.g.tb;
         d.accum.kind = t.g.acc_kind;
         d.accum.chunk = t.g.chunk;
+        if (t.g.chain >= 0 && (t.g.chunk > 1 || t.g.chain != kChainMant))
+            return launch_chain(t.g, chain_default_tile(t.g.M, t.g.N), st, "lof_grouped launch");
         return launch_gemm(t.g, resolve_gemm_config(d, -1), st);
     }
     }
@@ -433,7 +496,7 @@ LOF_API lof_status lof_grouped_create(const lof_group_item* items, int32_t count
     *plan = nullptr;
     if (config >= kNumGConfigs)
         return set_error(LOF_ERR_INVALID_ARGUMENT, "lof_grouped_create: config out of range");
-    config = resolve_gconfig(config);
+    config = resolve_gconfig(config, items, count);
     const GroupedConfig& cfg = kGConfigs[config];
     auto* p = new lof_grouped();
     p->config = config;
@@ -568,7 +631,7 @@ LOF_API lof_status lof_grouped_run_noalloc(const lof_group_item* items, int32_t 
                          "(use lof_grouped_create for larger lists)", count, kNoallocMaxItems);
     if (config >= kNumGConfigs)
         return set_error(LOF_ERR_INVALID_ARGUMENT, "lof_grouped_run_noalloc: config out of range");
-    config = resolve_gconfig(config);
+    config = resolve_gconfig(config, items, count);
     const GroupedConfig& cfg = kGConfigs[config];
     int device = 0;
     lof_status s = check_hip(hipGetDevice(&device), "hipGetDevice");
