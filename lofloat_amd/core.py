@@ -67,7 +67,7 @@ class FloatFormatDescriptor:
     """
 
     __slots__ = ("_total_bits", "_mantissa_bits", "_bias", "_inf_behavior", "_nan_behavior",
-                 "_signedness", "_is_inf_checker", "_is_nan_checker", "__weakref__")
+                 "_signedness", "_is_inf_checker", "_is_nan_checker", "_c_fmt", "__weakref__")
 
     def __init__(self, total_bits: int, mantissa_bits: int, bias: int,
                  inf_behavior: InfBehavior, nan_behavior: NaNBehavior, signedness: Signedness,
@@ -102,9 +102,18 @@ class FloatFormatDescriptor:
     is_nan_checker = property(lambda self: self._is_nan_checker)
 
     def c_format(self) -> _lib.Format:
-        return _lib.Format(self._total_bits, self._mantissa_bits, self._bias,
-                           int(self._inf_behavior), int(self._nan_behavior),
-                           int(self._signedness))
+        """The C struct of these fields (read-only, built once; callers copy it)."""
+        try:
+            return self._c_fmt
+        except AttributeError:
+            self._c_fmt = _lib.Format(self._total_bits, self._mantissa_bits, self._bias,
+                                      int(self._inf_behavior), int(self._nan_behavior),
+                                      int(self._signedness))
+            return self._c_fmt
+
+    def __getstate__(self):   # without the C struct, which is rebuilt
+        return None, {n: getattr(self, n) for n in self.__slots__
+                      if n not in ("_c_fmt", "__weakref__")}
 
     def as_tuple(self) -> tuple:
         return (self._total_bits, self._mantissa_bits, self._bias, int(self._inf_behavior),

@@ -179,6 +179,8 @@ def _lof_gemm_2d(A, B, accum_mant_bits, gemm_round_mode, stochastic_rounding_bit
 
 
 def _alpha(scale_a: float, scale_b: float) -> float:
+    if scale_a == 1.0 and scale_b == 1.0:
+        return 1.0
     import numpy as np
     denom = np.float32(scale_a) * np.float32(scale_b)
     return 1.0 if denom == 0 else float(np.float32(1.0) / denom)

@@ -21,7 +21,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .core import FloatFormatDescriptor, RoundingMode
+from .core import STOCHASTIC_MODES, FloatFormatDescriptor, RoundingMode
 
 _seed_lock = threading.Lock()
 _seed_state = {"seed": 12345, "calls": 0}
@@ -43,8 +43,28 @@ def next_seed() -> int:
     return (int(hi) << 32) | int(lo)
 
 
-def _stream(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+def _stream(t: torch.Tensor) -> int:
+    """The raw HIP stream that torch works on now, on t's device."""
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
+
+
+class _Here:
+    """A context that does nothing."""
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        return False
+
+
+_HERE = _Here()
+
+
+def _on_device(t: torch.Tensor):
+    """t's device made current; nothing to do when it is (a context switch there and back costs
+    a small launch two microseconds)."""
+    return _HERE if torch._C._cuda_getDevice() == t.device.index else torch.cuda.device(t.device)
 
 
 def _require_device_f32(t: torch.Tensor, what: str) -> None:
@@ -73,22 +93,22 @@ def _bits_ptr(rand_bits, ref: torch.Tensor, what: str):
     if rand_bits.device != ref.device or rand_bits.numel() != ref.numel():
         raise ValueError(f"{what}: rand_bits needs one word per element on {ref.device}")
     rb = rand_bits.contiguous()
-    return ctypes.c_void_p(rb.data_ptr()), rb
+    return rb.data_ptr(), rb
+
+
+_MODES = frozenset(int(m) for m in RoundingMode)
+_STOCHASTIC = frozenset(int(m) for m in STOCHASTIC_MODES)
 
 
 def _mode(m) -> int:
-    return int(RoundingMode(int(m)))
+    m = int(m)
+    return m if m in _MODES else int(RoundingMode(m))   # the enum raises for any other integer
 
 
 def _seed_for(mode: int, seed) -> int:
     if seed is not None:
         return int(seed) & 0xFFFFFFFFFFFFFFFF
-    if RoundingMode(mode) in (RoundingMode.StochasticRoundingA, RoundingMode.StochasticRoundingB,
-                              RoundingMode.StochasticRoundingC, RoundingMode.StochasticRoundingD,
-                              RoundingMode.True_StochasticRounding,
-                              RoundingMode.ProbabilisticRounding):
-        return next_seed()
-    return 0
+    return next_seed() if mode in _STOCHASTIC else 0
 
 
 def virtual_round(input: torch.Tensor, params, round_mode=RoundingMode.RoundToNearestEven,
@@ -107,17 +127,16 @@ def virtual_round(input: torch.Tensor, params, round_mode=RoundingMode.RoundToNe
     bptr, keep = _bits_ptr(rand_bits, x, "virtual_round")
     spec = _lib.RoundSpec(mode, 0, int(stoch_len))
     s = _seed_for(mode, seed)
-    sc = float(np.float32(scale))  # static_cast<float>(scale); the kernel multiplies in FP32
-    with torch.cuda.device(x.device):
+    sc = float(scale)  # the C float argument is static_cast<float>(scale)
+    with _on_device(x):
         if isinstance(params, FloatFormatDescriptor):
-            fmt = params.c_format()
             st = _lib.lib.lof_virtual_round_f32(
-                ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(y.data_ptr()), x.numel(),
-                ctypes.byref(fmt), spec, sc, bptr, s, _stream(x))
+                x.data_ptr(), y.data_ptr(), x.numel(), ctypes.byref(params.c_format()), spec, sc,
+                bptr, s, _stream(x))
         elif isinstance(params, int) and not isinstance(params, bool):
             st = _lib.lib.lof_virtual_round_mant_f32(
-                ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(y.data_ptr()), x.numel(),
-                int(params), spec, sc, bptr, s, _stream(x))
+                x.data_ptr(), y.data_ptr(), x.numel(), int(params), spec, sc, bptr, s,
+                _stream(x))
         else:
             raise TypeError("virtual_round: params must be a FloatFormatDescriptor or an int "
                             "number of mantissa bits")
@@ -144,9 +163,9 @@ def virtual_mx_round(input: torch.Tensor, block_size: int, element_format: Float
     mode = _mode(round_mode)
     bptr, keep = _bits_ptr(rand_bits, x, "virtual_mx_round")
     ef, sf = element_format.c_format(), scale_format.c_format()
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         st = _lib.lib.lof_virtual_mx_round_f32(
-            ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(y.data_ptr()), x.numel(),
+            x.data_ptr(), y.data_ptr(), x.numel(),
             int(block_size), ctypes.byref(ef), ctypes.byref(sf),
             _lib.RoundSpec(mode, 0, int(stoch_len)), _mode(scale_round_mode), bptr,
             _seed_for(mode, seed), _stream(x))
@@ -158,7 +177,7 @@ def virtual_mx_round(input: torch.Tensor, block_size: int, element_format: Float
 def fill_random_u32(n: int, seed: int, device="cuda", offset: int = 0) -> torch.Tensor:
     """A uint32 tensor of n counter-based random words lof_rand_u32(seed, offset + i)."""
     t = torch.empty(int(n), dtype=torch.uint32, device=device)
-    with torch.cuda.device(t.device):
+    with _on_device(t):
         st = _lib.lib.lof_fill_random_u32(ctypes.c_void_p(t.data_ptr()), int(n),
                                           int(seed) & 0xFFFFFFFFFFFFFFFF, int(offset), _stream(t))
     _lib.check(st, "fill_random_u32")
@@ -168,6 +187,9 @@ def fill_random_u32(n: int, seed: int, device="cuda", offset: int = 0) -> torch.
 # ------------------------------------------------------------------------------------
 # emulated-accumulation GEMM
 # ------------------------------------------------------------------------------------
+_NO_FORMAT = _lib.Format(0, 0, 0, 0, 0, 0)
+
+
 @dataclass(frozen=True)
 class AccumSpec:
     """How the FP32 accumulator is re-rounded.  ``fmt=None``: mantissa-only to
@@ -179,11 +201,11 @@ class AccumSpec:
     mode: int = int(RoundingMode.RoundToNearestEven)
 
     def c_accum(self) -> _lib.Accum:
+        """The C struct of these (frozen) fields; callers copy it."""
+        spec = _lib.RoundSpec(int(self.mode), 0, 0)
         if self.fmt is None:
-            return _lib.Accum(0, int(self.mant_bits), _lib.Format(0, 0, 0, 0, 0, 0),
-                              _lib.RoundSpec(int(self.mode), 0, 0), int(self.chunk))
-        return _lib.Accum(1, 0, self.fmt.c_format(), _lib.RoundSpec(int(self.mode), 0, 0),
-                          int(self.chunk))
+            return _lib.Accum(0, int(self.mant_bits), _NO_FORMAT, spec, int(self.chunk))
+        return _lib.Accum(1, 0, self.fmt.c_format(), spec, int(self.chunk))
 
 
 def _mat_view(t: torch.Tensor, what: str):
@@ -219,9 +241,12 @@ def gemm(A: torch.Tensor, B: torch.Tensor, accum: AccumSpec, alpha: float = 1.0,
     Bv, ldb, tb = _mat_view(B, "lof_gemm B")
     _require_same_device(out, A, "lof_gemm: out")
     _require_same_device(C if beta != 0.0 else None, A, "lof_gemm: C")
-    D = torch.empty((M, N), dtype=torch.float32, device=A.device) if out is None else out
-    if D.shape != (M, N) or not D.is_contiguous() or D.dtype != torch.float32:
-        raise ValueError("lof_gemm: out must be a contiguous float32 (M, N) tensor")
+    if out is None:
+        D = torch.empty((M, N), dtype=torch.float32, device=A.device)
+    else:
+        D = out
+        if D.shape != (M, N) or not D.is_contiguous() or D.dtype != torch.float32:
+            raise ValueError("lof_gemm: out must be a contiguous float32 (M, N) tensor")
     if M == 0 or N == 0:
         return D
     Cc = None
@@ -233,7 +258,7 @@ def gemm(A: torch.Tensor, B: torch.Tensor, accum: AccumSpec, alpha: float = 1.0,
     desc = _lib.GemmDesc(M, N, K, Av.data_ptr(), lda, int(ta), Bv.data_ptr(), ldb, int(tb),
                          D.data_ptr(), max(N, 1), float(alpha), accum.c_accum(),
                          Cc.data_ptr() if Cc is not None else None, max(N, 1), float(beta))
-    with torch.cuda.device(A.device):
+    with _on_device(A):
         st = _lib.lib.lof_gemm_f32(ctypes.byref(desc), int(config), _stream(A))
     _lib.check(st, "lof_gemm")
     return D
@@ -247,9 +272,11 @@ def lof_gemm(A: torch.Tensor, B: torch.Tensor, accum_mant_bits: int,
     reference kernel, the accumulator always rounds to nearest even: ``round_mode`` and
     ``stochastic_rounding_bits`` are accepted and ignored (cutlass_gemms.cuh:122)."""
     RoundingMode(int(round_mode))
-    # run_scaled (cutlass_gemms.cuh:1777-1787), all in float
-    denom = np.float32(scale_a) * np.float32(scale_b)
-    alpha = 1.0 if denom == 0 else float(np.float32(1.0) / denom)
+    if scale_a == 1.0 and scale_b == 1.0:
+        alpha = 1.0
+    else:   # run_scaled (cutlass_gemms.cuh:1777-1787), all in float
+        denom = np.float32(scale_a) * np.float32(scale_b)
+        alpha = 1.0 if denom == 0 else float(np.float32(1.0) / denom)
     return gemm(A, B, AccumSpec(mant_bits=int(accum_mant_bits), chunk=1), alpha=alpha)
 
 
@@ -316,7 +343,7 @@ def conv2d(x: torch.Tensor, w: torch.Tensor, accum: AccumSpec, stride=1, padding
                            xc.data_ptr(), wc.data_ptr(), y.data_ptr(), float(alpha),
                            accum.c_accum(), Cc.data_ptr() if Cc is not None else None,
                            float(beta))
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         st = _lib.lib.lof_conv2d_f32(ctypes.byref(desc), int(config), _stream(x))
     _lib.check(st, "conv2d")
     return y
@@ -366,7 +393,7 @@ def pwl_silu(input: torch.Tensor, lut: torch.Tensor, R: float) -> torch.Tensor:
     x = input.contiguous()
     t = lut.to(device=x.device, dtype=torch.float32).contiguous()
     y = torch.empty_like(x)
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         st = _lib.lib.lof_pwl_silu(ctypes.c_void_p(y.data_ptr()), ctypes.c_void_p(x.data_ptr()),
                                    x.numel(), dt, ctypes.c_void_p(t.data_ptr()), t.numel() - 1,
                                    float(R), _stream(x))
@@ -399,7 +426,7 @@ def gemm_autotune(A: torch.Tensor, B: torch.Tensor, accum: AccumSpec, iters: int
     desc = _lib.GemmDesc(M, N, K, Av.data_ptr(), lda, int(ta), Bv.data_ptr(), ldb, int(tb),
                          D.data_ptr(), N, 1.0, accum.c_accum())
     best, ms = ctypes.c_int32(-1), ctypes.c_float(0.0)
-    with torch.cuda.device(A.device):
+    with _on_device(A):
         st = _lib.lib.lof_gemm_autotune(ctypes.byref(desc), int(iters), _stream(A),
                                         ctypes.byref(best), ctypes.byref(ms))
     _lib.check(st, "gemm_autotune")

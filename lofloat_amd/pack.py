@@ -16,7 +16,7 @@ import torch
 
 from . import _lib
 from .core import FloatFormatDescriptor, RoundingMode
-from .ops import _bits_ptr, _mode, _require_device_f32, _seed_for, _stream
+from .ops import _bits_ptr, _mode, _on_device, _require_device_f32, _seed_for, _stream
 
 __all__ = ["packed_size", "encode", "decode", "pack_reps", "unpack_reps", "pack_format",
            "rep_dtype", "to_reps", "from_reps"]
@@ -71,7 +71,7 @@ def encode(input: torch.Tensor, params: FloatFormatDescriptor,
                          f">= {nbytes} bytes")
     mode = _mode(round_mode)
     bptr, keep = _bits_ptr(rand_bits, x, "pack.encode")
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         st = _lib.lib.lof_pack_encode_f32(
             ctypes.c_void_p(y.data_ptr()), ctypes.c_void_p(x.data_ptr()), x.numel(),
             ctypes.byref(pf), _lib.RoundSpec(mode, int(saturation), int(stoch_len)),
@@ -95,7 +95,7 @@ def decode(buf: torch.Tensor, params: FloatFormatDescriptor, count: int, endian=
         raise ValueError(f"pack.decode: out must be on {buf.device} (got {y.device})")
     if y.dtype != torch.float32 or y.numel() != count or not y.is_contiguous():
         raise ValueError("pack.decode: out must be a contiguous float32 tensor of count elements")
-    with torch.cuda.device(buf.device):
+    with _on_device(buf):
         st = _lib.lib.lof_pack_decode_f32(ctypes.c_void_p(y.data_ptr()),
                                           ctypes.c_void_p(buf.data_ptr()), int(count),
                                           ctypes.byref(pf), _ENDIAN[endian], _stream(buf))
@@ -109,7 +109,7 @@ def pack_reps(reps: torch.Tensor, bitwidth: int, endian="forward") -> torch.Tens
         raise RuntimeError("pack.pack_reps: reps must be an int32 / uint32 device tensor")
     r = reps.contiguous().reshape(-1)
     y = torch.empty(packed_size(bitwidth, r.numel()), dtype=torch.uint8, device=r.device)
-    with torch.cuda.device(r.device):
+    with _on_device(r):
         st = _lib.lib.lof_pack_reps(ctypes.c_void_p(y.data_ptr()), ctypes.c_void_p(r.data_ptr()),
                                     r.numel(), int(bitwidth), _ENDIAN[endian], _stream(r))
     _lib.check(st, "pack.pack_reps")
@@ -123,7 +123,7 @@ def unpack_reps(buf: torch.Tensor, bitwidth: int, count: int, endian="forward") 
     if buf.numel() < packed_size(bitwidth, count):
         raise ValueError("pack.unpack_reps: buf is shorter than packed_size(bitwidth, count)")
     y = torch.empty(int(count), dtype=torch.int32, device=buf.device)
-    with torch.cuda.device(buf.device):
+    with _on_device(buf):
         st = _lib.lib.lof_unpack_reps(ctypes.c_void_p(y.data_ptr()),
                                       ctypes.c_void_p(buf.data_ptr()), int(count),
                                       int(bitwidth), _ENDIAN[endian], _stream(buf))
@@ -158,7 +158,7 @@ def to_reps(input: torch.Tensor, params: FloatFormatDescriptor,
         raise ValueError(f"to_reps: out must be a contiguous {dt} tensor of shape {tuple(x.shape)}")
     mode = _mode(round_mode)
     bptr, keep = _bits_ptr(rand_bits, x, "to_reps")
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         st = _lib.lib.lof_cast_to_rep_f32(
             ctypes.c_void_p(y.data_ptr()), ctypes.c_void_p(x.data_ptr()), x.numel(),
             ctypes.byref(pf), _lib.RoundSpec(mode, int(saturation), int(stoch_len)), bptr,
@@ -181,7 +181,7 @@ def from_reps(reps: torch.Tensor, params: FloatFormatDescriptor, *, unsigned_beh
     y = torch.empty(r.shape, dtype=torch.float32, device=r.device) if out is None else out
     if y.dtype != torch.float32 or y.shape != r.shape or not y.is_contiguous():
         raise ValueError("from_reps: out must be a contiguous float32 tensor of reps' shape")
-    with torch.cuda.device(r.device):
+    with _on_device(r):
         st = _lib.lib.lof_cast_from_rep_f32(ctypes.c_void_p(y.data_ptr()),
                                             ctypes.c_void_p(r.data_ptr()), r.numel(),
                                             ctypes.byref(pf), _stream(r))
