@@ -351,6 +351,53 @@ __device__ __forceinline__ void rto_fnma4(const float* a, float b, float* na) {
         : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b));
 }
 
+// Launches of at most a block a CU, one wave a SIMD.
+constexpr unsigned kOneWaveBlocks = 256;
+
+// The same for four outputs while round-down holds (between round_down and round_nearest): the
+// rounding up is the negated rounding down of the negated sum, one instruction more a leaf and no
+// mode switch, whose waits a single wave's four leaves cannot cover (8x4096x4096 on FP32 operands,
+// 23 bits, one wave a SIMD: 367 us with rto_fnma4, 338 us so; 1000x768x3072, three blocks a
+// CU, 375 and 403 us).
+__device__ __forceinline__ void rto_fnma4_down(const float* a, float b, float* na) {
+    float d[4], m[4];
+    asm(
+        "v_fma_f32 %4, -%12, %16, %0\n\t"
+        "v_fma_f32 %5, -%13, %16, %1\n\t"
+        "v_fma_f32 %6, -%14, %16, %2\n\t"
+        "v_fma_f32 %7, -%15, %16, %3\n\t"
+        "v_fma_f32 %0, %12, %16, -%0\n\t"
+        "v_fma_f32 %1, %13, %16, -%1\n\t"
+        "v_fma_f32 %2, %14, %16, -%2\n\t"
+        "v_fma_f32 %3, %15, %16, -%3\n\t"
+        "v_bfe_i32 %8, %4, 0, 1\n\t"
+        "v_bfe_i32 %9, %5, 0, 1\n\t"
+        "v_bfe_i32 %10, %6, 0, 1\n\t"
+        "v_bfe_i32 %11, %7, 0, 1\n\t"
+        "v_xor_b32 %0, 0x80000000, %0\n\t"
+        "v_xor_b32 %1, 0x80000000, %1\n\t"
+        "v_xor_b32 %2, 0x80000000, %2\n\t"
+        "v_xor_b32 %3, 0x80000000, %3\n\t"
+        "v_bfi_b32 %0, %8, %4, %0\n\t"
+        "v_bfi_b32 %1, %9, %5, %1\n\t"
+        "v_bfi_b32 %2, %10, %6, %2\n\t"
+        "v_bfi_b32 %3, %11, %7, %3"
+        : "+v"(na[0]), "+v"(na[1]), "+v"(na[2]), "+v"(na[3]),
+          "=&v"(d[0]), "=&v"(d[1]), "=&v"(d[2]), "=&v"(d[3]),
+          "=&v"(m[0]), "=&v"(m[1]), "=&v"(m[2]), "=&v"(m[3])
+        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b));
+}
+// Enter and leave round-down.  The accumulators pass through both statements, so nothing computed
+// from them moves into the region.
+__device__ __forceinline__ void round_down(float (&x)[4]) {
+    asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 2\n\ts_nop 1"
+                 : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]));
+}
+__device__ __forceinline__ void round_nearest(float (&x)[4]) {
+    asm volatile("s_nop 1\n\ts_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0\n\ts_nop 1"
+                 : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]));
+}
+
 // h <- binary16(h - a b), one rounding of the exact difference (see mix_fnma16), for the
 // binary16 pairs h[i] = (h[2 i], h[2 i + 1]); the low halves first, so that no instruction follows
 // the one that wrote half of its register.
@@ -831,9 +878,10 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
     };
     // every leaf by directed roundings
     auto directed = [&](const float* As, const float* Bs, int kmax) {
-        for_k(As, Bs, kmax, [&](int bi, int bj, const float* a, float b) {
+        auto leaf = [&](auto down, int bi, int bj, const float* a, float b) {
             float (&x)[NR] = acc[bi][bj];
             if constexpr (NR == 16) rto_fnma16(a, b, x);
+            else if constexpr (down.value) rto_fnma4_down(a, b, x);
             else rto_fnma4(a, b, x);
             if constexpr (KIND != kChainMant23)
 #pragma unroll
@@ -842,6 +890,20 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
                     x[r] = __uint_as_float((t + g.dr_half + __builtin_amdgcn_ubfe(t, g.dr_rf, 1u)) &
                                            g.dr_mask);
                 }
+        };
+        if constexpr (NR == 4) {
+            static_assert(WMB * WNB == 1, "one block of four outputs a lane");
+            if (gridDim.x <= kOneWaveBlocks) {
+                round_down(acc[0][0]);
+                for_k(As, Bs, kmax, [&](int bi, int bj, const float* a, float b) {
+                    leaf(std::true_type{}, bi, bj, a, b);
+                });
+                round_nearest(acc[0][0]);
+                return;
+            }
+        }
+        for_k(As, Bs, kmax, [&](int bi, int bj, const float* a, float b) {
+            leaf(std::false_type{}, bi, bj, a, b);
         });
     };
     auto step_slice = [&](const float* As, const float* Bs, int kmax, bool special, bool wide16,
