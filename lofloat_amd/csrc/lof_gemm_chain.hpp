@@ -1,5 +1,5 @@
-// lof_gemm_chain.hpp -- emulated-accumulation GEMM tile for chunks of 2 to 32, with every chunk
-// sum on the f32 matrix cores (gfx950).
+// lof_gemm_chain.hpp -- emulated-accumulation GEMM tile for chunks of 1 to 32 (gfx950): chunk
+// sums of 2 to 32 products on the f32 matrix cores, chunk 1 leaf by leaf.
 //
 // For chunk c > 1 the rule is: p = FP32 fmaf chain over the chunk's c products in ascending
 // k, from +0, then acc <- round(RTO24(p + acc)).  v_mfma_f32_32x32x2_f32 and
@@ -23,6 +23,20 @@
 //                               top binade (or 2^15) redo the leaf in its general form.
 // A slice with an infinity or a NaN among its operands has the NaN sums brought to one pattern
 // before the leaf, so that rounding cannot carry a payload out of the NaN range.
+//
+// Chunk 1 (acc <- round(RTO24(a b + acc)) for every k) works on the negated accumulators; what
+// bounds it is VALU issue.  Cycles a wave on gfx950, measured with four waves a SIMD: FP32 add,
+// multiply, FMA and 32-bit logic 2.5 to 3, v_bfi_b32, v_bfe_i32, conversions and v_pk_fma_f16
+// (two leaves) 4.4, v_fma_mixlo_f16 and v_min3_f16 8.4, v_min_f16 2.6.  By accumulator:
+//   any mantissa                two directed FMAs and the odd one of them (rto_fnma16), 15 cycles a
+//                               leaf, and three instructions more below 23 bits;
+//   23 bits, exact sums         the f32 MFMA (4 cycles a leaf);
+//   binary16-shaped, 10 bits    one binary16 FMA on binary16 operands, two leaves an instruction,
+//                               from slices kept as binary16 pairs (2.2 cycles a leaf); one
+//                               mixed FMA on FP32 operands (8.4; 10 bits: 2.6 more for the check).
+// e4m3 operands, 10 bits, before and after the slices were kept as binary16 pairs: 4096^3 3.6 ->
+// 2.28 ms, 1000x768x3072 259 -> 196 us, a 3x3 convolution 128x25088x1152 290 -> 190 us; binary16-
+// shaped: 1.84 ms, 133 us, 152 us.
 //
 // Tile: 4 waves, each WMB x WNB blocks of BS x BS outputs (BS = 32, or 16 for products with few
 // outputs, where a 32-row block would leave most of the chip idle).  A and B slices of BK k sit
@@ -68,7 +82,7 @@ struct ChainTile {
     static constexpr int NR = BS * BS / 64;        // outputs per lane and block
     static constexpr int KI = BS == 32 ? 2 : 4;    // k per MFMA
     static constexpr int BUF_FLOATS = ChainLds<BM, BK, KI>::FLOATS + ChainLds<BN, BK, KI>::FLOATS;
-    static constexpr int SMEM_FLOATS = 2 * BUF_FLOATS + 40;   // + 3 flags, statistics, 3 flags
+    static constexpr int SMEM_FLOATS = 2 * BUF_FLOATS + 44;   // + 3 flags, statistics, 2 x 3 flags
     static constexpr int NA4 = BM * BK / 1024, NB4 = BN * BK / 1024;   // float4 per thread
     static_assert(NA4 * 1024 == BM * BK && NB4 * 1024 == BN * BK, "whole float4s per thread");
 };
@@ -232,45 +246,45 @@ __device__ __forceinline__ void chain_leaves(float (&p)[NR], float (&acc)[NR], b
 // and both roundings after it are odd functions, so rto_fma16's construction applied to
 // y = na - a b gives the negated result; only an exact zero changes: -(RTO24's zero of the sum)
 // is roundTowardPositive's zero of y, so the pick is by rd's last bit and falls to ru.
-__device__ __forceinline__ void rto_fnma16(const float* a, float b, float* na) {
+__device__ __forceinline__ void rto_fnma16(const float* a, const float* b, float* na) {
     float rd[16], mask[4];
     asm volatile(
         "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 2\n\t"
         "s_nop 1\n\t"
         "v_fma_f32 %16, -%36, %52, %0\n\t"
-        "v_fma_f32 %17, -%37, %52, %1\n\t"
-        "v_fma_f32 %18, -%38, %52, %2\n\t"
-        "v_fma_f32 %19, -%39, %52, %3\n\t"
-        "v_fma_f32 %20, -%40, %52, %4\n\t"
-        "v_fma_f32 %21, -%41, %52, %5\n\t"
-        "v_fma_f32 %22, -%42, %52, %6\n\t"
-        "v_fma_f32 %23, -%43, %52, %7\n\t"
-        "v_fma_f32 %24, -%44, %52, %8\n\t"
-        "v_fma_f32 %25, -%45, %52, %9\n\t"
-        "v_fma_f32 %26, -%46, %52, %10\n\t"
-        "v_fma_f32 %27, -%47, %52, %11\n\t"
-        "v_fma_f32 %28, -%48, %52, %12\n\t"
-        "v_fma_f32 %29, -%49, %52, %13\n\t"
-        "v_fma_f32 %30, -%50, %52, %14\n\t"
-        "v_fma_f32 %31, -%51, %52, %15\n\t"
+        "v_fma_f32 %17, -%37, %53, %1\n\t"
+        "v_fma_f32 %18, -%38, %54, %2\n\t"
+        "v_fma_f32 %19, -%39, %55, %3\n\t"
+        "v_fma_f32 %20, -%40, %56, %4\n\t"
+        "v_fma_f32 %21, -%41, %57, %5\n\t"
+        "v_fma_f32 %22, -%42, %58, %6\n\t"
+        "v_fma_f32 %23, -%43, %59, %7\n\t"
+        "v_fma_f32 %24, -%44, %60, %8\n\t"
+        "v_fma_f32 %25, -%45, %61, %9\n\t"
+        "v_fma_f32 %26, -%46, %62, %10\n\t"
+        "v_fma_f32 %27, -%47, %63, %11\n\t"
+        "v_fma_f32 %28, -%48, %64, %12\n\t"
+        "v_fma_f32 %29, -%49, %65, %13\n\t"
+        "v_fma_f32 %30, -%50, %66, %14\n\t"
+        "v_fma_f32 %31, -%51, %67, %15\n\t"
         "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 1\n\t"
         "s_nop 1\n\t"
         "v_fma_f32 %0, -%36, %52, %0\n\t"
-        "v_fma_f32 %1, -%37, %52, %1\n\t"
-        "v_fma_f32 %2, -%38, %52, %2\n\t"
-        "v_fma_f32 %3, -%39, %52, %3\n\t"
-        "v_fma_f32 %4, -%40, %52, %4\n\t"
-        "v_fma_f32 %5, -%41, %52, %5\n\t"
-        "v_fma_f32 %6, -%42, %52, %6\n\t"
-        "v_fma_f32 %7, -%43, %52, %7\n\t"
-        "v_fma_f32 %8, -%44, %52, %8\n\t"
-        "v_fma_f32 %9, -%45, %52, %9\n\t"
-        "v_fma_f32 %10, -%46, %52, %10\n\t"
-        "v_fma_f32 %11, -%47, %52, %11\n\t"
-        "v_fma_f32 %12, -%48, %52, %12\n\t"
-        "v_fma_f32 %13, -%49, %52, %13\n\t"
-        "v_fma_f32 %14, -%50, %52, %14\n\t"
-        "v_fma_f32 %15, -%51, %52, %15\n\t"
+        "v_fma_f32 %1, -%37, %53, %1\n\t"
+        "v_fma_f32 %2, -%38, %54, %2\n\t"
+        "v_fma_f32 %3, -%39, %55, %3\n\t"
+        "v_fma_f32 %4, -%40, %56, %4\n\t"
+        "v_fma_f32 %5, -%41, %57, %5\n\t"
+        "v_fma_f32 %6, -%42, %58, %6\n\t"
+        "v_fma_f32 %7, -%43, %59, %7\n\t"
+        "v_fma_f32 %8, -%44, %60, %8\n\t"
+        "v_fma_f32 %9, -%45, %61, %9\n\t"
+        "v_fma_f32 %10, -%46, %62, %10\n\t"
+        "v_fma_f32 %11, -%47, %63, %11\n\t"
+        "v_fma_f32 %12, -%48, %64, %12\n\t"
+        "v_fma_f32 %13, -%49, %65, %13\n\t"
+        "v_fma_f32 %14, -%50, %66, %14\n\t"
+        "v_fma_f32 %15, -%51, %67, %15\n\t"
         "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0\n\t"
         "v_bfe_i32 %32, %16, 0, 1\n\t"
         "v_bfe_i32 %33, %17, 0, 1\n\t"
@@ -317,24 +331,28 @@ __device__ __forceinline__ void rto_fnma16(const float* a, float b, float* na) {
         : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]),
           "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]),
           "v"(a[8]), "v"(a[9]), "v"(a[10]), "v"(a[11]),
-          "v"(a[12]), "v"(a[13]), "v"(a[14]), "v"(a[15]), "v"(b));
+          "v"(a[12]), "v"(a[13]), "v"(a[14]), "v"(a[15]),
+          "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]),
+          "v"(b[4]), "v"(b[5]), "v"(b[6]), "v"(b[7]),
+          "v"(b[8]), "v"(b[9]), "v"(b[10]), "v"(b[11]),
+          "v"(b[12]), "v"(b[13]), "v"(b[14]), "v"(b[15]));
 }
 
-__device__ __forceinline__ void rto_fnma4(const float* a, float b, float* na) {
+__device__ __forceinline__ void rto_fnma4(const float* a, const float* b, float* na) {
     float rd[4], mask[4];
     asm volatile(
         "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 2\n\t"
         "s_nop 1\n\t"
         "v_fma_f32 %4, -%12, %16, %0\n\t"
-        "v_fma_f32 %5, -%13, %16, %1\n\t"
-        "v_fma_f32 %6, -%14, %16, %2\n\t"
-        "v_fma_f32 %7, -%15, %16, %3\n\t"
+        "v_fma_f32 %5, -%13, %17, %1\n\t"
+        "v_fma_f32 %6, -%14, %18, %2\n\t"
+        "v_fma_f32 %7, -%15, %19, %3\n\t"
         "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 1\n\t"
         "s_nop 1\n\t"
         "v_fma_f32 %0, -%12, %16, %0\n\t"
-        "v_fma_f32 %1, -%13, %16, %1\n\t"
-        "v_fma_f32 %2, -%14, %16, %2\n\t"
-        "v_fma_f32 %3, -%15, %16, %3\n\t"
+        "v_fma_f32 %1, -%13, %17, %1\n\t"
+        "v_fma_f32 %2, -%14, %18, %2\n\t"
+        "v_fma_f32 %3, -%15, %19, %3\n\t"
         "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0\n\t"
         "v_bfe_i32 %8, %4, 0, 1\n\t"
         "v_bfe_i32 %9, %5, 0, 1\n\t"
@@ -348,7 +366,8 @@ __device__ __forceinline__ void rto_fnma4(const float* a, float b, float* na) {
         : "+v"(na[0]), "+v"(na[1]), "+v"(na[2]), "+v"(na[3]),
           "=&v"(rd[0]), "=&v"(rd[1]), "=&v"(rd[2]), "=&v"(rd[3]),
           "=&v"(mask[0]), "=&v"(mask[1]), "=&v"(mask[2]), "=&v"(mask[3])
-        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b));
+        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]),
+          "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]));
 }
 
 // Launches of at most a block a CU, one wave a SIMD.
@@ -359,17 +378,17 @@ constexpr unsigned kOneWaveBlocks = 256;
 // mode switch, whose waits a single wave's four leaves cannot cover (8x4096x4096 on FP32 operands,
 // 23 bits, one wave a SIMD: 367 us with rto_fnma4, 338 us so; 1000x768x3072, three blocks a
 // CU, 375 and 403 us).
-__device__ __forceinline__ void rto_fnma4_down(const float* a, float b, float* na) {
+__device__ __forceinline__ void rto_fnma4_down(const float* a, const float* b, float* na) {
     float d[4], m[4];
     asm(
         "v_fma_f32 %4, -%12, %16, %0\n\t"
-        "v_fma_f32 %5, -%13, %16, %1\n\t"
-        "v_fma_f32 %6, -%14, %16, %2\n\t"
-        "v_fma_f32 %7, -%15, %16, %3\n\t"
+        "v_fma_f32 %5, -%13, %17, %1\n\t"
+        "v_fma_f32 %6, -%14, %18, %2\n\t"
+        "v_fma_f32 %7, -%15, %19, %3\n\t"
         "v_fma_f32 %0, %12, %16, -%0\n\t"
-        "v_fma_f32 %1, %13, %16, -%1\n\t"
-        "v_fma_f32 %2, %14, %16, -%2\n\t"
-        "v_fma_f32 %3, %15, %16, -%3\n\t"
+        "v_fma_f32 %1, %13, %17, -%1\n\t"
+        "v_fma_f32 %2, %14, %18, -%2\n\t"
+        "v_fma_f32 %3, %15, %19, -%3\n\t"
         "v_bfe_i32 %8, %4, 0, 1\n\t"
         "v_bfe_i32 %9, %5, 0, 1\n\t"
         "v_bfe_i32 %10, %6, 0, 1\n\t"
@@ -385,7 +404,8 @@ __device__ __forceinline__ void rto_fnma4_down(const float* a, float b, float* n
         : "+v"(na[0]), "+v"(na[1]), "+v"(na[2]), "+v"(na[3]),
           "=&v"(d[0]), "=&v"(d[1]), "=&v"(d[2]), "=&v"(d[3]),
           "=&v"(m[0]), "=&v"(m[1]), "=&v"(m[2]), "=&v"(m[3])
-        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b));
+        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]),
+          "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]));
 }
 // Enter and leave round-down.  The accumulators pass through both statements, so nothing computed
 // from them moves into the region.
@@ -401,90 +421,113 @@ __device__ __forceinline__ void round_nearest(float (&x)[4]) {
 // h <- binary16(h - a b), one rounding of the exact difference (see mix_fnma16), for the
 // binary16 pairs h[i] = (h[2 i], h[2 i + 1]); the low halves first, so that no instruction follows
 // the one that wrote half of its register.
-__device__ __forceinline__ void mix_fnma_pairs16(const float* a, float b, uint32_t* h) {
+__device__ __forceinline__ void mix_fnma_pairs16(const float* a, const float* b, uint32_t* h) {
     asm volatile(
         "v_fma_mixlo_f16 %0, -%8, %24, %0 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixlo_f16 %1, -%10, %24, %1 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixlo_f16 %2, -%12, %24, %2 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixlo_f16 %3, -%14, %24, %3 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixlo_f16 %4, -%16, %24, %4 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixlo_f16 %5, -%18, %24, %5 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixlo_f16 %6, -%20, %24, %6 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixlo_f16 %7, -%22, %24, %7 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %0, -%9, %24, %0 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %1, -%11, %24, %1 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %2, -%13, %24, %2 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %3, -%15, %24, %3 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %4, -%17, %24, %4 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %5, -%19, %24, %5 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %6, -%21, %24, %6 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %7, -%23, %24, %7 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %1, -%10, %26, %1 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %2, -%12, %28, %2 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %3, -%14, %30, %3 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %4, -%16, %32, %4 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %5, -%18, %34, %5 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %6, -%20, %36, %6 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %7, -%22, %38, %7 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %0, -%9, %25, %0 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %1, -%11, %27, %1 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %2, -%13, %29, %2 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %3, -%15, %31, %3 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %4, -%17, %33, %4 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %5, -%19, %35, %5 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %6, -%21, %37, %6 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %7, -%23, %39, %7 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
         "s_nop 1"
         : "+v"(h[0]), "+v"(h[1]), "+v"(h[2]), "+v"(h[3]),
           "+v"(h[4]), "+v"(h[5]), "+v"(h[6]), "+v"(h[7])
         : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]),
           "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]),
           "v"(a[8]), "v"(a[9]), "v"(a[10]), "v"(a[11]),
-          "v"(a[12]), "v"(a[13]), "v"(a[14]), "v"(a[15]), "v"(b));
+          "v"(a[12]), "v"(a[13]), "v"(a[14]), "v"(a[15]),
+          "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]),
+          "v"(b[4]), "v"(b[5]), "v"(b[6]), "v"(b[7]),
+          "v"(b[8]), "v"(b[9]), "v"(b[10]), "v"(b[11]),
+          "v"(b[12]), "v"(b[13]), "v"(b[14]), "v"(b[15]));
 }
 
-__device__ __forceinline__ void mix_fnma_pairs4(const float* a, float b, uint32_t* h) {
+__device__ __forceinline__ void mix_fnma_pairs4(const float* a, const float* b, uint32_t* h) {
     asm volatile(
         "v_fma_mixlo_f16 %0, -%2, %6, %0 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixlo_f16 %1, -%4, %6, %1 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %0, -%3, %6, %0 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %1, -%5, %6, %1 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %1, -%4, %8, %1 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %0, -%3, %7, %0 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %1, -%5, %9, %1 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
         "s_nop 1"
         : "+v"(h[0]), "+v"(h[1])
-        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b));
+        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]),
+          "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]));
 }
 
-// The same, with the least magnitude of every result so far in `least`'s low half.
-__device__ __forceinline__ void mix_fnma_pairs16(const float* a, float b, uint32_t* h, uint32_t& least) {
+// The same on one value a register (its low half), with the least magnitude of every result so far
+// in `least`: mixed FMAs take 8 cycles a wave on gfx950, v_min_f16 2.5, v_min3_f16 over a pair 8.
+__device__ __forceinline__ void mix_fnma16_least(const float* a, const float* b, uint32_t* u, uint32_t& least) {
     asm volatile(
-        "v_fma_mixlo_f16 %0, -%9, %25, %0 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixlo_f16 %1, -%11, %25, %1 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixlo_f16 %2, -%13, %25, %2 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixlo_f16 %3, -%15, %25, %3 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixlo_f16 %4, -%17, %25, %4 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixlo_f16 %5, -%19, %25, %5 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixlo_f16 %6, -%21, %25, %6 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixlo_f16 %7, -%23, %25, %7 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %0, -%10, %25, %0 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %1, -%12, %25, %1 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %2, -%14, %25, %2 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %3, -%16, %25, %3 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %4, -%18, %25, %4 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %5, -%20, %25, %5 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %6, -%22, %25, %6 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %7, -%24, %25, %7 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
-        "v_min3_f16 %8, %8, |%0|, |%0| op_sel:[0,0,1,0]\n\t"
-        "v_min3_f16 %8, %8, |%1|, |%1| op_sel:[0,0,1,0]\n\t"
-        "v_min3_f16 %8, %8, |%2|, |%2| op_sel:[0,0,1,0]\n\t"
-        "v_min3_f16 %8, %8, |%3|, |%3| op_sel:[0,0,1,0]\n\t"
-        "v_min3_f16 %8, %8, |%4|, |%4| op_sel:[0,0,1,0]\n\t"
-        "v_min3_f16 %8, %8, |%5|, |%5| op_sel:[0,0,1,0]\n\t"
-        "v_min3_f16 %8, %8, |%6|, |%6| op_sel:[0,0,1,0]\n\t"
-        "v_min3_f16 %8, %8, |%7|, |%7| op_sel:[0,0,1,0]"
-        : "+v"(h[0]), "+v"(h[1]), "+v"(h[2]), "+v"(h[3]),
-          "+v"(h[4]), "+v"(h[5]), "+v"(h[6]), "+v"(h[7]), "+v"(least)
+        "v_fma_mixlo_f16 %0, -%17, %33, %0 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %1, -%18, %34, %1 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %2, -%19, %35, %2 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %3, -%20, %36, %3 op_sel_hi:[0,0,1]\n\t"
+        "v_min_f16 %16, %16, |%0|\n\t"
+        "v_fma_mixlo_f16 %4, -%21, %37, %4 op_sel_hi:[0,0,1]\n\t"
+        "v_min_f16 %16, %16, |%1|\n\t"
+        "v_fma_mixlo_f16 %5, -%22, %38, %5 op_sel_hi:[0,0,1]\n\t"
+        "v_min_f16 %16, %16, |%2|\n\t"
+        "v_fma_mixlo_f16 %6, -%23, %39, %6 op_sel_hi:[0,0,1]\n\t"
+        "v_min_f16 %16, %16, |%3|\n\t"
+        "v_fma_mixlo_f16 %7, -%24, %40, %7 op_sel_hi:[0,0,1]\n\t"
+        "v_min_f16 %16, %16, |%4|\n\t"
+        "v_fma_mixlo_f16 %8, -%25, %41, %8 op_sel_hi:[0,0,1]\n\t"
+        "v_min_f16 %16, %16, |%5|\n\t"
+        "v_fma_mixlo_f16 %9, -%26, %42, %9 op_sel_hi:[0,0,1]\n\t"
+        "v_min_f16 %16, %16, |%6|\n\t"
+        "v_fma_mixlo_f16 %10, -%27, %43, %10 op_sel_hi:[0,0,1]\n\t"
+        "v_min_f16 %16, %16, |%7|\n\t"
+        "v_fma_mixlo_f16 %11, -%28, %44, %11 op_sel_hi:[0,0,1]\n\t"
+        "v_min_f16 %16, %16, |%8|\n\t"
+        "v_fma_mixlo_f16 %12, -%29, %45, %12 op_sel_hi:[0,0,1]\n\t"
+        "v_min_f16 %16, %16, |%9|\n\t"
+        "v_fma_mixlo_f16 %13, -%30, %46, %13 op_sel_hi:[0,0,1]\n\t"
+        "v_min_f16 %16, %16, |%10|\n\t"
+        "v_fma_mixlo_f16 %14, -%31, %47, %14 op_sel_hi:[0,0,1]\n\t"
+        "v_min_f16 %16, %16, |%11|\n\t"
+        "v_fma_mixlo_f16 %15, -%32, %48, %15 op_sel_hi:[0,0,1]\n\t"
+        "v_min_f16 %16, %16, |%12|\n\t"
+        "v_min_f16 %16, %16, |%13|\n\t"
+        "v_min_f16 %16, %16, |%14|\n\t"
+        "v_min_f16 %16, %16, |%15|"
+        : "+v"(u[0]), "+v"(u[1]), "+v"(u[2]), "+v"(u[3]),
+          "+v"(u[4]), "+v"(u[5]), "+v"(u[6]), "+v"(u[7]),
+          "+v"(u[8]), "+v"(u[9]), "+v"(u[10]), "+v"(u[11]),
+          "+v"(u[12]), "+v"(u[13]), "+v"(u[14]), "+v"(u[15]), "+v"(least)
         : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]),
           "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]),
           "v"(a[8]), "v"(a[9]), "v"(a[10]), "v"(a[11]),
-          "v"(a[12]), "v"(a[13]), "v"(a[14]), "v"(a[15]), "v"(b));
+          "v"(a[12]), "v"(a[13]), "v"(a[14]), "v"(a[15]),
+          "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]),
+          "v"(b[4]), "v"(b[5]), "v"(b[6]), "v"(b[7]),
+          "v"(b[8]), "v"(b[9]), "v"(b[10]), "v"(b[11]),
+          "v"(b[12]), "v"(b[13]), "v"(b[14]), "v"(b[15]));
 }
 
-__device__ __forceinline__ void mix_fnma_pairs4(const float* a, float b, uint32_t* h, uint32_t& least) {
+__device__ __forceinline__ void mix_fnma4_least(const float* a, const float* b, uint32_t* u, uint32_t& least) {
     asm volatile(
-        "v_fma_mixlo_f16 %0, -%3, %7, %0 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixlo_f16 %1, -%5, %7, %1 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %0, -%4, %7, %0 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %1, -%6, %7, %1 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %0, -%5, %9, %0 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %1, -%6, %10, %1 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %2, -%7, %11, %2 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %3, -%8, %12, %3 op_sel_hi:[0,0,1]\n\t"
         "s_nop 0\n\t"
-        "v_min3_f16 %2, %2, |%0|, |%0| op_sel:[0,0,1,0]\n\t"
-        "v_min3_f16 %2, %2, |%1|, |%1| op_sel:[0,0,1,0]"
-        : "+v"(h[0]), "+v"(h[1]), "+v"(least)
-        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b));
+        "v_min_f16 %4, %4, |%0|\n\t"
+        "v_min_f16 %4, %4, |%1|\n\t"
+        "v_min_f16 %4, %4, |%2|\n\t"
+        "v_min_f16 %4, %4, |%3|"
+        : "+v"(u[0]), "+v"(u[1]), "+v"(u[2]), "+v"(u[3]), "+v"(least)
+        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]),
+          "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]));
 }
 
 // B of an implicit-GEMM convolution: a thread's four columns n = n0 + 4 * (tid % (BN / 4)) + j are
@@ -549,6 +592,48 @@ struct SliceKey {
     __device__ __forceinline__ void add(const float4& v) { add(v.x); add(v.y); add(v.z); add(v.w); }
 };
 
+// The same of values stored as binary16 pairs, two at a time on the packed 16-bit units: the
+// largest magnitude, and the least value of a lowest set bit, less one (x - (x with that bit
+// cleared), exact in binary16; half of it for a power of two, whose pattern's lowest bit is the
+// exponent's).  bad: a value that binary16 does not hold.
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+template <bool STAT>
+struct PairKey {
+    bool bad = false;
+    u16x2 mx = {0, 0}, ls = {0xFFFF, 0xFFFF};
+    __device__ __forceinline__ uint32_t add(float x, float y) {
+        // truncation keeps a binary16 value
+        const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x, y));
+        const f16x2 v = __builtin_bit_cast(f16x2, h);
+        bad |= ((float)v.x != x) | ((float)v.y != y);
+        if constexpr (STAT) {
+            const u16x2 p = __builtin_bit_cast(u16x2, h & 0x7FFF7FFFu), one = {1, 1};
+            const f16x2 d = __builtin_bit_cast(f16x2, p) - __builtin_bit_cast(f16x2, p & (p - one));
+            mx = __builtin_elementwise_max(mx, p);
+            ls = __builtin_elementwise_min(ls, __builtin_bit_cast(u16x2, d) - one);
+        }
+        return h;
+    }
+    // of both operands over the wave, valid in lane 63: {amax A, key A, amax B, key B} as SliceKey's
+    static __device__ __forceinline__ uint4 wave(const PairKey& a, const PairKey& b) {
+        auto least2 = [](u16x2 v) {
+            return __builtin_bit_cast(u16x2, wave_last_u32(__builtin_bit_cast(uint32_t, v), ~0u, [](uint32_t x, uint32_t y) {
+                return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, x),
+                                                                              __builtin_bit_cast(u16x2, y)));
+            }));
+        };
+        const u16x2 m = least2(~u16x2{max(a.mx.x, a.mx.y), max(b.mx.x, b.mx.y)});
+        const u16x2 l = least2(u16x2{min(a.ls.x, a.ls.y), min(b.ls.x, b.ls.y)});
+        auto bits = [](unsigned short x) {
+            return __float_as_uint((float)__builtin_bit_cast(_Float16, x));
+        };
+        auto key = [&](unsigned short x) {
+            return x == 0xFFFF ? 0xFFFFFFFFu : (bits((unsigned short)(x + 1)) >> 23) + 23u;
+        };
+        return make_uint4(bits((unsigned short)~m.x) << 1, key(l.x), bits((unsigned short)~m.y) << 1, key(l.y));
+    }
+};
+
 template <class T, int CHUNK, int KIND, bool CONV>
 __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, int tile_n, int tid,
                                                 float* smem) {
@@ -565,6 +650,16 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
     // operand statistics: exact sums (23 bits), binary16's grid (10 bits)
     constexpr bool kStat = kStep && (KIND == kChainMant23 || KIND == kChainMant10);
     constexpr bool kWide = kStep && KIND == kChainMant10;   // a second flag: not binary16 operands
+    // Chunk 1 without the matrix cores: a lane's outputs are SQ x SQ neighbours, SQ values of
+    // each operand a k (an MFMA block's are 16 rows of one column, 17 values).  Kinds that
+    // hold binary16 pairs also keep their slices as binary16 pairs while every value is one: half the
+    // LDS bytes, no conversions, operands read as the packed FMA takes them.
+    constexpr bool kOuter = kStep && KIND != kChainMant23;
+    constexpr bool kPack = kStep && (KIND == kChainHalf || KIND == kChainMant10);
+    constexpr int SQ = NR == 16 ? 4 : 2, SP = SQ / 2;
+    constexpr int PGA = BM / 2 + 1, PGB = BN / 2 + 1;   // packed: uint4s per four k, one for the banks
+    static_assert(!kStep || WMB * WNB == 1, "chunk 1: one block a wave");
+    static_assert(4 * PGA * (BK / 4) <= LA::FLOATS && 4 * PGB * (BK / 4) <= LB::FLOATS, "packed slices fit");
     static_assert(kStep || (CHUNK >= KI && BK % CHUNK == 0),
                   "whole MFMAs per chunk, whole chunks per slice");
     constexpr float kPadA = kStep ? 0.0f : -0.0f;   // k past K, see the head comment
@@ -582,7 +677,10 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
     // .. + 3 of a transposed one; likewise B.  Offsets are from the tile's corner.  They are
     // recomputed for every slice from a copy of tid that the compiler cannot see through:
     // held across the loop, they and the edges' element offsets spill.
+    // kPack: row-major rows come in neighbouring pairs (it, it + 1), a packed store each.
     auto otid = [&]() { int t = tid; asm volatile("" : "+v"(t)); return t; };
+    auto rows_of = [](int t) { return kPack ? t / (BK / 4) * 2 : t / (BK / 4); };
+    auto rows_step = [](int it) { return kPack ? (it & 1) + (it >> 1) * (2048 / BK) : it * (1024 / BK); };
     ConvCols<BN> cols;
     if constexpr (CONV) cols.init(g, n0, tid);
     const float* A0 = g.A + (g.ta ? (int64_t)m0 : (int64_t)m0 * g.lda);
@@ -597,10 +695,10 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
         constexpr int R = decltype(rows)::value, NV = R * BK / 1024;
         if (kl >= BK && left >= R) {
             const uint32_t o = kmaj ? (uint32_t)(tid / (R / 4)) * (uint32_t)ld + (uint32_t)(4 * (tid % (R / 4)))
-                                    : (uint32_t)(tid / (BK / 4)) * (uint32_t)ld + (uint32_t)(4 * (tid % (BK / 4)));
-            const int64_t step = (kmaj ? 1024 / R : 1024 / BK) * ld;
+                                    : (uint32_t)rows_of(tid) * (uint32_t)ld + (uint32_t)(4 * (tid % (BK / 4)));
 #pragma unroll
-            for (int it = 0; it < NV; ++it) v[it] = gld4u(p + it * step + o);
+            for (int it = 0; it < NV; ++it)
+                v[it] = gld4u(p + (kmaj ? it * (1024 / R) : rows_step(it)) * ld + o);
             return;
         }
         const int t = otid();   // an edge: elements from clamped addresses, `pad` past K
@@ -622,7 +720,7 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
                 }
             } else {
                 const int k = 4 * (t % (BK / 4));
-                const int r = min(t / (BK / 4) + it * (1024 / BK), left - 1);
+                const int r = min(rows_of(t) + rows_step(it), left - 1);
                 const uint32_t o = (uint32_t)r * (uint32_t)ld;
                 if (kl >= BK) {
                     v[it] = gld4u(p + (o + (uint32_t)k));
@@ -653,62 +751,89 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
                     0.0f);
         }
     };
-    // registers -> LDS buffer; fl: the slice's non-finite flag
-    auto store_slice = [&](int buf, int fl) {
+    // registers -> LDS buffer, as FP32 or as binary16 pairs
+    using Pairs = PairKey<kStat>;
+    auto put_slice = [&](int buf, bool packed, Pairs& ka, Pairs& kb) {
         float* As = smem + buf * T::BUF_FLOATS;
-        float z = 0.0f;   // 0 * v summed: NaN as soon as one v is not finite
-        bool wide = false;
-        SliceKey ka, kb;
-        auto put = [&](float* S, auto lds, auto rows, const auto& v, bool kmaj) {
+        auto put = [&](float* S, auto lds, auto rows, const auto& v, bool kmaj, Pairs& key) {
             using L = decltype(lds);
-            constexpr int R = decltype(rows)::value, NV = R * BK / 1024;
+            constexpr int R = decltype(rows)::value, NV = R * BK / 1024, PG = R / 2 + 1;
+            if (kPack && packed) {   // [k / 4][row pair][k % 4]
+                auto pk = [&](float x, float y) { return key.add(x, y); };
+                if (kmaj) {
+                    const int k = tid / (R / 4);
+                    uint32_t* d = (uint32_t*)S + (k >> 2) * 4 * PG + 8 * (tid % (R / 4)) + (k & 3);
+#pragma unroll
+                    for (int it = 0; it < NV; ++it) {
+                        d[it * (256 / R) * 4 * PG] = pk(v[it].x, v[it].y);
+                        d[it * (256 / R) * 4 * PG + 4] = pk(v[it].z, v[it].w);
+                    }
+                } else {
+                    uint4* d = (uint4*)S + (tid % (BK / 4)) * PG + tid / (BK / 4);
+#pragma unroll
+                    for (int it = 0; it + 1 < NV; it += 2)
+                        d[it * (512 / BK)] = make_uint4(pk(v[it].x, v[it + 1].x), pk(v[it].y, v[it + 1].y),
+                                                        pk(v[it].z, v[it + 1].z), pk(v[it].w, v[it + 1].w));
+                }
+                return;
+            }
             if (kmaj) {   // float4 `it` lies 1024 / R (a multiple of 4) k further
                 const int k = tid / (R / 4);
                 float* d = S + L::row(k) + ((4 * (tid % (R / 4))) ^ L::swz(k));
 #pragma unroll
                 for (int it = 0; it < NV; ++it) *(float4*)(d + it * (256 / R) * L::GROUP) = v[it];
             } else {      // 4 k of a row, 1024 / BK (at most 32) rows further each time
-                float* d = S + (tid % (BK / 4)) * L::GROUP + tid / (BK / 4);
+                // MFMA kinds' rows lie at least 32 apart, past the swizzle
+                float* d = S + (tid % (BK / 4)) * L::GROUP + (kPack ? 0 : tid / (BK / 4));
 #pragma unroll
                 for (int it = 0; it < NV; ++it) {
-                    const int r = it * (1024 / BK);
+                    const int r = (kPack ? rows_of(tid) : 0) + rows_step(it);
                     d[0 * R + (r ^ L::swz(0))] = v[it].x;
                     d[1 * R + (r ^ L::swz(1))] = v[it].y;
                     d[2 * R + (r ^ L::swz(2))] = v[it].z;
                     d[3 * R + (r ^ L::swz(3))] = v[it].w;
                 }
             }
-            if constexpr (kF16Flag) {
-                auto w = [](float x) { return (float)(_Float16)x != x; };
-#pragma unroll
-                for (int it = 0; it < NV; ++it)
-                    wide |= w(v[it].x) | w(v[it].y) | w(v[it].z) | w(v[it].w);
-            } else if constexpr (kFlag) {
-#pragma unroll
-                for (int it = 0; it < NV; ++it) {
-                    z = __builtin_fmaf(v[it].x, 0.0f, z);
-                    z = __builtin_fmaf(v[it].y, 0.0f, z);
-                    z = __builtin_fmaf(v[it].z, 0.0f, z);
-                    z = __builtin_fmaf(v[it].w, 0.0f, z);
-                }
-            }
         };
-        put(As, LA{}, std::integral_constant<int, BM>{}, va, g.ta != 0);
-        put(As + LA::FLOATS, LB{}, std::integral_constant<int, BN>{}, vb, CONV || g.tb == 0);
-        if constexpr (kFlag)
-            if (wide || z != 0.0f) flags[fl] = 1u;   // z is +-0 or NaN
-        if constexpr (kWide) {   // A binary16 values, B of at most 11 significant bits
-            uint32_t low = 0u;
-#pragma unroll
-            for (int it = 0; it < NA4; ++it) {
-                auto w = [](float x) { return (float)(_Float16)x != x; };
-                wide |= w(va[it].x) | w(va[it].y) | w(va[it].z) | w(va[it].w);
+        put(As, LA{}, std::integral_constant<int, BM>{}, va, g.ta != 0, ka);
+        put(As + LA::FLOATS, LB{}, std::integral_constant<int, BN>{}, vb, CONV || g.tb == 0, kb);
+    };
+    // fl: the slice's flags
+    auto store_slice = [&](int buf, int fl, bool packed) {
+        Pairs pa, pb;
+        put_slice(buf, packed, pa, pb);
+        if (kPack && packed) {
+            bool bad = pa.bad | pb.bad;
+            if constexpr (kStat) {
+                const u16x2 m = __builtin_elementwise_max(pa.mx, pb.mx);
+                bad |= max(m.x, m.y) >= 0x7C00;   // an infinity
+                const uint4 w = Pairs::wave(pa, pb);
+                if (lane == 63) *(uint4*)(stats + buf * 16 + wave * 4) = w;
             }
+            if (bad) flags[fl + (kStat ? 40 : 0)] = 1u;
+            return;
+        }
+        SliceKey ka, kb;
+        auto over = [](const auto& v, auto f) {
+            bool any = false;
 #pragma unroll
-            for (int it = 0; it < NB4; ++it)
-                low |= __float_as_uint(vb[it].x) | __float_as_uint(vb[it].y) |
-                       __float_as_uint(vb[it].z) | __float_as_uint(vb[it].w);
-            if (wide || (low & 0x1FFFu) != 0u) flags[fl + 36] = 1u;
+            for (int it = 0; it < (int)(sizeof(v) / sizeof(float4)); ++it)
+                any |= f(v[it].x) | f(v[it].y) | f(v[it].z) | f(v[it].w);
+            return any;
+        };
+        auto not16 = [](float x) { return (float)(_Float16)x != x; };
+        if constexpr (kF16Flag) {
+            if (over(va, not16) | over(vb, not16)) flags[fl] = 1u;
+        } else if constexpr (kFlag) {
+            float z = 0.0f;   // 0 * v summed: NaN as soon as one v is not finite
+            auto sum = [&](float x) { z = __builtin_fmaf(x, 0.0f, z); return false; };
+            over(va, sum);
+            over(vb, sum);
+            if (z != 0.0f) flags[fl] = 1u;   // z is +-0 or NaN
+        }
+        if constexpr (kWide) {   // A binary16 values, B of at most 11 significant bits
+            if (over(va, not16) | over(vb, [](float x) { return (__float_as_uint(x) & 0x1FFFu) != 0u; }))
+                flags[fl + 36] = 1u;
         }
         if constexpr (kStat) {
 #pragma unroll
@@ -780,34 +905,47 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
         rb[bj] = lhi * BN + ((bn0 + bj * BS + lcol) ^ LB::swz(lhi));
 
     // ---- chunk 1: every k's leaf, on the negated accumulators
-    // Row quads of a lane's outputs (rows 8 rq + 4 lhi .. + 3 of a block) and its column, at the
-    // swizzle of k's place in its group of four.
-    auto a_quad = [&](const float* As, int k, int bi, int rq) -> float4 {
-        return *(const float4*)&As[LA::row(k) + ((am0 + bi * BS + rq * 8 + lhi * 4) ^ LA::swz(k))];
-    };
-    auto b_col = [&](const float* Bs, int k, int bj) -> float {
-        return Bs[LB::row(k) + ((bn0 + bj * BS + lcol) ^ LB::swz(k))];
-    };
-    // leaf(bi, bj, a, b) for every k < kmax, in groups of four k (those past K add -0): a group's
-    // next k is read while the current one computes
-    auto for_k = [&](const float* As, const float* Bs, int kmax, auto leaf) {
-        float a[2][WMB][NR], b[2][WNB];
-        auto fetch = [&](int set, const float* Ap, const float* Bp, int k) {
-#pragma unroll
-            for (int bi = 0; bi < WMB; ++bi)
-#pragma unroll
-                for (int rq = 0; rq < NR / 4; ++rq) {
-                    const float4 v = a_quad(Ap, k, bi, rq);
-                    a[set][bi][4 * rq + 0] = v.x;
-                    a[set][bi][4 * rq + 1] = v.y;
-                    a[set][bi][4 * rq + 2] = v.z;
-                    a[set][bi][4 * rq + 3] = v.w;
-                }
-#pragma unroll
-            for (int bj = 0; bj < WNB; ++bj) b[set][bj] = b_col(Bp, k, bj);
+    // This lane's outputs: r is row out_row(r), column out_col(r) of the wave's block.
+    const int orow = kOuter ? SQ * (lane >> 3) : lhi * 4, ocol = kOuter ? SQ * (lane & 7) : lcol;
+    auto out_row = [&](int r) { return orow + (kOuter ? r % SQ : (r >> 2) * 8 + (r & 3)); };
+    auto out_col = [&](int r) { return ocol + (kOuter ? r / SQ : 0); };
+    // operand values of output r, as the leaves take them
+    auto ax = [](int r) { return kOuter ? r % SQ : r; };
+    auto bx = [](int r) { return kOuter ? r / SQ : 0; };
+    constexpr int NA = kOuter ? SQ : NR, NB = kOuter ? SQ : 1;
+    auto fetch_k = [&](const float* Ap, const float* Bp, int k, float* a, float* b) {
+        auto quads = [](float* o, const float* p) {
+            const float4 v = *(const float4*)p;
+            o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
         };
+        auto pair = [](float* o, const float* p) {
+            const float2 v = *(const float2*)p;
+            o[0] = v.x; o[1] = v.y;
+        };
+        const float* ap = Ap + LA::row(k);
+        const float* bp = Bp + LB::row(k) + ((bn0 + ocol) ^ LB::swz(k));
+        if constexpr (kOuter) {
+            ap += (am0 + orow) ^ LA::swz(k);
+            if constexpr (SQ == 4) {
+                quads(a, ap);
+                quads(b, bp);
+            } else {
+                pair(a, ap);
+                pair(b, bp);
+            }
+        } else {
+#pragma unroll
+            for (int rq = 0; rq < NR / 4; ++rq)
+                quads(a + 4 * rq, ap + ((am0 + rq * 8 + orow) ^ LA::swz(k)));
+            b[0] = *bp;
+        }
+    };
+    // leaf(a, b), a[NA] and b[NB], for every k < kmax, in groups of four k (those past K add -0):
+    // a group's next k is read while the current one computes
+    auto for_k32 = [&](const float* As, const float* Bs, int kmax, auto leaf) {
+        float a[2][NA], b[2][NB];
         constexpr bool kAhead = NR == 4;
-        if constexpr (kAhead) fetch(0, As, Bs, 0);
+        if constexpr (kAhead) fetch_k(As, Bs, 0, a[0], b[0]);
         const int ng = (kmax + 3) / 4;
         for (int q = 0; q < ng; ++q) {
             const float* Aq = As + q * LA::GROUP;
@@ -815,74 +953,138 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
             const int adv = q + 1 < ng ? 1 : 0;   // the last group reads its own first k again
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                if constexpr (!kAhead) fetch(j & 1, Aq, Bq, j);
-                else if (j < 3) fetch((j + 1) & 1, Aq, Bq, j + 1);
-                else fetch(0, Aq + adv * LA::GROUP, Bq + adv * LB::GROUP, 0);
-#pragma unroll
-                for (int bi = 0; bi < WMB; ++bi)
-#pragma unroll
-                    for (int bj = 0; bj < WNB; ++bj) leaf(bi, bj, a[j & 1][bi], b[j & 1][bj]);
+                if constexpr (!kAhead) fetch_k(Aq, Bq, j, a[j & 1], b[j & 1]);
+                else if (j < 3) fetch_k(Aq, Bq, j + 1, a[(j + 1) & 1], b[(j + 1) & 1]);
+                else fetch_k(Aq + adv * LA::GROUP, Bq + adv * LB::GROUP, 0, a[0], b[0]);
+                leaf(a[j & 1], b[j & 1]);
             }
         }
     };
+    // A packed slice's pairs of four k: group q of this lane's rows (columns), pair p, k % 4 = j is
+    // component j of [p].  leaf(a, b) for every group; ahead: the next one read while it computes,
+    // groups in twos (a slice is padded to its full length).
+    auto for_k16 = [&](auto ahead, const float* As, const float* Bs, int kmax, auto leaf) {
+        const uint4* Ap = (const uint4*)As + (am0 + orow) / 2;
+        const uint4* Bp = (const uint4*)Bs + (bn0 + ocol) / 2;
+        uint4 a[2][SP], b[2][SP];
+        auto fetch = [&](int set, int q) {
+#pragma unroll
+            for (int p = 0; p < SP; ++p) {
+                a[set][p] = Ap[q * PGA + p];
+                b[set][p] = Bp[q * PGB + p];
+            }
+        };
+        if constexpr (!ahead.value) {
+            for (int q = 0; q < (kmax + 3) / 4; ++q) {
+                fetch(0, q);
+                leaf(a[0], b[0]);
+            }
+            return;
+        }
+        const int ng = (kmax + 7) / 8 * 2;
+        fetch(0, 0);
+        for (int q = 0; q < ng; q += 2) {
+            fetch(1, q + 1);
+            leaf(a[0], b[0]);
+            fetch(0, q + 2 < ng ? q + 2 : q);
+            leaf(a[1], b[1]);
+        }
+    };
+    auto word = [](const uint4& v, int j) { return j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w; };
+    auto pair_of = [&](const uint4& v, int j) { return __builtin_bit_cast(f16x2, word(v, j)); };
+    // for_k32 over either form of slice
+    auto for_k = [&](bool packed, const float* As, const float* Bs, int kmax, auto leaf) {
+        if constexpr (kPack) {
+            if (packed) {
+                for_k16(std::false_type{}, As, Bs, kmax, [&](const uint4* a4, const uint4* b4) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        float a[SQ], b[SQ];
+#pragma unroll
+                        for (int p = 0; p < SP; ++p) {
+                            a[2 * p] = (float)pair_of(a4[p], j).x;
+                            a[2 * p + 1] = (float)pair_of(a4[p], j).y;
+                            b[2 * p] = (float)pair_of(b4[p], j).x;
+                            b[2 * p + 1] = (float)pair_of(b4[p], j).y;
+                        }
+                        leaf(a, b);
+                    }
+                });
+                return;
+            }
+        }
+        for_k32(As, Bs, kmax, leaf);
+    };
     // The general leaf over a slice, out of line per leaf: slices with an infinity or a NaN, and
     // binary16 sums that reach 65520 (or held values that are not binary16).
-    auto general_slice = [&](const float* As, const float* Bs, int kmax) {
+    auto general_slice = [&](bool packed, const float* As, const float* Bs, int kmax) {
         const LeafGen L = leaf_gen(g);
+        auto at = [&](const float* S, auto lds, int pg, int k, int row) -> float {
+            if (kPack && packed)
+                return (float)((const _Float16*)S)[((k >> 2) * pg + row / 2) * 8 + (k & 3) * 2 + row % 2];
+            using L = decltype(lds);
+            return S[L::row(k) + (row ^ L::swz(k))];
+        };
         for (int k = 0; k < kmax; ++k)
 #pragma unroll
-            for (int bi = 0; bi < WMB; ++bi)
-#pragma unroll
-                for (int bj = 0; bj < WNB; ++bj) {
-                    const float b = b_col(Bs, k, bj);
-#pragma unroll
-                    for (int rq = 0; rq < NR / 4; ++rq) {
-                        const float4 a4 = a_quad(As, k, bi, rq);
-                        const float av[4] = {a4.x, a4.y, a4.z, a4.w};
-#pragma unroll
-                        for (int x = 0; x < 4; ++x) {
-                            float& na = acc[bi][bj][4 * rq + x];
-                            na = -(float)leaf_slow<LeafGen>((double)av[x] * (double)b, -(double)na, L);
-                        }
-                    }
-                }
+            for (int r = 0; r < NR; ++r) {
+                const float a = at(As, LA{}, PGA, k, am0 + out_row(r)), b = at(Bs, LB{}, PGB, k, bn0 + out_col(r));
+                float& na = acc[0][0][r];
+                na = -(float)leaf_slow<LeafGen>((double)a * (double)b, -(double)na, L);
+            }
     };
-    uint32_t h[WMB][WNB][NR / 2];   // the accumulators as binary16 pairs while `held`
+    // While `held`, the accumulators are binary16 pairs scaled by 2^hs (exact both ways where
+    // they are used), in the first half of acc's registers.
     bool held = false;
-    int accL = 1000;   // 23 bits: every accumulator of the wave is a multiple of 2^accL
-    // to and from binary16 pairs scaled by 2^hs (exact both ways where they are used)
     int hs = 0;
+    float acc_bound = 0.0f;   // 10 bits, held: above every accumulator of the wave
+    int accL = 1000;   // 23 and 10 bits: every accumulator of the wave is a multiple of 2^accL
+    auto get_held = [&](uint32_t (&h)[NR / 2]) {
+#pragma unroll
+        for (int r = 0; r < NR / 2; ++r) h[r] = __float_as_uint(acc[0][0][r]);
+    };
+    auto put_held = [&](const uint32_t (&h)[NR / 2]) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r) acc[0][0][r] = r < NR / 2 ? __uint_as_float(h[r]) : 0.0f;
+    };
     auto hold = [&](int to) {
         hs = to;
+        uint32_t h[NR / 2];
 #pragma unroll
-        for (int bi = 0; bi < WMB; ++bi)
-#pragma unroll
-            for (int bj = 0; bj < WNB; ++bj)
-#pragma unroll
-                for (int r = 0; r < NR / 2; ++r)
-                    h[bi][bj][r] = __builtin_bit_cast(
-                        uint32_t, f16x2{(_Float16)__builtin_ldexpf(acc[bi][bj][2 * r], hs),
-                                        (_Float16)__builtin_ldexpf(acc[bi][bj][2 * r + 1], hs)});
+        for (int r = 0; r < NR / 2; ++r)
+            h[r] = __builtin_bit_cast(uint32_t, f16x2{(_Float16)__builtin_ldexpf(acc[0][0][2 * r], hs),
+                                                      (_Float16)__builtin_ldexpf(acc[0][0][2 * r + 1], hs)});
+        put_held(h);
+        held = true;
     };
     auto unhold = [&]() {
+        uint32_t h[NR / 2];
+        get_held(h);
 #pragma unroll
-        for (int bi = 0; bi < WMB; ++bi)
+        for (int r = 0; r < NR / 2; ++r) {
+            const f16x2 v = __builtin_bit_cast(f16x2, h[r]);
+            acc[0][0][2 * r] = __builtin_ldexpf((float)v.x, -hs);
+            acc[0][0][2 * r + 1] = __builtin_ldexpf((float)v.y, -hs);
+        }
+        held = false;
+    };
+    // a leaf's operands per output, for the assembly
+    auto spread = [&](const float* a, const float* b, float (&av)[NR], float (&bv)[NR]) {
 #pragma unroll
-            for (int bj = 0; bj < WNB; ++bj)
-#pragma unroll
-                for (int r = 0; r < NR / 2; ++r) {
-                    const f16x2 v = __builtin_bit_cast(f16x2, h[bi][bj][r]);
-                    acc[bi][bj][2 * r] = __builtin_ldexpf((float)v.x, -hs);
-                    acc[bi][bj][2 * r + 1] = __builtin_ldexpf((float)v.y, -hs);
-                }
+        for (int r = 0; r < NR; ++r) {
+            av[r] = a[ax(r)];
+            bv[r] = b[bx(r)];
+        }
     };
     // every leaf by directed roundings
-    auto directed = [&](const float* As, const float* Bs, int kmax) {
-        auto leaf = [&](auto down, int bi, int bj, const float* a, float b) {
-            float (&x)[NR] = acc[bi][bj];
-            if constexpr (NR == 16) rto_fnma16(a, b, x);
-            else if constexpr (down.value) rto_fnma4_down(a, b, x);
-            else rto_fnma4(a, b, x);
+    auto directed = [&](bool packed, const float* As, const float* Bs, int kmax) {
+        float (&x)[NR] = acc[0][0];
+        auto leaf = [&](auto down, const float* a, const float* b) {
+            float av[NR], bv[NR];
+            spread(a, b, av, bv);
+            if constexpr (NR == 16) rto_fnma16(av, bv, x);
+            else if constexpr (down.value) rto_fnma4_down(av, bv, x);
+            else rto_fnma4(av, bv, x);
             if constexpr (KIND != kChainMant23)
 #pragma unroll
                 for (int r = 0; r < NR; ++r) {
@@ -892,22 +1094,58 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
                 }
         };
         if constexpr (NR == 4) {
-            static_assert(WMB * WNB == 1, "one block of four outputs a lane");
             if (gridDim.x <= kOneWaveBlocks) {
-                round_down(acc[0][0]);
-                for_k(As, Bs, kmax, [&](int bi, int bj, const float* a, float b) {
-                    leaf(std::true_type{}, bi, bj, a, b);
-                });
-                round_nearest(acc[0][0]);
+                round_down(x);
+                for_k(packed, As, Bs, kmax, [&](const float* a, const float* b) { leaf(std::true_type{}, a, b); });
+                round_nearest(x);
                 return;
             }
         }
-        for_k(As, Bs, kmax, [&](int bi, int bj, const float* a, float b) {
-            leaf(std::false_type{}, bi, bj, a, b);
-        });
+        for_k(packed, As, Bs, kmax, [&](const float* a, const float* b) { leaf(std::false_type{}, a, b); });
     };
-    auto step_slice = [&](const float* As, const float* Bs, int kmax, bool special, bool wide16,
-                          int buf) {
+    // the packed binary16 leaves of a packed slice, B scaled by 2^hs where `scaled`
+    auto packed_leaves = [&](const float* As, const float* Bs, int kmax, auto scaled) {
+        const _Float16 sc = (_Float16)__builtin_ldexpf(1.0f, hs);
+        uint32_t hp[NR / 2];
+        get_held(hp);
+        for_k16(std::true_type{}, As, Bs, kmax, [&](const uint4* a4, const uint4* b4) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int c = 0; c < SQ; ++c) {
+                    f16x2 b = pair_of(b4[c / 2], j);
+                    if constexpr (scaled.value) b = b * f16x2{sc, sc};
+                    b = c & 1 ? f16x2{b.y, b.y} : f16x2{b.x, b.x};
+#pragma unroll
+                    for (int p = 0; p < SP; ++p)
+                        hp[c * SP + p] = __builtin_bit_cast(
+                            uint32_t, __builtin_elementwise_fma(-pair_of(a4[p], j), b,
+                                                                __builtin_bit_cast(f16x2, hp[c * SP + p])));
+                }
+        });
+        put_held(hp);
+    };
+    // the same from an FP32 slice of binary16 values (scaled: B of binary16's significand)
+    auto packed_leaves32 = [&](const float* As, const float* Bs, int kmax) {
+        uint32_t hp[NR / 2];
+        get_held(hp);
+        for_k32(As, Bs, kmax, [&](const float* a, const float* b) {
+#pragma unroll
+            for (int c = 0; c < SQ; ++c) {
+                const _Float16 bv = (_Float16)__builtin_ldexpf(b[c], hs);
+#pragma unroll
+                for (int p = 0; p < SP; ++p) {
+                    const f16x2 av = {(_Float16)a[2 * p], (_Float16)a[2 * p + 1]};
+                    hp[c * SP + p] = __builtin_bit_cast(
+                        uint32_t, __builtin_elementwise_fma(-av, f16x2{bv, bv},
+                                                            __builtin_bit_cast(f16x2, hp[c * SP + p])));
+                }
+            }
+        });
+        put_held(hp);
+    };
+    auto step_slice = [&](bool packed, const float* As, const float* Bs, int kmax, bool special,
+                          bool wide16, int buf) {
         if constexpr (KIND == kChainHalf) {
             // Held as binary16 pairs while every accumulator is a binary16 value below 2^15 at a
             // slice's start.  The binary16 FMA (operands binary16 too: packed, two leaves an
@@ -925,61 +1163,42 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
                             const float x = acc[bi][bj][r];
                             ok &= (float)(_Float16)x == x && fabsf(x) < 32768.0f;
                         }
-                held = __all(ok);
-                if (held) hold(0);
+                if (__all(ok)) hold(0);
             }
             if (held) {
-                uint32_t h0[WMB][WNB][NR / 2];
-#pragma unroll
-                for (int bi = 0; bi < WMB; ++bi)
-#pragma unroll
-                    for (int bj = 0; bj < WNB; ++bj)
-#pragma unroll
-                        for (int r = 0; r < NR / 2; ++r) h0[bi][bj][r] = h[bi][bj][r];
-                if (!special) {
-                    for_k(As, Bs, kmax, [&](int bi, int bj, const float* a, float b) {
-                        const _Float16 bv = (_Float16)b;
-#pragma unroll
-                        for (int r = 0; r < NR / 2; ++r) {
-                            const f16x2 av = {(_Float16)a[2 * r], (_Float16)a[2 * r + 1]};
-                            h[bi][bj][r] = __builtin_bit_cast(
-                                uint32_t, __builtin_elementwise_fma(
-                                              -av, f16x2{bv, bv},
-                                              __builtin_bit_cast(f16x2, h[bi][bj][r])));
-                        }
-                    });
+                uint32_t h0[NR / 2], h[NR / 2];
+                get_held(h0);
+                if (packed) {
+                    packed_leaves(As, Bs, kmax, std::false_type{});
+                } else if (!special) {
+                    packed_leaves32(As, Bs, kmax);
                 } else {
-                    for_k(As, Bs, kmax, [&](int bi, int bj, const float* a, float b) {
-                        if constexpr (NR == 16) mix_fnma_pairs16(a, b, h[bi][bj]);
-                        else mix_fnma_pairs4(a, b, h[bi][bj]);
+                    get_held(h);
+                    for_k32(As, Bs, kmax, [&](const float* a, const float* b) {
+                        float av[NR], bv[NR];
+                        spread(a, b, av, bv);
+                        if constexpr (NR == 16) mix_fnma_pairs16(av, bv, h);
+                        else mix_fnma_pairs4(av, bv, h);
                     });
+                    put_held(h);
                 }
+                get_held(h);
                 bool over = false;
 #pragma unroll
-                for (int bi = 0; bi < WMB; ++bi)
-#pragma unroll
-                    for (int bj = 0; bj < WNB; ++bj)
-#pragma unroll
-                        for (int r = 0; r < NR / 2; ++r) {
-                            const uint32_t e = ~h[bi][bj][r];   // exponent all ones: inf or NaN
-                            over |= (e & 0x7C00u) == 0u || (e & 0x7C000000u) == 0u;
-                        }
-                const bool redo = __any(over);
-                if (redo) {
-#pragma unroll
-                    for (int bi = 0; bi < WMB; ++bi)
-#pragma unroll
-                        for (int bj = 0; bj < WNB; ++bj)
-#pragma unroll
-                            for (int r = 0; r < NR / 2; ++r) h[bi][bj][r] = h0[bi][bj][r];
+                for (int r = 0; r < NR / 2; ++r) {
+                    const uint32_t e = ~h[r];   // exponent all ones: inf or NaN
+                    over |= (e & 0x7C00u) == 0u || (e & 0x7C000000u) == 0u;
+                }
+                if (__any(over)) {
+                    put_held(h0);
                     unhold();
                 }
-                held = !redo;
             }
-            if (__builtin_expect(!held, 0)) general_slice(As, Bs, kmax);
+            if (__builtin_expect(!held, 0)) general_slice(packed, As, Bs, kmax);
         } else {
             if (__builtin_expect(special, 0)) {
-                general_slice(As, Bs, kmax);
+                if (KIND == kChainMant10 && held) unhold();
+                general_slice(packed, As, Bs, kmax);
                 accL = -1000;
                 return;
             }
@@ -1069,12 +1288,12 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
                                 for (int r = 0; r < NR; ++r) acc[bi][bj][r] = c[bi][bj][r];
                     } else {
                         accL = -1000;
-                        directed(Aq, Bq, min(32, kmax - kq));
+                        directed(false, Aq, Bq, min(32, kmax - kq));
                     }
                 }
             } else if constexpr (KIND == kChainMant10) {
-                // 10 bits: binary16's significand, any exponent.  Held for 32 k as binary16 pairs
-                // scaled by 2^hs, hs the same for the wave: below 2^15, and from 2^-14 up, binary16 rounds a
+                // 10 bits: binary16's significand, any exponent.  Held as binary16 values scaled by
+                // 2^hs, hs the same for the wave: below 2^15, and from 2^-14 up, binary16 rounds a
                 // sum as the accumulator does.  Below 2^-14 it does too where every sum is a
                 // multiple of 2^-24 scaled (then it has at most 10 bits there); elsewhere the least
                 // result tells: above 2^-14, no sum was below.  Bounds per 32 k, for the wave: sums
@@ -1093,10 +1312,28 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
                 const int bTop = amB == 0u ? -1000 : (int)(amB >> 24) - 127;
                 const float pm = fmaxf(__uint_as_float(amA >> 1) * __uint_as_float(amB >> 1), 0x1p-126f) *
                                  1.0000152587890625f;
+                auto held_leaves = [&](const float* Aq, const float* Bq, int kn) {
+                    if (!packed) packed_leaves32(Aq, Bq, kn);
+                    else if (hs == 0) packed_leaves(Aq, Bq, kn, std::false_type{});
+                    else packed_leaves(Aq, Bq, kn, std::true_type{});
+                };
                 for (int kq = 0; kq < kmax; kq += 32) {
-                    const float* Aq = As + kq / 4 * LA::GROUP;
-                    const float* Bq = Bs + kq / 4 * LB::GROUP;
+                    const float* Aq = As + kq / 4 * (packed ? 4 * PGA : LA::GROUP);
+                    const float* Bq = Bs + kq / 4 * (packed ? 4 * PGB : LB::GROUP);
                     const int kn = min(32, kmax - kq);
+                    // Held already: a bound carried from one 32 k to the next, no look at the values.
+                    if (held) {
+                        const float bnd = __builtin_fmaf(33.0f, pm, acc_bound) * 1.0158f;   // 1.015749...
+                        const int S = __builtin_amdgcn_readfirstlane((int)(__float_as_uint(bnd) >> 23)) - 126;
+                        if (!wide16 && S <= 15 - hs && S <= 127 && bTop <= 15 - hs &&
+                            min(sL, bLsb) >= -24 - hs && sL >= -126) {
+                            accL = min(accL, sL);
+                            acc_bound = bnd;
+                            held_leaves(Aq, Bq, kn);
+                            continue;
+                        }
+                        unhold();
+                    }
                     // the wave's largest and smallest accumulator magnitudes
                     float hi_f = 0.0f, lo_f = 0x1.fffffep+127f;
 #pragma unroll
@@ -1133,22 +1370,15 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
                     const int L = min(sL, accL);
                     // hs for the grid: 2^L to 2^-24 or above, 2^S to 2^15 or below, B within binary16
                     const int gLo = max(-24 - L, -24 - bLsb), gHi = min(15 - S, 15 - bTop);
-                    grid = grid && L >= -126 && gLo <= gHi;
+                    grid = grid && L >= -126 && gLo <= gHi && (!packed || (gLo <= 15 && gHi >= -24));
                     if (grid) {
                         accL = L;
-                        hold(gHi);
-                        for_k(Aq, Bq, kn, [&](int bi, int bj, const float* a, float b) {
-                            const _Float16 bv = (_Float16)__builtin_ldexpf(b, hs);
-#pragma unroll
-                            for (int r = 0; r < NR / 2; ++r) {
-                                const f16x2 av = {(_Float16)a[2 * r], (_Float16)a[2 * r + 1]};
-                                h[bi][bj][r] = __builtin_bit_cast(
-                                    uint32_t, __builtin_elementwise_fma(
-                                                  -av, f16x2{bv, bv},
-                                                  __builtin_bit_cast(f16x2, h[bi][bj][r])));
-                            }
-                        });
-                        unhold();
+                        // none where it can be, else in the middle, so that it lasts; itself a
+                        // binary16 value where a packed B is scaled
+                        const int mid = gLo <= 0 && gHi >= 0 ? 0 : (gLo + gHi) >> 1;
+                        hold(packed ? max(min(mid, 15), -24) : mid);
+                        acc_bound = bnd;
+                        held_leaves(Aq, Bq, kn);
                         continue;
                     }
                     accL = -1000;
@@ -1157,22 +1387,30 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
                     const int eLo = (int)(lo >> 23) - 127;
                     const int cLo = max(-14 - eLo, -126 - bLsb), cHi = min(min(15 - S, 112), 126 - bTop);
                     if (in && lo != 0u && cLo <= cHi) {
-                        hold(cHi);
-                        uint32_t least = 0x7BFFu;
-                        for_k(Aq, Bq, kn, [&](int bi, int bj, const float* a, float b) {
-                            const float bs = __builtin_ldexpf(b, hs);
-                            if constexpr (NR == 16) mix_fnma_pairs16(a, bs, h[bi][bj], least);
-                            else mix_fnma_pairs4(a, bs, h[bi][bj], least);
+                        uint32_t u[NR], least = 0x7BFFu;
+#pragma unroll
+                        for (int r = 0; r < NR; ++r)
+                            u[r] = __builtin_bit_cast(uint16_t, (_Float16)__builtin_ldexpf(acc[0][0][r], cHi));
+                        for_k(packed, Aq, Bq, kn, [&](const float* a, const float* b) {
+                            float bs[NB], av[NR], bv[NR];
+#pragma unroll
+                            for (int c = 0; c < NB; ++c) bs[c] = __builtin_ldexpf(b[c], cHi);
+                            spread(a, bs, av, bv);
+                            if constexpr (NR == 16) mix_fnma16_least(av, bv, u, least);
+                            else mix_fnma4_least(av, bv, u, least);
                         });
                         if (__all((least & 0xFFFFu) > 0x0400u)) {   // 2^-14
-                            unhold();
+#pragma unroll
+                            for (int r = 0; r < NR; ++r)
+                                acc[0][0][r] = __builtin_ldexpf(
+                                    (float)__builtin_bit_cast(_Float16, (uint16_t)u[r]), -cHi);
                             continue;
                         }
                     }
-                    directed(Aq, Bq, kn);
+                    directed(packed, Aq, Bq, kn);
                 }
             } else {
-                directed(As, Bs, kmax);
+                directed(false, As, Bs, kmax);
             }
         }
     };
@@ -1181,9 +1419,12 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
     // meanwhile the store of slice s + 1 sets flag (s + 1) % 3 and flag (s + 2) % 3 (read last by
     // slice s - 1, before this slice's barrier) is cleared for slice s + 2.
     if constexpr (kFlag) {
-        if (tid < 3) flags[tid] = flags[tid + 36] = 0u;
+        if (tid < 3) flags[tid] = flags[tid + 36] = flags[tid + 40] = 0u;
         lds_barrier();
     }
+    // Slices are stored packed until one does not fit: that one is stored again, from the registers
+    // that still hold it, and the tile's others as FP32.
+    bool packed = kPack;
     int fs = 0, buf = 1;
     for (int k0 = -BK; k0 < g.K; k0 += BK) {   // the first pass only loads slice 0
         bool special = false, wide16 = false;
@@ -1191,12 +1432,20 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
         const int fn = k0 < 0 ? 0 : fs == 2 ? 0 : fs + 1;
         if constexpr (kFlag) {
             if (k0 >= 0) {
-                special = __builtin_amdgcn_readfirstlane((int)flags[fs]) != 0;
-                if constexpr (kWide) wide16 = __builtin_amdgcn_readfirstlane((int)flags[fs + 36]) != 0;
+                auto flag = [&](int i) { return __builtin_amdgcn_readfirstlane((int)flags[fs + i]) != 0; };
+                if (kPack && packed) {
+                    packed = !flag(kStat ? 40 : 0);
+                    if (!packed) {   // (no other slice's flags are set or read here)
+                        store_slice(buf, fs, false);
+                        lds_barrier();
+                    }
+                }
+                special = flag(0);
+                if constexpr (kWide) wide16 = flag(36);
                 if (tid == 0) {
                     const int fc = fn == 2 ? 0 : fn + 1;
                     flags[fc] = 0u;
-                    if constexpr (kWide) flags[fc + 36] = 0u;
+                    if constexpr (kWide) flags[fc + 36] = flags[fc + 40] = 0u;
                 }
             }
         }
@@ -1205,7 +1454,7 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
         const float* As = smem + buf * T::BUF_FLOATS;
         const float* Bs = As + LA::FLOATS;
         if constexpr (kStep) {
-            if (k0 >= 0) step_slice(As, Bs, min(BK, g.K - k0), special, wide16, buf);
+            if (k0 >= 0) step_slice(packed, As, Bs, min(BK, g.K - k0), special, wide16, buf);
         }
         // chunks that hold a k < K (none in the first pass)
         const int nq = kStep || k0 < 0 ? 0 : min(BK, g.K - k0 + CHUNK - 1) / CHUNK;
@@ -1279,7 +1528,7 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
             }
         }
         buf ^= 1;
-        if (has_next) store_slice(buf, fn);
+        if (has_next) store_slice(buf, fn, packed);
         fs = fn;
     }
     if constexpr (PIPE) {   // the last chunk's leaves
@@ -1288,7 +1537,7 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
         for (int n = 0; n < PIECES; ++n) piece(prev, n, sprev);
     }
 
-    if constexpr (kStep && KIND == kChainHalf)
+    if constexpr (kPack)
         if (held) unhold();
     // epilogue (cutlass LinearCombination): D = alpha * acc, or fma(alpha, acc, beta * C);
     // a convolution's D(m, n) / C(m, n) sit at b * sdb + m * sdm + (p * Q + q) * sdpq
@@ -1296,16 +1545,19 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
     for (int bi = 0; bi < WMB; ++bi)
 #pragma unroll
         for (int bj = 0; bj < WNB; ++bj) {
-            const int gn = n0 + bn0 + bj * BS + lcol;
-            int64_t col = gn, row_stride_d = g.ldd, row_stride_c = g.ldc;
-            if constexpr (CONV) {
-                const uint32_t b = fast_div((uint32_t)gn, g.cv.div_pq);
-                col = (int64_t)b * g.cv.sdb + (int64_t)((uint32_t)gn - b * g.cv.PQ) * g.cv.sdpq;
-                row_stride_d = row_stride_c = g.cv.sdm;
-            }
+            int64_t col = 0;
+            const int64_t row_stride_d = CONV ? g.cv.sdm : g.ldd, row_stride_c = CONV ? g.cv.sdm : g.ldc;
 #pragma unroll
             for (int r = 0; r < NR; ++r) {
-                const int gm = m0 + am0 + bi * BS + (r >> 2) * 8 + lhi * 4 + (r & 3);
+                const int gn = n0 + bn0 + bj * BS + out_col(r);
+                if (r == 0 || out_col(r) != out_col(r - 1)) {
+                    col = gn;
+                    if constexpr (CONV) {
+                        const uint32_t b = fast_div((uint32_t)gn, g.cv.div_pq);
+                        col = (int64_t)b * g.cv.sdb + (int64_t)((uint32_t)gn - b * g.cv.PQ) * g.cv.sdpq;
+                    }
+                }
+                const int gm = m0 + am0 + bi * BS + out_row(r);
                 if (gm >= g.M || gn >= g.N) continue;
                 const float a = kNeg ? -acc[bi][bj][r] : acc[bi][bj][r];
                 float d;

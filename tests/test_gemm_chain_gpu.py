@@ -111,7 +111,7 @@ def test_conv(dev, case, chunk):
             assert_bits(y, ref, f"conv {case} {kind} chunk {chunk} config {cfg}")
 
 
-@pytest.mark.parametrize("bits", [10, 23])
+@pytest.mark.parametrize("bits", [10, 23, HALF], ids=str)
 @pytest.mark.parametrize("case", ["grows", "mixed", "zeros", "one_bit", "columns", "zero_a"])
 def test_chunk_1_leaf_changes(dev, case, bits):
     """Chunk 1, 23 bits: slices whose sums are all exact run on the MFMA, the others leaf by leaf,
@@ -119,7 +119,8 @@ def test_chunk_1_leaf_changes(dev, case, bits):
     half way), as columns of 24-bit values come in, over zero sums of both signs, and with one
     inexact term in an otherwise exact product.  10 bits: from the packed binary16 leaves on the
     grid to the checked and the directed ones and back, with columns 2^40 apart in a wave and a
-    zero operand slice beside large values."""
+    zero operand slice beside large values.  Binary16: from packed slices to FP32 ones where a value
+    is no binary16 one."""
     import lofloat_amd as lof
     M, N, K = 70, 66, 520
     g = np.random.default_rng(31)
