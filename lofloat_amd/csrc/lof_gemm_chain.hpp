@@ -34,9 +34,9 @@
 //   binary16-shaped, 10 bits    one binary16 FMA on binary16 operands, two leaves an instruction,
 //                               from slices kept as binary16 pairs (2.2 cycles a leaf); one
 //                               mixed FMA on FP32 operands (8.4; 10 bits: 2.6 more for the check).
-// e4m3 operands, 10 bits, before and after the slices were kept as binary16 pairs: 4096^3 3.6 ->
-// 2.28 ms, 1000x768x3072 259 -> 196 us, a 3x3 convolution 128x25088x1152 290 -> 190 us; binary16-
-// shaped: 1.84 ms, 133 us, 152 us.
+// e4m3 operands, before and after the slices were kept as binary16 pairs, 10 bits: 4096^3 3.68 ->
+// 2.28 ms, 1000x768x3072 293 -> 196 us, 128x25088x1152 301 -> 190 us; binary16-shaped: 2.86 -> 1.84
+// ms, 216 -> 133 us, 243 -> 152 us.
 //
 // Tile: 4 waves, each WMB x WNB blocks of BS x BS outputs (BS = 32, or 16 for products with few
 // outputs, where a 32-row block would leave most of the chip idle).  A and B slices of BK k sit
@@ -798,8 +798,18 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
         put(As, LA{}, std::integral_constant<int, BM>{}, va, g.ta != 0, ka);
         put(As + LA::FLOATS, LB{}, std::integral_constant<int, BN>{}, vb, CONV || g.tb == 0, kb);
     };
-    // fl: the slice's flags
-    auto store_slice = [&](int buf, int fl, bool packed) {
+    // Statistics that cannot help are not taken: after a slice whose products alone are too wide
+    // for exact sums or the grid, the next ones (1, 3, 7, then 15 in turn, for as long as they stay
+    // so) are stored without them (a 2048x1024x4096 training step on FP32 operands, 23 bits: 2.77 ->
+    // 2.45 ms; 4096^3 on FP32 operands, 10 bits: 7.34 -> 7.08 ms).
+    int skip = 0, last_skip = 0;
+    auto judge = [&](bool hopeless) {
+        last_skip = hopeless ? min(2 * last_skip + 1, 15) : 0;
+        skip = last_skip;
+    };
+    // fl: the slice's flags; full: with every statistic (else 10 bits' largest magnitudes and a
+    // bound on B's exponents only)
+    auto store_slice = [&](int buf, int fl, bool packed, bool full) {
         Pairs pa, pb;
         put_slice(buf, packed, pa, pb);
         if (kPack && packed) {
@@ -830,6 +840,24 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
             over(va, sum);
             over(vb, sum);
             if (z != 0.0f) flags[fl] = 1u;   // z is +-0 or NaN
+        }
+        if (!full) {
+            if constexpr (kWide) {
+                uint32_t ma = 0u, mb = 0u, nb = ~0u;
+                over(va, [&](float x) { ma = max(ma, __float_as_uint(x) << 1); return false; });
+                over(vb, [&](float x) {
+                    const uint32_t b = __float_as_uint(x) << 1;
+                    mb = max(mb, b);
+                    nb = min(nb, b - 1u);
+                    return false;
+                });
+                ma = wave_max_u32(ma);
+                mb = wave_max_u32(mb);
+                nb = wave_min_u32(nb) >> 24;   // the least exponent of B's values, in place of the lowest bit's
+                if (lane == 63)
+                    *(uint4*)(stats + buf * 16 + wave * 4) = make_uint4(ma, 0u, mb, nb == 0u ? 1u : nb + 23u);
+            }
+            return;
         }
         if constexpr (kWide) {   // A binary16 values, B of at most 11 significant bits
             if (over(va, not16) | over(vb, [](float x) { return (__float_as_uint(x) & 0x1FFFu) != 0u; }))
@@ -1145,7 +1173,7 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
         put_held(hp);
     };
     auto step_slice = [&](bool packed, const float* As, const float* Bs, int kmax, bool special,
-                          bool wide16, int buf) {
+                          bool wide16, bool full, int buf) {
         if constexpr (KIND == kChainHalf) {
             // Held as binary16 pairs while every accumulator is a binary16 value below 2^15 at a
             // slice's start.  The binary16 FMA (operands binary16 too: packed, two leaves an
@@ -1209,6 +1237,11 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
                 // are the negated RTO24 zeros.  All sums are multiples of 2^L, L the lower of the
                 // products' lowest bit (from the slice's statistics) and the accumulators', and
                 // below 2^S with 2^S > |acc| + 33 amax_A amax_B: exact when S <= L + 24.
+                if (!full) {
+                    accL = -1000;
+                    directed(false, As, Bs, kmax);
+                    return;
+                }
                 uint32_t amA = 0u, amB = 0u, kyA = ~0u, kyB = ~0u;
 #pragma unroll
                 for (int w = 0; w < 4; ++w) {
@@ -1220,6 +1253,8 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
                 // an upper bound on a product's magnitude, at least 2^-126
                 const float pm = fmaxf(__uint_as_float(amA >> 1) * __uint_as_float(amB >> 1), 0x1p-126f) *
                                  1.0000152587890625f;
+                judge(__builtin_amdgcn_readfirstlane((int)(__float_as_uint(pm) >> 23)) - 126 >
+                      __builtin_amdgcn_readfirstlane(sL) + 24);
                 for (int kq = 0; kq < kmax; kq += 32) {
                     float am = 0.0f;
 #pragma unroll
@@ -1307,11 +1342,14 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
                     amB = max(amB, v.z); kyB = min(kyB, v.w);
                 }
                 const bool zero = amA == 0u || amB == 0u;
-                const int sL = zero ? 1000 : (int)kyA + (int)kyB - 300;
+                const int sL = !full ? -1000 : zero ? 1000 : (int)kyA + (int)kyB - 300;
                 const int bLsb = amB == 0u ? 1000 : (int)kyB - 150;
                 const int bTop = amB == 0u ? -1000 : (int)(amB >> 24) - 127;
                 const float pm = fmaxf(__uint_as_float(amA >> 1) * __uint_as_float(amB >> 1), 0x1p-126f) *
                                  1.0000152587890625f;
+                if (full && !packed)
+                    judge(wide16 || __builtin_amdgcn_readfirstlane((int)(__float_as_uint(pm) >> 23)) - 126 >
+                                        __builtin_amdgcn_readfirstlane(sL) + 39);
                 auto held_leaves = [&](const float* Aq, const float* Bq, int kn) {
                     if (!packed) packed_leaves32(Aq, Bq, kn);
                     else if (hs == 0) packed_leaves(Aq, Bq, kn, std::false_type{});
@@ -1425,6 +1463,7 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
     // Slices are stored packed until one does not fit: that one is stored again, from the registers
     // that still hold it, and the tile's others as FP32.
     bool packed = kPack;
+    bool full = true;   // slice k0's statistics
     int fs = 0, buf = 1;
     for (int k0 = -BK; k0 < g.K; k0 += BK) {   // the first pass only loads slice 0
         bool special = false, wide16 = false;
@@ -1436,7 +1475,7 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
                 if (kPack && packed) {
                     packed = !flag(kStat ? 40 : 0);
                     if (!packed) {   // (no other slice's flags are set or read here)
-                        store_slice(buf, fs, false);
+                        store_slice(buf, fs, false, true);
                         lds_barrier();
                     }
                 }
@@ -1454,7 +1493,7 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
         const float* As = smem + buf * T::BUF_FLOATS;
         const float* Bs = As + LA::FLOATS;
         if constexpr (kStep) {
-            if (k0 >= 0) step_slice(packed, As, Bs, min(BK, g.K - k0), special, wide16, buf);
+            if (k0 >= 0) step_slice(packed, As, Bs, min(BK, g.K - k0), special, wide16, full, buf);
         }
         // chunks that hold a k < K (none in the first pass)
         const int nq = kStep || k0 < 0 ? 0 : min(BK, g.K - k0 + CHUNK - 1) / CHUNK;
@@ -1528,7 +1567,11 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
             }
         }
         buf ^= 1;
-        if (has_next) store_slice(buf, fn, packed);
+        if (has_next) {
+            full = skip == 0;
+            skip = full ? 0 : skip - 1;
+            store_slice(buf, fn, packed, full);
+        }
         fs = fn;
     }
     if constexpr (PIPE) {   // the last chunk's leaves
