@@ -70,11 +70,15 @@ const GemmConfig kConfigs[] = {
     LOF_GEMM_SHORT_CFG(32, 32),
     LOF_GEMM_SHORT_CFG(16, 64),
     LOF_GEMM_SHORT_CFG(64, 16),
+    LOF_GEMM_SHORT_CFG(16, 16),
 };
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
 constexpr int kFirstMfma = 5, kMfma64 = 7, kMfma64x128 = 8, kFirstShort = 9;
-constexpr bool kShortTile[kChainTiles] = {false, false, true, true, true};
-constexpr int kShortMantTiles = 64;
+constexpr bool kShortTile[kChainTiles] = {false, false, true, true, true, true};
+// 64x64 tiles up to which a directed accumulator takes the short tiles.  Measured (us, 7 bits, the wave
+// tile and 32x32; e4m3 / FP32 operands): 2048x1024x1024, 512 tiles, 374 / 507 against 362 / 364;
+// 2048x2048x1024, 1024 tiles, 618 / 848 against 677 / 680.
+constexpr int kShortMantTiles = 512;
 
 // chunks whose sums can run on MFMA
 bool chunk_fits_mfma(int chunk) { return chunk >= 2 && chunk <= 32 && (32 % chunk) == 0; }
@@ -127,14 +131,16 @@ TuneKey tune_key(const lof_gemm_desc& d) {
 // tile for other chunks, the 32x32 one when there are too few tiles to fill the chip.
 int default_config(const lof_gemm_desc& d) {
     if (chunk_fits_wave_tile(d.accum.chunk)) {
-        const int t = chain_default_tile(d.M, d.N);
         const lof_accum& ac = d.accum;
         const bool mant = ac.kind == LOF_ACCUM_MANTISSA;
+        const bool directed = mant && ac.chunk == 1 && ac.mant_bits != 23 && ac.mant_bits != 10;
+        const int t = chain_default_tile(d.M, d.N, ac.chunk,
+                                         few_takes(d.M, d.N, d.K, d.trans_a != 0, d.trans_b != 0), directed);
         const bool half = !mant && ac.fmt.mantissa_bits == 10 && ac.fmt.bias == 15;
         if (ac.spec.mode == RNE && (half || (mant && (ac.chunk > 1 || ac.mant_bits == 23 || ac.mant_bits == 10))))
             return kChainConfigOf[t];
         if (ac.spec.mode == RNE && mant && kShortTile[t] &&
-            (int64_t)((d.M + 63) / 64) * ((d.N + 63) / 64) < kShortMantTiles)
+            (int64_t)((d.M + 63) / 64) * ((d.N + 63) / 64) <= kShortMantTiles)
             return kChainConfigOf[t];
         const int64_t tiles_64x128 = (int64_t)((d.M + 63) / 64) * ((d.N + 127) / 128);
         return tiles_64x128 >= 768 ? kMfma64x128 : kMfma64;
@@ -162,16 +168,24 @@ void set_chain(GemmArgs* g, bool conv) {
     }
 }
 
-// Short dimensions take the tile that wastes least of them; else 64x64 from 768 tiles (three a
-// CU) on and 32x32 below, where 64x64 leaves CUs idle or unevenly loaded.  Measured (us, chunk
-// 32 / 8, 23 / 10 bits): 2048x2048x2048, 1024 tiles, 64x64 178 / 364, 32x32 244 / 410;
-// 2048x1024x4096, 512 tiles, 226 / 458 against 241 / 408; 1000x768x3072, 192 tiles, 189 / 322
-// against 98 / 156.  8x4096x4096: 16x64 86 / 151, 32x32 106 / 171.  128x128 ties with 64x64 on the
-// largest products and loses below 1024 tiles of its own.
-int chain_default_tile(int64_t M, int64_t N) {
+// The 16x16 tile, an output a lane, up to three workgroups a CU; above, short dimensions take the
+// tile that wastes least of them, else 64x64 from 768 tiles (three a CU) on and 32x32 below, where
+// 64x64 leaves CUs idle or unevenly loaded.  Measured (us, chunk 32 / 8, 23 / 10 bits):
+// 2048x2048x2048, 1024 tiles, 64x64 178 / 364, 32x32 244 / 410; 2048x1024x4096, 512 tiles, 226 /
+// 458 against 241 / 408; 1000x768x3072, 192 tiles, 189 / 322 against 98 / 156.  128x128 ties with
+// 64x64 on the largest products and loses below 1024 tiles of its own.  16x16 against the best of the others
+// (FP32 operands, chunk 1 at 23 / 10 bits, chunk 8 at 10, chunk 32 at 23): 8x4096x4096, 256 tiles, 88 /
+// 108, 61, 55 against 305 / 328, 149, 84; 256x512x1024, 512 tiles, 32 / 40, 20, 19 against 76 / 84, 35,
+// 19; 512x512x1024, 1024 tiles, 49 / 58, 30, 29 against 78 / 85, 36, 20.  Chunk 2 has no 16-row MFMA (it
+// takes 4 k), and 16x16 ties with 64x64 only at 2048x1024 (1024x1024x1024 158 against 249).
+// Accumulators whose chunk-1 leaves are all directed (`directed`) gain up to twelve workgroups a CU:
+// 1000x768x3072 462 against 32x32's 490, 1024x1024x1024 212 against 207.
+int chain_default_tile(int64_t M, int64_t N, int chunk, bool few, bool directed) {
+    const int64_t t16 = ((M + 15) / 16) * ((N + 15) / 16), t64 = ((M + 63) / 64) * ((N + 63) / 64);
+    if (few && (t16 <= (directed ? 3072 : 768) || (chunk == 2 && t64 < 512))) return 5;
     if (M <= 16) return 3;
     if (N <= 16) return 4;
-    return ((M + 63) / 64) * ((N + 63) / 64) >= 768 ? 1 : 2;
+    return t64 >= 768 ? 1 : 2;
 }
 
 lof_status launch_chain(const GemmArgs& g, int tile, hipStream_t st, const char* what) {
@@ -180,6 +194,7 @@ lof_status launch_chain(const GemmArgs& g, int tile, hipStream_t st, const char*
                           : g.chain == kChainMant10 ? kChainTableMant10
                                                     : kChainTableMant;
     const int l2 = 31 - __builtin_clz((unsigned)g.chunk);
+    if (tile == 5 && !few_takes(g.M, g.N, g.K, g.ta != 0, g.tb != 0)) tile = 2;
     ChainKernel k = g.cv.conv ? t.conv[tile][l2] : t.gemm[tile][l2];
     if (!k) {   // chunk 2 on a 16-row block (its MFMA takes 4 k), chunk 1 on the widest tile
         tile = 1;

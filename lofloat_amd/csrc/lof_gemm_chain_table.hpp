@@ -3,6 +3,7 @@
 #pragma once
 
 #include "lof_gemm_chain.hpp"
+#include "lof_gemm_few.hpp"
 
 namespace lofamd {
 
@@ -11,6 +12,7 @@ namespace lofamd {
 //          wave, are slower than both at 4096^3 and at 1537 x 3001 x 2047 on every kind.)
 //   2      32x32: four 16x16 blocks, slices of 64 k
 //   3, 4   16x64 and 64x16: slices of 128 k
+//   5      16x16, an output a lane (lof_gemm_few.hpp)
 // The short blocks need few outputs for a full chip, and longer slices per barrier because a
 // slice of one block is only a quarter as long on the matrix cores.
 using ChainT0 = ChainTile<32, 2, 2, 2, 2, 32>;
@@ -18,7 +20,7 @@ using ChainT1 = ChainTile<32, 2, 2, 1, 1, 32>;
 using ChainT2 = ChainTile<16, 2, 2, 1, 1, 64>;
 using ChainT3 = ChainTile<16, 1, 4, 1, 1, 128>;
 using ChainT4 = ChainTile<16, 4, 1, 1, 1, 128>;
-constexpr int kChainTiles = 5;
+constexpr int kChainTiles = 6;
 
 // Tile t of `tiles` in launch order: each XCD (workgroups go to the 8 XCDs in turn) takes a
 // contiguous run of tiles, walked in groups of 8 tile rows, so that the tiles in flight on one
@@ -50,6 +52,13 @@ __global__ __launch_bounds__(256, kChainWaves<T>) void k_gemm_chain(GemmArgs g, 
     gemm_tile_chain<T, CHUNK, KIND, CONV>(g, t.x, t.y, (int)threadIdx.x, smem);
 }
 
+template <int CHUNK, int KIND>
+__global__ __launch_bounds__(256, 4) void k_gemm_few(GemmArgs g, unsigned tm, unsigned tn) {
+    __shared__ __align__(16) float smem[kFewSmem];
+    const int2 t = chain_tile_of(blockIdx.x, tm, tn);
+    gemm_tile_few<CHUNK, KIND>(g, t.x, t.y, (int)threadIdx.x, smem);
+}
+
 using ChainKernel = void (*)(GemmArgs, unsigned, unsigned);
 
 // [tile][log2(chunk)]; nullptr where a chunk of 2 is shorter than the block's MFMA, and for chunk
@@ -73,25 +82,28 @@ constexpr ChainKernel chain_kernel() {
 #define LOF_CHAIN_TABLE(KIND)                                                               \
     {{LOF_CHAIN_ROW(ChainT0, KIND, false), LOF_CHAIN_ROW(ChainT1, KIND, false),              \
       LOF_CHAIN_ROW(ChainT2, KIND, false), LOF_CHAIN_ROW(ChainT3, KIND, false),              \
-      LOF_CHAIN_ROW(ChainT4, KIND, false)},                                                  \
+      LOF_CHAIN_ROW(ChainT4, KIND, false),                                                   \
+      {k_gemm_few<1, KIND>, k_gemm_few<2, KIND>, k_gemm_few<4, KIND>, k_gemm_few<8, KIND>,   \
+       k_gemm_few<16, KIND>, k_gemm_few<32, KIND>}},                                         \
      {{}, LOF_CHAIN_ROW(ChainT1, KIND, true), LOF_CHAIN_ROW(ChainT2, KIND, true),            \
-      LOF_CHAIN_ROW(ChainT3, KIND, true), {}}}
+      LOF_CHAIN_ROW(ChainT3, KIND, true), {}, {}}}
 
 // chunk 1 alone (longer chunks of a 10-bit accumulator are kChainMant's)
 #define LOF_CHAIN_ROW1(T, KIND, CONV) {chain_kernel<T, 1, KIND, CONV>(), {}, {}, {}, {}, {}}
 #define LOF_CHAIN_TABLE1(KIND)                                                              \
     {{{}, LOF_CHAIN_ROW1(ChainT1, KIND, false), LOF_CHAIN_ROW1(ChainT2, KIND, false),        \
-      LOF_CHAIN_ROW1(ChainT3, KIND, false), LOF_CHAIN_ROW1(ChainT4, KIND, false)},           \
+      LOF_CHAIN_ROW1(ChainT3, KIND, false), LOF_CHAIN_ROW1(ChainT4, KIND, false),            \
+      {k_gemm_few<1, KIND>, {}, {}, {}, {}, {}}},                                            \
      {{}, LOF_CHAIN_ROW1(ChainT1, KIND, true), LOF_CHAIN_ROW1(ChainT2, KIND, true),          \
-      LOF_CHAIN_ROW1(ChainT3, KIND, true), {}}}
+      LOF_CHAIN_ROW1(ChainT3, KIND, true), {}, {}}}
 
 extern const ChainTable kChainTableMant, kChainTableMant10, kChainTableMant23, kChainTableHalf;
 
 // The dimensions of tile t.
 struct ChainDims { int bm, bn; };
-constexpr ChainDims kChainDims[kChainTiles] = {{128, 128}, {64, 64}, {32, 32}, {16, 64}, {64, 16}};
+constexpr ChainDims kChainDims[kChainTiles] = {{128, 128}, {64, 64}, {32, 32}, {16, 64}, {64, 16}, {16, 16}};
 // GEMM configs 5.. (lof_gemm.hip) and the tile each runs on here, and back
-constexpr int kChainTileOf[7] = {0, 1, 1, 1, 2, 3, 4};
-constexpr int kChainConfigOf[kChainTiles] = {5, 7, 9, 10, 11};
+constexpr int kChainTileOf[8] = {0, 1, 1, 1, 2, 3, 4, 5};
+constexpr int kChainConfigOf[kChainTiles] = {5, 7, 9, 10, 11, 12};
 
 }  // namespace lofamd

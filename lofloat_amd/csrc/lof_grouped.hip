@@ -456,7 +456,11 @@ lof_status launch_alone(const GroupTask& t, hipStream_t st) {
         d.accum.kind = t.g.acc_kind;
         d.accum.chunk = t.g.chunk;
         if (t.g.chain >= 0 && (t.g.chunk > 1 || t.g.chain != kChainMant))
-            return launch_chain(t.g, chain_default_tile(t.g.M, t.g.N), st, "lof_grouped launch");
+            return launch_chain(t.g,
+                                chain_default_tile(t.g.M, t.g.N, t.g.chunk,
+                                                   few_takes(t.g.M, t.g.N, t.g.K, t.g.ta != 0, t.g.tb != 0),
+                                                   t.g.chunk == 1 && t.g.chain == kChainMant),
+                                st, "lof_grouped launch");
         return launch_gemm(t.g, resolve_gemm_config(d, -1), st);
     }
     }

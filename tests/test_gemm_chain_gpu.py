@@ -12,7 +12,7 @@ from conftest import assert_bits
 pytestmark = pytest.mark.gpu
 
 HALF, HALF_EXT, HALF_WIDE = (16, 10, 15, 1, 0, 0), (16, 10, 15, 0, 0, 0), (18, 10, 15, 1, 0, 0)
-CONFIGS = range(5, 12)   # 128x128, 128x64, 64x64, 64x128, 32x32, 16x64, 64x16
+CONFIGS = range(5, 13)   # 128x128, 128x64, 64x64, 64x128, 32x32, 16x64, 64x16, 16x16
 
 
 def _accums(lof, kind, chunk):
