@@ -205,9 +205,13 @@ __device__ __noinline__ float chain_half_slow(float p, float na, LeafGen L) {
 }
 
 // The leaves of NR (4 or 8) outputs of a chunk.  acc: the accumulators (kChainHalf: negated).
-template <int KIND, int NR>
+// inside(o), wave-uniform: output o of some lane lies in the matrix.  Outputs past its edges repeat a
+// row or a column of it and are dropped: on their own they never take the general leaf
+// (sums past the top binade, chunk 2, 64x64 tile, us: 3x40000x256 5572 -> 872, 20x40000x256
+// 5611 -> 3105).
+template <int KIND, int NR, class Inside>
 __device__ __forceinline__ void chain_leaves(float (&p)[NR], float (&acc)[NR], bool special,
-                                             const GemmArgs& g) {
+                                             const GemmArgs& g, Inside inside) {
     if constexpr (KIND == kChainHalf) {
         float t[NR], top = 0.0f;
 #pragma unroll
@@ -218,7 +222,8 @@ __device__ __forceinline__ void chain_leaves(float (&p)[NR], float (&acc)[NR], b
         if (__builtin_expect(__any(top >= g.half_top), 0)) {
 #pragma unroll
             for (int o = 0; o < NR; ++o)
-                if (fabsf(t[o]) >= g.half_top) t[o] = chain_half_slow(p[o], acc[o], leaf_gen(g));
+                if (inside(o) && fabsf(t[o]) >= g.half_top)
+                    t[o] = chain_half_slow(p[o], acc[o], leaf_gen(g));
         }
 #pragma unroll
         for (int o = 0; o < NR; ++o) acc[o] = t[o];
@@ -884,6 +889,11 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
 #pragma unroll
             for (int r = 0; r < NR; ++r) acc[bi][bj][r] = kNeg ? -0.0f : 0.0f;
 
+    // rows and columns of the matrix from this wave's corner on
+    const int rows_in = g.M - m0 - __builtin_amdgcn_readfirstlane(am0);
+    const int cols_in = g.N - n0 - __builtin_amdgcn_readfirstlane(bn0);
+    const bool wave_in = rows_in > 0 && cols_in > 0;
+
     // Leaves in pieces of PN outputs.  PIPE: a chunk's leaves run between the next chunk's
     // MFMAs, from its second step on (the first piece still waits for the sums to settle), so
     // one wave keeps both the matrix cores and the VALU busy; the leaf before the first chunk
@@ -903,7 +913,10 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
             p[r] = sums[bi][bj][o0 + r];
             x[r] = acc[bi][bj][o0 + r];
         }
-        chain_leaves<KIND, PN>(p, x, spec, g);
+        chain_leaves<KIND, PN>(p, x, spec, g, [&](int o) {   // the lowest row of output o0 + o
+            const int row = bi * BS + ((o0 + o) >> 2) * 8 + ((o0 + o) & 3);
+            return row < rows_in && bj * BS < cols_in;
+        });
 #pragma unroll
         for (int r = 0; r < PN; ++r) acc[bi][bj][o0 + r] = x[r];
     };
@@ -1191,7 +1204,7 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
                             const float x = acc[bi][bj][r];
                             ok &= (float)(_Float16)x == x && fabsf(x) < 32768.0f;
                         }
-                if (__all(ok)) hold(0);
+                if (!wave_in || __all(ok)) hold(0);
             }
             if (held) {
                 uint32_t h0[NR / 2], h[NR / 2];
@@ -1217,7 +1230,7 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
                     const uint32_t e = ~h[r];   // exponent all ones: inf or NaN
                     over |= (e & 0x7C00u) == 0u || (e & 0x7C000000u) == 0u;
                 }
-                if (__any(over)) {
+                if (wave_in && __any(over)) {
                     put_held(h0);
                     unhold();
                 }

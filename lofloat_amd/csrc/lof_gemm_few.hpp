@@ -132,6 +132,9 @@ __device__ __forceinline__ void gemm_tile_few(const GemmArgs& g, int tile_m, int
     const int lane = tid & 63, wave = tid >> 6;
     const int row = tid / kFewB, colm = tid % kFewB;
     const int m0 = tile_m * kFewB, n0 = tile_n * kFewB;
+    // A wave past the matrix's rows repeats its last one; its outputs are dropped and take no general
+    // leaves.
+    const bool wave_in = m0 + 4 * __builtin_amdgcn_readfirstlane(wave) < g.M;
     uint32_t* flags = (uint32_t*)(smem + 2 * kFewBuf);
     uint32_t* stats = flags + 4;   // [buffer][wave][amax A, key A, amax B, key B]
     const float* A0 = g.A + (g.ta ? (int64_t)m0 : (int64_t)m0 * g.lda);
@@ -330,14 +333,14 @@ __device__ __forceinline__ void gemm_tile_few(const GemmArgs& g, int tile_m, int
     auto step_slice = [&](const float* S, int buf, int kmax, bool special, bool full) {
         if constexpr (KIND == kChainHalf) {
             // as gemm_tile_chain: one mixed FMA a k, redone if a result passed 65504
-            if (!held && __all((float)(_Float16)acc == acc && fabsf(acc) < 32768.0f)) {
+            if (!held && (!wave_in || __all((float)(_Float16)acc == acc && fabsf(acc) < 32768.0f))) {
                 held = true;
                 h = __builtin_bit_cast(uint16_t, (_Float16)acc);
             }
             if (held) {
                 const uint32_t h0 = h;
                 for_k4(S, 0, kmax, [&](const float4& a, const float4& b) { few_mix4(a, b, h); });
-                if (__any((h & 0x7C00u) == 0x7C00u)) {
+                if (wave_in && __any((h & 0x7C00u) == 0x7C00u)) {
                     acc = (float)__builtin_bit_cast(_Float16, (uint16_t)h0);
                     held = false;
                 }
@@ -484,7 +487,7 @@ __device__ __forceinline__ void gemm_tile_few(const GemmArgs& g, int tile_m, int
                    if (PER == 1 || st % PER == PER - 1) leaves();
                });
         if constexpr (KIND == kChainHalf)
-            if (__builtin_expect(__any(top >= g.half_top), 0)) {   // the top binade: the slice again
+            if (__builtin_expect(wave_in && __any(top >= g.half_top), 0)) {   // the top binade: the slice again
                 acc = acc0;
                 for (int k = 0; k < kmax; k += CHUNK) {
                     float x = 0.0f;

@@ -1,0 +1,65 @@
+"""GPU checks of the GEMM kernels at the edges of what their dispatch takes: outputs past the matrix,
+leading dimensions, output sizes, and which kernel a call runs on."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from conftest import assert_bits
+
+pytestmark = pytest.mark.gpu
+
+HALF = (16, 10, 15, 1, 0, 0)
+
+
+def _fmt(t):
+    import lofloat_amd as lof
+    return lof.FloatFormatDescriptor(*t, lof.formats.P3109_InfChecker(t[0]),
+                                     lof.formats.P3109_NaNChecker(t[0]))
+
+
+def _best_us(run, reps=8):
+    run()
+    times = []
+    for _ in range(reps):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        run()
+        b.record()
+        b.synchronize()
+        times.append(a.elapsed_time(b) * 1e3)
+    return min(times)
+
+
+def _overflowing(M, N, K, seed):
+    """Operands whose binary16 sums pass the format's top binade within a few k."""
+    g = np.random.default_rng(seed)
+    return ((g.uniform(0, 400, (M, K))).astype(np.float32),
+            (g.uniform(-40, 400, (K, N))).astype(np.float32))
+
+
+@pytest.mark.parametrize("chunk", [1, 2, 4, 8, 16, 32])
+@pytest.mark.parametrize("shape", [(3, 70, 64), (20, 130, 65), (33, 17, 96), (66, 65, 64)], ids=str)
+def test_overflow_at_the_matrix_edges(dev, shape, chunk):
+    import lofloat_amd as lof
+    M, N, K = shape
+    A, B = _overflowing(M, N, K, M + chunk)
+    ref = oracle.gemm(A, B, oracle.accum_fmt(HALF, chunk))
+    assert np.isinf(ref).any() or np.abs(ref).max() > 32768
+    Ad, Bd = torch.from_numpy(A).to(dev), torch.from_numpy(B).to(dev)
+    for cfg in (-1, *range(5, 13)):
+        y = lof.gemm(Ad, Bd, lof.AccumSpec(fmt=_fmt(HALF), chunk=chunk), config=cfg).cpu().numpy()
+        assert_bits(y, ref, f"{shape} chunk {chunk} config {cfg}")
+
+
+@pytest.mark.parametrize("chunk", [2, 8])
+def test_rows_past_the_matrix_take_no_general_leaf(dev, chunk):
+    """On the 64x64 tile, 3 rows of overflowing binary16 sums need at most a quarter of the general
+    leaves of 64 rows (none in the tile's lower half, 3 of 16 of a lane's outputs above); rows that
+    repeat the last one took as long as real ones."""
+    import lofloat_amd as lof
+    A, B = (torch.from_numpy(v).to(dev) for v in _overflowing(64, 20000, 128, 1))
+    acc = lof.AccumSpec(fmt=_fmt(HALF), chunk=chunk)
+    few = _best_us(lambda: lof.gemm(A[:3], B, acc, config=7))
+    full = _best_us(lambda: lof.gemm(A, B, acc, config=7))
+    assert few < 0.7 * full, (few, full)
