@@ -125,28 +125,10 @@ TuneKey tune_key(const lof_gemm_desc& d) {
                    d.accum.chunk};
 }
 
-// Untuned choice: the chunk-sum kernels' tile (chain_default_tile) where they run; at chunk 1 with
-// another accumulator 64x128 (each lane's A values serve two B columns) from 768 such tiles on
-// (4096^3: e4m3 +10-15 % over 64x64, 8e7m on the RTO leaves -4-9 %), else 64x64; the 32x64 VALU
-// tile for other chunks, the 32x32 one when there are too few tiles to fill the chip.
-int default_config(const lof_gemm_desc& d) {
-    if (chunk_fits_wave_tile(d.accum.chunk)) {
-        const lof_accum& ac = d.accum;
-        const bool mant = ac.kind == LOF_ACCUM_MANTISSA;
-        const bool directed = mant && ac.chunk == 1 && ac.mant_bits != 23 && ac.mant_bits != 10;
-        const int t = chain_default_tile(d.M, d.N, ac.chunk,
-                                         few_takes(d.M, d.N, d.K, d.trans_a != 0, d.trans_b != 0), directed);
-        const bool half = !mant && ac.fmt.mantissa_bits == 10 && ac.fmt.bias == 15;
-        if (ac.spec.mode == RNE && (half || (mant && (ac.chunk > 1 || ac.mant_bits == 23 || ac.mant_bits == 10))))
-            return kChainConfigOf[t];
-        if (ac.spec.mode == RNE && mant && kShortTile[t] &&
-            (int64_t)((d.M + 63) / 64) * ((d.N + 63) / 64) <= kShortMantTiles)
-            return kChainConfigOf[t];
-        const int64_t tiles_64x128 = (int64_t)((d.M + 63) / 64) * ((d.N + 127) / 128);
-        return tiles_64x128 >= 768 ? kMfma64x128 : kMfma64;
-    }
-    if ((int64_t)((d.M + 31) / 32) * ((d.N + 63) / 64) >= 1024) return 3;
-    return 4;
+int tuned_or_default(const lof_gemm_desc& d, const GemmArgs& g) {
+    std::lock_guard<std::mutex> lk(g_tune_mu);
+    auto it = g_tuned.find(tune_key(d));
+    return it != g_tuned.end() ? it->second : gemm_default_config(g);
 }
 
 }  // namespace
@@ -186,6 +168,32 @@ int chain_default_tile(int64_t M, int64_t N, int chunk, bool few, bool directed)
     if (M <= 16) return 3;
     if (N <= 16) return 4;
     return t64 >= 768 ? 1 : 2;
+}
+
+// Untuned choice: the chunk-sum kernels' tile (chain_default_tile) where they run, but for directed
+// accumulators only the short tiles, and only up to kShortMantTiles; the 32x64 VALU tile for chunks
+// the wave tiles do not take, the 32x32 one when there are too few tiles to fill the chip.  The other
+// products take the wave tile, 64x128 (each lane's A values serve two B columns) from 768 such tiles
+// on, else 64x64.  Measured (us, 64x64 and 64x128, FP32 operands): 8e7m accumulator, 4096x4096x1024,
+// chunk 4 2801 / 2252, chunk 8 1551 / 1360, chunk 32 925 / 819; 2048x2048x512, 512 tiles, chunk 4 404 /
+// 367, chunk 8 237 / 232, chunk 32 143 / 153; 1537x3001x511, 600 tiles, chunk 8 395 / 517.  Modes other
+// than nearest-even and binary16 formats short of 2^15 (general leaves, 6 to 60 times as long) take
+// 64x64 at every size: 10 bits towards zero, 4096x4096x1024, chunk 8 18503 / 22599, 2048x4096x2048
+// 18650 / 28912.  So do 0-bit accumulators at chunks 2 and 4: 3000x5000x300, chunk 2 879 / 998 (chunk 32
+// 287 / 272).
+int gemm_default_config(const GemmArgs& g) {
+    if (!chunk_fits_wave_tile(g.chunk))
+        return (int64_t)((g.M + 31) / 32) * ((g.N + 63) / 64) >= 1024 ? 3 : 4;
+    if (g.chain >= 0) {
+        const bool directed = g.chunk == 1 && g.chain == kChainMant;
+        const int t = chain_default_tile(g.M, g.N, g.chunk, few_takes(g.M, g.N, g.K, g.ta != 0, g.tb != 0),
+                                         directed);
+        if (!directed || (kShortTile[t] && (int64_t)((g.M + 63) / 64) * ((g.N + 63) / 64) <= kShortMantTiles))
+            return kChainConfigOf[t];
+    }
+    const bool pairs = g.acc_mode == RNE && !g.sum_f16 &&
+                       (g.acc_kind == 1 || g.chunk == 1 || g.chunk >= 8 || g.acc_r < 23);
+    return pairs && (int64_t)((g.M + 63) / 64) * ((g.N + 127) / 128) >= 768 ? kMfma64x128 : kMfma64;
 }
 
 lof_status launch_chain(const GemmArgs& g, int tile, hipStream_t st, const char* what) {
@@ -370,13 +378,6 @@ bool gemm_chunk_fits_mfma(int chunk) { return chunk_fits_mfma(chunk); }
 int gemm_config_bm(int c) { return kConfigs[c].bm; }
 int gemm_config_bn(int c) { return kConfigs[c].bn; }
 
-int resolve_gemm_config(const lof_gemm_desc& d, int config) {
-    if (config >= 0) return config;
-    std::lock_guard<std::mutex> lk(g_tune_mu);
-    auto it = g_tuned.find(tune_key(d));
-    return it != g_tuned.end() ? it->second : default_config(d);
-}
-
 }  // namespace lofamd
 
 using namespace lofamd;
@@ -412,7 +413,7 @@ LOF_API lof_status lof_gemm_f32(const lof_gemm_desc* desc, int32_t config, lof_s
     }
     if (config >= 0 && (config & 0x200)) g.mfma_mode = 1;
     else if (config >= 0 && (config & 0x400)) g.mfma_mode = 2;
-    return launch_gemm(g, resolve_gemm_config(*desc, cfg_bits), (hipStream_t)stream);
+    return launch_gemm(g, cfg_bits >= 0 ? cfg_bits : tuned_or_default(*desc, g), (hipStream_t)stream);
 }
 
 LOF_API int32_t lof_gemm_num_configs(void) { return kNumConfigs; }

@@ -19,7 +19,7 @@ void set_chain(GemmArgs* g, bool conv);
 int chain_default_tile(int64_t M, int64_t N, int chunk, bool few, bool directed);
 lof_status launch_chain(const GemmArgs& g, int tile, hipStream_t st, const char* what);
 lof_status launch_gemm(const GemmArgs& g, int config, hipStream_t st);
-int resolve_gemm_config(const lof_gemm_desc& d, int config);
+int gemm_default_config(const GemmArgs& g);   // the untuned config of lof_gemm_f32
 int gemm_num_configs();
 int gemm_config_bm(int c);
 int gemm_config_bn(int c);

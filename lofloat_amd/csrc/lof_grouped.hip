@@ -449,20 +449,7 @@ lof_status launch_alone(const GroupTask& t, hipStream_t st) {
     case LOF_ITEM_ROUND: return launch_round(t.r, false, t.mode, t.rsrc, st);
     case LOF_ITEM_ROUND_MANT: return launch_round(t.r, true, t.mode, t.rsrc, st);
     case LOF_ITEM_MX: return launch_mx(t.x, t.mode, t.rsrc, st);
-    default: {
-        lof_gemm_desc d{};
-        d.M = t.g.M; d.N = t.g.N; d.K = t.g.K;
-        d.trans_a = t.g.ta; d.trans_b = t.g.tb;
-        d.accum.kind = t.g.acc_kind;
-        d.accum.chunk = t.g.chunk;
-        if (t.g.chain >= 0 && (t.g.chunk > 1 || t.g.chain != kChainMant))
-            return launch_chain(t.g,
-                                chain_default_tile(t.g.M, t.g.N, t.g.chunk,
-                                                   few_takes(t.g.M, t.g.N, t.g.K, t.g.ta != 0, t.g.tb != 0),
-                                                   t.g.chunk == 1 && t.g.chain == kChainMant),
-                                st, "lof_grouped launch");
-        return launch_gemm(t.g, resolve_gemm_config(d, -1), st);
-    }
+    default: return launch_gemm(t.g, gemm_default_config(t.g), st);
     }
 }
 

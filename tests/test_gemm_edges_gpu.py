@@ -31,6 +31,17 @@ def _best_us(run, reps=8):
     return min(times)
 
 
+def _kernels(run):
+    """Names of the device kernels that run() launches, without their arguments."""
+    from torch.profiler import ProfilerActivity, profile
+    run()
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        run()
+        torch.cuda.synchronize()
+    return [e.name.split("(lofamd")[0] for e in prof.events() if "lofamd::" in e.name]
+
+
 def _overflowing(M, N, K, seed):
     """Operands whose binary16 sums pass the format's top binade within a few k."""
     g = np.random.default_rng(seed)
@@ -63,3 +74,23 @@ def test_rows_past_the_matrix_take_no_general_leaf(dev, chunk):
     few = _best_us(lambda: lof.gemm(A[:3], B, acc, config=7))
     full = _best_us(lambda: lof.gemm(A, B, acc, config=7))
     assert few < 0.7 * full, (few, full)
+
+
+@pytest.mark.parametrize("accum, mode, chunk", [
+    (10, 1, 8), (10, 0, 8), (0, 0, 8), (0, 0, 2), (7, 0, 1), (23, 0, 1), (10, 0, 3),
+    ((16, 7, 127, 1, 0, 0), 0, 8), ((16, 7, 127, 1, 0, 0), 1, 1), (HALF, 0, 32),
+    ((14, 10, 15, 1, 0, 0), 0, 1)], ids=str)
+@pytest.mark.parametrize("shape", [(2048, 4096, 8), (600, 500, 40)], ids=str)
+def test_a_plans_own_launches_take_the_calls_kernel(dev, shape, accum, mode, chunk):
+    """A product of a grouped plan that is launched on its own runs on the kernel of its own call."""
+    import lofloat_amd as lof
+    M, N, K = shape
+    A, B = (torch.randn(s, device=dev) for s in ((M, K), (K, N)))
+    acc = lof.AccumSpec(mant_bits=accum, chunk=chunk, mode=mode) if isinstance(accum, int) else \
+        lof.AccumSpec(fmt=_fmt(accum), chunk=chunk, mode=mode)
+    job = lof.GemmJob(A, B, acc)
+    plan = lof.GroupedPlan([job])
+    own = _kernels(lambda: lof.gemm(A, B, acc))
+    assert len(own) == 1
+    assert _kernels(plan.run_separate) == own
+    assert torch.equal(job.out.view(torch.int32), lof.gemm(A, B, acc).view(torch.int32))
