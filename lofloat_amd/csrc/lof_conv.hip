@@ -196,7 +196,7 @@ LOF_API lof_status lof_conv2d_f32(const lof_conv2d_desc* desc, int32_t config,
     if (g.chain >= 0 && (g.chunk > 1 || g.chain != kChainMant)) {
         int t = 1;
         if (cfg < 0) {
-            t = chain_default_tile(c.K, Ncols, g.chunk, false, false);
+            t = chain_default_tile(c.K, Ncols, g.chunk, false, false, false);
             if (t == 4) t = 2;
         }
         return launch_chain(g, t, (hipStream_t)stream, "lof_conv2d_f32 launch");

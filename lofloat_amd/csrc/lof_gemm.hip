@@ -162,9 +162,14 @@ void set_chain(GemmArgs* g, bool conv) {
 // takes 4 k), and 16x16 ties with 64x64 only at 2048x1024 (1024x1024x1024 158 against 249).
 // Accumulators whose chunk-1 leaves are all directed (`directed`) gain up to twelve workgroups a CU:
 // 1000x768x3072 462 against 32x32's 490, 1024x1024x1024 212 against 207.
-int chain_default_tile(int64_t M, int64_t N, int chunk, bool few, bool directed) {
+// Binary16-shaped accumulators with at most 16 rows or columns take 16x16 at any number of tiles at
+// chunks 1 and 4 to 16: once sums pass the top binade, the general leaf runs for each of a lane's
+// outputs, 4 on the 16x64 tile (3x40000x256, us, 16x64 and 16x16: chunk 1 3625 / 936, chunk 4 1080 /
+// 375, chunk 16 292 / 120; ordinary sums, 16x40000x256: chunk 1 53 / 26, chunk 4 47 / 23, chunk 16 25 / 23).
+int chain_default_tile(int64_t M, int64_t N, int chunk, bool few, bool directed, bool half) {
     const int64_t t16 = ((M + 15) / 16) * ((N + 15) / 16), t64 = ((M + 63) / 64) * ((N + 63) / 64);
     if (few && (t16 <= (directed ? 3072 : 768) || (chunk == 2 && t64 < 512))) return 5;
+    if (few && half && chunk != 2 && chunk <= 16 && (M <= 16 || N <= 16)) return 5;
     if (M <= 16) return 3;
     if (N <= 16) return 4;
     return t64 >= 768 ? 1 : 2;
@@ -187,7 +192,7 @@ int gemm_default_config(const GemmArgs& g) {
     if (g.chain >= 0) {
         const bool directed = g.chunk == 1 && g.chain == kChainMant;
         const int t = chain_default_tile(g.M, g.N, g.chunk, few_takes(g.M, g.N, g.K, g.ta != 0, g.tb != 0),
-                                         directed);
+                                         directed, g.chain == kChainHalf);
         if (!directed || (kShortTile[t] && (int64_t)((g.M + 63) / 64) * ((g.N + 63) / 64) <= kShortMantTiles))
             return kChainConfigOf[t];
     }

@@ -15,8 +15,8 @@ void set_fast_path(GemmArgs* g, bool on, int m);
 // through ldb.  prepare_gemm calls it for a stored B.
 void set_chain(GemmArgs* g, bool conv);
 // Tile of the chunk-sum kernels for an M x N product, and its launch.  few: the 16x16 tile takes it;
-// directed: a mantissa-only accumulator at chunk 1, 10 and 23 bits aside.
-int chain_default_tile(int64_t M, int64_t N, int chunk, bool few, bool directed);
+// directed: a mantissa-only accumulator at chunk 1, 10 and 23 bits aside; half: a binary16-shaped one.
+int chain_default_tile(int64_t M, int64_t N, int chunk, bool few, bool directed, bool half);
 lof_status launch_chain(const GemmArgs& g, int tile, hipStream_t st, const char* what);
 lof_status launch_gemm(const GemmArgs& g, int config, hipStream_t st);
 int gemm_default_config(const GemmArgs& g);   // the untuned config of lof_gemm_f32

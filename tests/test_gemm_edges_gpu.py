@@ -76,6 +76,22 @@ def test_rows_past_the_matrix_take_no_general_leaf(dev, chunk):
     assert few < 0.7 * full, (few, full)
 
 
+@pytest.mark.parametrize("chunk", [1, 4, 8, 16])
+@pytest.mark.parametrize("shape", [(3, 24000, 128), (24000, 16, 128)], ids=str)
+def test_few_rows_that_overflow(dev, shape, chunk):
+    """Binary16 sums past the top binade with few rows or columns: one general leaf a lane and k (the
+    16x16 tile), where the 16x64 and 64x16 tiles take up to four (measured 1.9 to 3.2 times as long)."""
+    import lofloat_amd as lof
+    M, N, K = shape
+    A, B = (torch.from_numpy(v).to(dev) for v in _overflowing(M, N, K, 2))
+    acc = lof.AccumSpec(fmt=_fmt(HALF), chunk=chunk)
+    by_default = _best_us(lambda: lof.gemm(A, B, acc))
+    wide = _best_us(lambda: lof.gemm(A, B, acc, config=10 if M <= 16 else 11))
+    assert by_default < 0.8 * wide, (by_default, wide)
+    assert torch.equal(lof.gemm(A, B, acc).view(torch.int32),
+                       lof.gemm(A, B, acc, config=7).view(torch.int32))
+
+
 @pytest.mark.parametrize("accum, mode, chunk", [
     (10, 1, 8), (10, 0, 8), (0, 0, 8), (0, 0, 2), (7, 0, 1), (23, 0, 1), (10, 0, 3),
     ((16, 7, 127, 1, 0, 0), 0, 8), ((16, 7, 127, 1, 0, 0), 1, 1), (HALF, 0, 32),
