@@ -206,7 +206,10 @@ LOF_API int32_t lof_gemm_num_configs(void);
  * in {1, 2, 4, 8, 16, 32}; chunk 1 runs on VALU), else 0.  No reference counterpart: the
  * reference has one kernel. */
 LOF_API int32_t lof_gemm_config_valid(int32_t config, int32_t chunk);
-/* Writes a short "BMxBN/TMxTN" style name; returns LOF_ERR_INVALID_ARGUMENT if out of range. */
+/* Writes a short "BMxBN/TMxTN" style name of the tile (mfma21: a wave tile of 128 x 64); returns
+ * LOF_ERR_INVALID_ARGUMENT if out of range.  The short tiles mfma32x32, mfma16x64, mfma64x16 and
+ * mfma16x16 exist for round-to-nearest-even mantissa-only accumulators of 1 to 23 bits and
+ * binary16-shaped formats; other products, and the first three at chunk 2, run 64 x 64 instead. */
 LOF_API lof_status lof_gemm_config_name(int32_t config, char* buf, int32_t buflen);
 
 /* Autotuner: times the candidate tile configs on this problem -- the wave tiles for chunks

@@ -193,7 +193,7 @@ LOF_API lof_status lof_conv2d_f32(const lof_conv2d_desc* desc, int32_t config,
         cv.sdm = 1;
         cv.sdpq = c.K;
     }
-    if (g.chain >= 0 && (g.chunk > 1 || g.chain != kChainMant)) {
+    if (g.chain >= 0 && (g.chunk > 1 || g.chain != kChainMant) && cfg != kCfgMfma21) {   // no 128x64 there
         int t = 1;
         if (cfg < 0) {
             t = chain_default_tile(c.K, Ncols, g.chunk, false, false, false);

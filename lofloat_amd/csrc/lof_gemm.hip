@@ -73,7 +73,7 @@ const GemmConfig kConfigs[] = {
     LOF_GEMM_SHORT_CFG(16, 16),
 };
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
-constexpr int kFirstMfma = 5, kMfma64 = 7, kMfma64x128 = 8, kFirstShort = 9;
+constexpr int kFirstMfma = 5, kMfma128 = 5, kMfma128x64 = 6, kMfma64 = 7, kMfma64x128 = 8, kFirstShort = 9;
 constexpr bool kShortTile[kChainTiles] = {false, false, true, true, true, true};
 // 64x64 tiles up to which a directed accumulator takes the short tiles.  Measured (us, 7 bits, the wave
 // tile and 32x32; e4m3 / FP32 operands): 2048x1024x1024, 512 tiles, 374 / 507 against 362 / 364;
@@ -92,11 +92,13 @@ bool config_valid(int config, int chunk) {
            (!is_mfma(config) || chunk_fits_wave_tile(chunk));
 }
 
-// Whether the chunk-sum kernels run this product on a wave-tile config.  At chunk 1 the mantissa-
+// Whether the chunk-sum kernels run this product on a wave-tile config: where they have the tile that
+// the config names (not 128x64 and 64x128, nor 128x128 at chunk 1).  At chunk 1 the mantissa-
 // only accumulators of 1 to 22 bits, 10 aside, keep the wave tile's exact-sum and held leaves (a third to
 // an eighth of the directed leaf's instructions) and take the short tiles only.
 bool chain_takes(const GemmArgs& g, int config) {
-    return g.chain >= 0 && (g.chunk > 1 || g.chain != kChainMant || config >= kFirstShort);
+    if (g.chain < 0 || config == kMfma128x64 || config == kMfma64x128) return false;
+    return g.chunk > 1 ? true : g.chain != kChainMant ? config != kMfma128 : config >= kFirstShort;
 }
 
 GemmKernel pick_kernel(const GemmConfig& c, const GemmArgs& g) {
@@ -209,7 +211,7 @@ lof_status launch_chain(const GemmArgs& g, int tile, hipStream_t st, const char*
     const int l2 = 31 - __builtin_clz((unsigned)g.chunk);
     if (tile == 5 && !few_takes(g.M, g.N, g.K, g.ta != 0, g.tb != 0)) tile = 2;
     ChainKernel k = g.cv.conv ? t.conv[tile][l2] : t.gemm[tile][l2];
-    if (!k) {   // chunk 2 on a 16-row block (its MFMA takes 4 k), chunk 1 on the widest tile
+    if (!k) {   // chunk 2 on a 16-row block (its MFMA takes 4 k)
         tile = 1;
         k = g.cv.conv ? t.conv[tile][l2] : t.gemm[tile][l2];
     }
@@ -469,8 +471,8 @@ LOF_API lof_status lof_gemm_autotune(const lof_gemm_desc* desc, int32_t iters,
     for (int c = 0; c < kNumConfigs && s == LOF_OK; ++c) {
         if (!config_valid(c, g.chunk) || is_mfma(c) != wave) continue;
         if (c >= kFirstShort && !chain_takes(g, c)) continue;   // would time mfma11 again
-        if ((c == 6 || c == 8) && chain_takes(g, c)) continue;
-        if (c == 5 && g.chunk == 1 && chain_takes(g, c)) continue;
+        // the wave tile's leaves are no match where the chunk-sum kernels run
+        if (c < kFirstShort && chain_takes(g, kMfma64) && !chain_takes(g, c)) continue;
         s = launch_gemm(g, c, st);  // warm-up
         if (s != LOF_OK) break;
         (void)hipEventRecord(e0, st);

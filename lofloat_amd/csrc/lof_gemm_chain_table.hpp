@@ -102,8 +102,8 @@ extern const ChainTable kChainTableMant, kChainTableMant10, kChainTableMant23, k
 // The dimensions of tile t.
 struct ChainDims { int bm, bn; };
 constexpr ChainDims kChainDims[kChainTiles] = {{128, 128}, {64, 64}, {32, 32}, {16, 64}, {64, 16}, {16, 16}};
-// GEMM configs 5.. (lof_gemm.hip) and the tile each runs on here, and back
-constexpr int kChainTileOf[8] = {0, 1, 1, 1, 2, 3, 4, 5};
+// GEMM configs 5.. (lof_gemm.hip) and the tile each runs on here (-1: 128x64 and 64x128, not here), and back
+constexpr int kChainTileOf[8] = {0, -1, 1, -1, 2, 3, 4, 5};
 constexpr int kChainConfigOf[kChainTiles] = {5, 7, 9, 10, 11, 12};
 
 }  // namespace lofamd

@@ -110,3 +110,44 @@ def test_a_plans_own_launches_take_the_calls_kernel(dev, shape, accum, mode, chu
     assert len(own) == 1
     assert _kernels(plan.run_separate) == own
     assert torch.equal(job.out.view(torch.int32), lof.gemm(A, B, acc).view(torch.int32))
+
+
+WAVE = {5: "k_gemm_mfma<2, 2,", 6: "k_gemm_mfma<2, 1,", 7: "k_gemm_mfma<1, 1,", 8: "k_gemm_mfma<1, 2,"}
+CHAIN = {5: "ChainTile<32, 2, 2, 2, 2,", 7: "ChainTile<32, 2, 2, 1, 1,", 9: "ChainTile<16, 2, 2,",
+         10: "ChainTile<16, 1, 4,", 11: "ChainTile<16, 4, 1,", 12: "k_gemm_few<"}
+
+
+@pytest.mark.parametrize("accum", [7, 10, 23, HALF, (16, 7, 127, 1, 0, 0)], ids=str)
+@pytest.mark.parametrize("chunk", [1, 4, 32])
+def test_a_config_runs_the_tile_it_names(dev, accum, chunk):
+    import lofloat_amd as lof
+    A, B = torch.randn(150, 70, device=dev), torch.randn(70, 140, device=dev)
+    acc = lof.AccumSpec(mant_bits=accum, chunk=chunk) if isinstance(accum, int) else \
+        lof.AccumSpec(fmt=_fmt(accum), chunk=chunk)
+    ref = lof.gemm(A, B, acc).view(torch.int32)
+    for cfg in range(5, 13):
+        if accum == (16, 7, 127, 1, 0, 0):        # no chunk-sum kernel: the short tiles are 64x64
+            want = WAVE.get(cfg, WAVE[7])
+        elif chunk == 1 and accum == 7:
+            want = WAVE.get(cfg) or CHAIN[cfg]
+        elif chunk == 1 and cfg == 5:
+            want = WAVE[5]
+        else:
+            want = CHAIN.get(cfg) or WAVE[cfg]
+        (name,) = _kernels(lambda: lof.gemm(A, B, acc, config=cfg))
+        assert want in name, (cfg, name)
+        assert torch.equal(lof.gemm(A, B, acc, config=cfg).view(torch.int32), ref), cfg
+
+
+@pytest.mark.parametrize("accum", [10, 23, HALF], ids=str)
+@pytest.mark.parametrize("chunk", [1, 8])
+def test_a_convolutions_config_runs_the_tile_it_names(dev, accum, chunk):
+    import lofloat_amd as lof
+    x, w = torch.randn(2, 5, 12, 12, device=dev), torch.randn(70, 5, 3, 3, device=dev)
+    acc = lof.AccumSpec(mant_bits=accum, chunk=chunk) if isinstance(accum, int) else \
+        lof.AccumSpec(fmt=_fmt(accum), chunk=chunk)
+    ref = lof.conv2d(x, w, acc, padding=1).view(torch.int32)
+    for cfg, want in ((6, "k_conv_mfma<2, 1,"), (7, "ChainTile<32, 2, 2, 1, 1,")):
+        (name,) = _kernels(lambda: lof.conv2d(x, w, acc, padding=1, config=cfg))
+        assert want in name, (cfg, name)
+        assert torch.equal(lof.conv2d(x, w, acc, padding=1, config=cfg).view(torch.int32), ref), cfg
