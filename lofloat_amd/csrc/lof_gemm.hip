@@ -73,7 +73,7 @@ const GemmConfig kConfigs[] = {
     LOF_GEMM_SHORT_CFG(16, 16),
 };
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
-constexpr int kFirstMfma = 5, kMfma128 = 5, kMfma128x64 = 6, kMfma64 = 7, kMfma64x128 = 8, kFirstShort = 9;
+constexpr int kFirstMfma = 5, kMfma128 = 5, kMfma128x64 = 6, kMfma64 = 7, kMfma64x128 = 8, kFirstShort = 9, kShort16 = 12;
 constexpr bool kShortTile[kChainTiles] = {false, false, true, true, true, true};
 // 64x64 tiles up to which a directed accumulator takes the short tiles.  Measured (us, 7 bits, the wave
 // tile and 32x32; e4m3 / FP32 operands): 2048x1024x1024, 512 tiles, 374 / 507 against 362 / 364;
@@ -97,6 +97,7 @@ bool config_valid(int config, int chunk) {
 // only accumulators of 1 to 22 bits, 10 aside, keep the wave tile's exact-sum and held leaves (a third to
 // an eighth of the directed leaf's instructions) and take the short tiles only.
 bool chain_takes(const GemmArgs& g, int config) {
+    if (g.chain >= 0 && chain_rows_far_apart(g, g.cv.conv != 0)) return config == kShort16;
     if (g.chain < 0 || config == kMfma128x64 || config == kMfma64x128) return false;
     return g.chunk > 1 ? true : g.chain != kChainMant ? config != kMfma128 : config >= kFirstShort;
 }
@@ -137,8 +138,13 @@ int tuned_or_default(const lof_gemm_desc& d, const GemmArgs& g) {
 
 void set_chain(GemmArgs* g, bool conv) {
     g->chain = -1;
-    if (!chunk_fits_wave_tile(g->chunk) || g->acc_mode != RNE || g->lda > kChainMaxLd ||
-        (!conv && g->ldb > kChainMaxLd))
+    if (!chunk_fits_wave_tile(g->chunk) || g->acc_mode != RNE) return;
+    // Rows further apart run on the wave tile, but for the accumulators whose chunk sums have no fast
+    // leaf there (20 bits and more), which the 16x16 tile takes.  1024x1024x64, rows 2^25 + 8 floats
+    // apart, chunk 8, 23 bits: 174 -> 45 us; 400x300x300 784 -> 20.
+    if (chain_rows_far_apart(*g, conv) &&
+        (conv || g->acc_kind != 0 || g->range_f != 0u || g->chunk < 8 ||
+         !few_takes(g->M, g->N, g->K, g->ta != 0, g->tb != 0)))
         return;
     if (g->sum_f16) {
         // chunk 1 holds the accumulator as binary16, whose top binade the format must reach
@@ -191,6 +197,7 @@ int chain_default_tile(int64_t M, int64_t N, int chunk, bool few, bool directed,
 int gemm_default_config(const GemmArgs& g) {
     if (!chunk_fits_wave_tile(g.chunk))
         return (int64_t)((g.M + 31) / 32) * ((g.N + 63) / 64) >= 1024 ? 3 : 4;
+    if (g.chain >= 0 && chain_rows_far_apart(g, g.cv.conv != 0)) return kShort16;
     if (g.chain >= 0) {
         const bool directed = g.chunk == 1 && g.chain == kChainMant;
         const int t = chain_default_tile(g.M, g.N, g.chunk, few_takes(g.M, g.N, g.K, g.ta != 0, g.tb != 0),

@@ -99,6 +99,11 @@ constexpr ChainKernel chain_kernel() {
 
 extern const ChainTable kChainTableMant, kChainTableMant10, kChainTableMant23, kChainTableHalf;
 
+// Leading dimensions past those of the tiles, 16x16 aside, which takes any (`conv`: B is gathered).
+inline bool chain_rows_far_apart(const GemmArgs& g, bool conv) {
+    return g.lda > kChainMaxLd || (!conv && g.ldb > kChainMaxLd);
+}
+
 // The dimensions of tile t.
 struct ChainDims { int bm, bn; };
 constexpr ChainDims kChainDims[kChainTiles] = {{128, 128}, {64, 64}, {32, 32}, {16, 64}, {64, 16}, {16, 16}};

@@ -121,7 +121,7 @@ inline bool few_takes(int64_t M, int64_t N, int64_t K, bool ta, bool tb) {
     return K >= 4 && (!ta || M >= 4) && (tb || N >= 4);
 }
 
-// One 16 x 16 output tile; g.lda, g.ldb <= kChainMaxLd, few_takes.
+// One 16 x 16 output tile (few_takes), for any leading dimensions.
 template <int CHUNK, int KIND>
 __device__ __forceinline__ void gemm_tile_few(const GemmArgs& g, int tile_m, int tile_n, int tid, float* smem) {
     constexpr int BK = kFewK, ROW = kFewRow;

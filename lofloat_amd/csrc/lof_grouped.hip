@@ -307,7 +307,7 @@ namespace {
 
 bool grouped_mfma_chunk(int chunk) { return chunk == 8 || chunk == 16 || chunk == 32; }
 bool grouped_on_chain(const GemmArgs& g) {
-    return g.chain >= 0 && (g.chunk == 1 || grouped_mfma_chunk(g.chunk));
+    return g.chain >= 0 && (g.chunk == 1 || grouped_mfma_chunk(g.chunk)) && !chain_rows_far_apart(g, false);
 }
 
 lof_status build_task(const lof_group_item& it, const GroupedConfig& cfg, GroupTask* t,

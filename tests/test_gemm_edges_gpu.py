@@ -151,3 +151,45 @@ def test_a_convolutions_config_runs_the_tile_it_names(dev, accum, chunk):
         (name,) = _kernels(lambda: lof.conv2d(x, w, acc, padding=1, config=cfg))
         assert want in name, (cfg, name)
         assert torch.equal(lof.conv2d(x, w, acc, padding=1, config=cfg).view(torch.int32), ref), cfg
+
+
+def _wide(x, ld, dev):
+    """x with rows ld floats apart; what lies between them is never read."""
+    buf = torch.empty((x.shape[0] - 1) * ld + x.shape[1], device=dev)
+    v = buf.as_strided(x.shape, (ld, 1))
+    v.copy_(torch.from_numpy(x))
+    return v
+
+
+@pytest.mark.parametrize("ld", [(1 << 22) + 1, (1 << 25) + 3])
+@pytest.mark.parametrize("ta, tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_leading_dimensions(dev, ld, ta, tb):
+    """Rows 16 MiB and 128 MiB apart (past 2^25 floats, offsets within a tile pass 2^32), against the
+    oracle.  Chunk sums of accumulators of 20 bits and more run on the chunk-sum kernels at any distance,
+    every kind up to 2^25."""
+    import lofloat_amd as lof
+    M, N, K = 130, 131, 129
+    g = np.random.default_rng(3)
+    A, B = (g.uniform(-1, 1, s).astype(np.float32) for s in ((M, K), (K, N)))
+    Aw, Bw = (_wide(np.ascontiguousarray(x.T) if t else x, ld, dev) for x, t in ((A, ta), (B, tb)))
+    Aw, Bw = (x.t() if t else x for x, t in ((Aw, ta), (Bw, tb)))
+    Ac, Bc = (torch.from_numpy(np.ascontiguousarray(x.T)).to(dev).t() if t else
+              torch.from_numpy(x).to(dev) for x, t in ((A, ta), (B, tb)))
+    for kind, chunk in ((23, 32), (22, 8), (20, 16), (23, 1), (10, 1), (7, 4), (HALF, 1), (HALF, 8)):
+        acc = lof.AccumSpec(mant_bits=kind, chunk=chunk) if isinstance(kind, int) else \
+            lof.AccumSpec(fmt=_fmt(kind), chunk=chunk)
+        oacc = oracle.accum_mant(kind, chunk) if isinstance(kind, int) else \
+            oracle.accum_fmt(kind, chunk)
+        ref = oracle.gemm(A, B, oacc)
+        for cfg in (-1, *range(5, 13)):
+            y = lof.gemm(Aw, Bw, acc, config=cfg).cpu().numpy()
+            assert_bits(y, ref, f"ld {ld} {kind} chunk {chunk} config {cfg}")
+        for cfg in (-1, 4, 8):
+            job = lof.GemmJob(Aw, Bw, acc)
+            lof.GroupedPlan([job], config=cfg).run()
+            assert_bits(job.out.cpu().numpy(), ref, f"grouped ld {ld} {kind} chunk {chunk} {cfg}")
+        (name,) = _kernels(lambda: lof.gemm(Aw, Bw, acc))
+        if ld <= 1 << 25:
+            assert [name] == _kernels(lambda: lof.gemm(Ac, Bc, acc))
+        else:
+            assert ("k_gemm_few" if kind in (20, 22, 23) and chunk > 1 else "k_gemm_mfma") in name, kind
