@@ -139,12 +139,14 @@ int tuned_or_default(const lof_gemm_desc& d, const GemmArgs& g) {
 void set_chain(GemmArgs* g, bool conv) {
     g->chain = -1;
     if (!chunk_fits_wave_tile(g->chunk) || g->acc_mode != RNE) return;
+    // too many tiles for one dimension of a grid: the wave tile's has two (1 x 2^30 outputs)
+    if (chain_tiles(g->M, g->N, 1) > kChainMaxTiles) return;
     // Rows further apart run on the wave tile, but for the accumulators whose chunk sums have no fast
     // leaf there (20 bits and more), which the 16x16 tile takes.  1024x1024x64, rows 2^25 + 8 floats
     // apart, chunk 8, 23 bits: 174 -> 45 us; 400x300x300 784 -> 20.
     if (chain_rows_far_apart(*g, conv) &&
         (conv || g->acc_kind != 0 || g->range_f != 0u || g->chunk < 8 ||
-         !few_takes(g->M, g->N, g->K, g->ta != 0, g->tb != 0)))
+         !few_takes(g->M, g->N, g->K, g->ta != 0, g->tb != 0) || chain_tiles(g->M, g->N, 5) > kChainMaxTiles))
         return;
     if (g->sum_f16) {
         // chunk 1 holds the accumulator as binary16, whose top binade the format must reach
@@ -177,7 +179,7 @@ void set_chain(GemmArgs* g, bool conv) {
 int chain_default_tile(int64_t M, int64_t N, int chunk, bool few, bool directed, bool half) {
     const int64_t t16 = ((M + 15) / 16) * ((N + 15) / 16), t64 = ((M + 63) / 64) * ((N + 63) / 64);
     if (few && (t16 <= (directed ? 3072 : 768) || (chunk == 2 && t64 < 512))) return 5;
-    if (few && half && chunk != 2 && chunk <= 16 && (M <= 16 || N <= 16)) return 5;
+    if (few && half && chunk != 2 && chunk <= 16 && (M <= 16 || N <= 16) && t16 <= kChainMaxTiles) return 5;
     if (M <= 16) return 3;
     if (N <= 16) return 4;
     return t64 >= 768 ? 1 : 2;
@@ -207,7 +209,8 @@ int gemm_default_config(const GemmArgs& g) {
     }
     const bool pairs = g.acc_mode == RNE && !g.sum_f16 &&
                        (g.acc_kind == 1 || g.chunk == 1 || g.chunk >= 8 || g.acc_r < 23);
-    return pairs && (int64_t)((g.M + 63) / 64) * ((g.N + 127) / 128) >= 768 ? kMfma64x128 : kMfma64;
+    const bool long_rows = (g.N + (int64_t)63) / 64 > kChainMaxTiles;   // past what a grid of 64 columns holds
+    return (pairs && (int64_t)((g.M + 63) / 64) * ((g.N + 127) / 128) >= 768) || long_rows ? kMfma64x128 : kMfma64;
 }
 
 lof_status launch_chain(const GemmArgs& g, int tile, hipStream_t st, const char* what) {
@@ -224,7 +227,7 @@ lof_status launch_chain(const GemmArgs& g, int tile, hipStream_t st, const char*
     }
     const ChainDims& d = kChainDims[tile];
     const int64_t tm = (g.M + d.bm - 1) / d.bm, tn = (g.N + d.bn - 1) / d.bn;
-    if (tm * tn > 0x7FFFFFFF) return set_error(LOF_ERR_UNSUPPORTED, "%s: output too large", what);
+    if (tm * tn > kChainMaxTiles) return set_error(LOF_ERR_UNSUPPORTED, "%s: output too large", what);
     hipLaunchKernelGGL(k, dim3((unsigned)(tm * tn)), dim3(256), 0, st, g, (unsigned)tm, (unsigned)tn);
     return check_hip(hipGetLastError(), what);
 }

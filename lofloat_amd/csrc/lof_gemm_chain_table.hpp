@@ -107,6 +107,11 @@ inline bool chain_rows_far_apart(const GemmArgs& g, bool conv) {
 // The dimensions of tile t.
 struct ChainDims { int bm, bn; };
 constexpr ChainDims kChainDims[kChainTiles] = {{128, 128}, {64, 64}, {32, 32}, {16, 64}, {64, 16}, {16, 16}};
+// Workgroups of one launch: HIP takes fewer than 2^32 threads in a dimension of the grid.
+constexpr int64_t kChainMaxTiles = (1 << 24) - 1;
+inline int64_t chain_tiles(int64_t M, int64_t N, int t) {
+    return ((M + kChainDims[t].bm - 1) / kChainDims[t].bm) * ((N + kChainDims[t].bn - 1) / kChainDims[t].bn);
+}
 // GEMM configs 5.. (lof_gemm.hip) and the tile each runs on here (-1: 128x64 and 64x128, not here), and back
 constexpr int kChainTileOf[8] = {0, -1, 1, -1, 2, 3, 4, 5};
 constexpr int kChainConfigOf[kChainTiles] = {5, 7, 9, 10, 11, 12};

@@ -193,3 +193,22 @@ def test_leading_dimensions(dev, ld, ta, tb):
             assert [name] == _kernels(lambda: lof.gemm(Ac, Bc, acc))
         else:
             assert ("k_gemm_few" if kind in (20, 22, 23) and chunk > 1 else "k_gemm_mfma") in name, kind
+
+
+@pytest.mark.parametrize("kind, chunk", [(10, 1), (23, 8), (HALF, 1), (HALF, 32)], ids=str)
+@pytest.mark.parametrize("N", [1 << 30, (1 << 28) + 5])
+def test_long_rows(dev, kind, chunk, N):
+    """One row of as many outputs as 2^24 tiles of 64, or of 16, columns: each is its operand, rounded."""
+    import lofloat_amd as lof
+    A = torch.ones(1, 1, device=dev)
+    B = torch.empty(1, N, device=dev)
+    B.copy_(torch.rand(1, 1 << 20, device=dev).repeat(1, -(-N // (1 << 20)))[:, :N])
+    acc = lof.AccumSpec(mant_bits=kind, chunk=chunk) if isinstance(kind, int) else \
+        lof.AccumSpec(fmt=_fmt(kind), chunk=chunk)
+    y = lof.gemm(A, B, acc)
+    ref = lof.virtual_round(B, kind if isinstance(kind, int) else _fmt(kind))
+    assert torch.equal(y.view(torch.int32), ref.view(torch.int32))
+    if kind == 10:
+        y = lof.gemm(A, B, lof.AccumSpec(mant_bits=10, chunk=1, mode=1))
+        ref = lof.virtual_round(B, 10, 1)
+        assert torch.equal(y.view(torch.int32), ref.view(torch.int32))
