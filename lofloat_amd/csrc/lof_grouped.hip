@@ -367,21 +367,23 @@ lof_status free_plan(lof_grouped* p) {
 }
 
 
-// The config asked for, else the tuned one, else the chunk-sum kernels' tile unless a GEMM of
-// chunk 8 to 32 has an accumulator they do not take (the wave tile then runs its chunk sums on MFMA;
-// here it would take the VALU tile).  An item that cannot be prepared is reported by build_task.
+// The config asked for, else the tuned one, else the chunk-sum kernels' tile -- but this one, tuned or
+// not, only where they take the accumulator of every GEMM of chunk 8 to 32: the others would run on
+// its VALU tile, where the wave tile has their chunk sums on MFMA (8e7m accumulator, chunk 32, 16 of
+// 512^3, us: 497 and 173).  An item that cannot be prepared is reported by build_task.
 int resolve_gconfig(int config, const lof_group_item* items, int count) {
     if (config >= 0) return config;
     {
         std::lock_guard<std::mutex> lk(g_gmu);
-        if (g_default_gconfig >= 0) return g_default_gconfig;
+        config = g_default_gconfig >= 0 ? g_default_gconfig : kChainGConfig;
     }
+    if (!kGConfigs[config].chain) return config;
     for (int i = 0; i < count; ++i) {
         if (items[i].kind != LOF_ITEM_GEMM || !grouped_mfma_chunk(items[i].gemm.accum.chunk)) continue;
         GemmArgs g;
         if (prepare_gemm(&items[i].gemm, &g) == LOF_OK && !grouped_on_chain(g)) return kWaveGConfig;
     }
-    return kChainGConfig;
+    return config;
 }
 
 // Validates every item and lays the jobs out in queue order: GEMMs first, largest first,
