@@ -7,6 +7,7 @@ checker validation (LoPy_bind.cpp:45-68).
 """
 from __future__ import annotations
 
+import copyreg
 import enum
 
 from . import _lib
@@ -111,9 +112,12 @@ class FloatFormatDescriptor:
                                       int(self._signedness))
             return self._c_fmt
 
-    def __getstate__(self):   # without the C struct, which is rebuilt
-        return None, {n: getattr(self, n) for n in self.__slots__
-                      if n not in ("_c_fmt", "__weakref__")}
+    def __getstate__(self):
+        """As the default's (a subclass's own attributes with it), without the C struct, which is
+        rebuilt."""
+        slots = {n: getattr(self, n) for n in copyreg._slotnames(type(self))
+                 if n != "_c_fmt" and hasattr(self, n)}
+        return getattr(self, "__dict__", None), slots
 
     def as_tuple(self) -> tuple:
         return (self._total_bits, self._mantissa_bits, self._bias, int(self._inf_behavior),
