@@ -103,7 +103,11 @@ class FloatFormatDescriptor:
     is_nan_checker = property(lambda self: self._is_nan_checker)
 
     def c_format(self) -> _lib.Format:
-        """The C struct of these fields (read-only, built once; callers copy it)."""
+        """The C struct of these fields, the caller's own."""
+        return _lib.Format.from_buffer_copy(self._c_struct())
+
+    def _c_struct(self) -> _lib.Format:
+        """The same, built once and shared: for calls that only read it or copy it."""
         try:
             return self._c_fmt
         except AttributeError:

@@ -64,7 +64,7 @@ class RoundJob:
         if mant:
             it.mant_bits = int(self.params)
         else:
-            it.fmt = self.params.c_format()
+            it.fmt = self.params._c_struct()
         it.spec = _lib.RoundSpec(int(self.mode), 0, int(self.stoch_len))
         it.scale = float(self.scale)
         it.rand_bits = self.rand_bits.data_ptr() if self.rand_bits is not None else None
@@ -100,8 +100,8 @@ class MXJob:
         it.in_ = self.input.data_ptr()
         it.out = self.out.data_ptr()
         it.n = self.input.numel()
-        it.fmt = self.element_format.c_format()
-        it.scale_fmt = self.scale_format.c_format()
+        it.fmt = self.element_format._c_struct()
+        it.scale_fmt = self.scale_format._c_struct()
         it.block_size = int(self.block_size)
         it.spec = _lib.RoundSpec(int(self.mode), 0, int(self.stoch_len))
         it.scale_mode = int(self.scale_mode)

@@ -131,7 +131,7 @@ def virtual_round(input: torch.Tensor, params, round_mode=RoundingMode.RoundToNe
     with _on_device(x):
         if isinstance(params, FloatFormatDescriptor):
             st = _lib.lib.lof_virtual_round_f32(
-                x.data_ptr(), y.data_ptr(), x.numel(), ctypes.byref(params.c_format()), spec, sc,
+                x.data_ptr(), y.data_ptr(), x.numel(), ctypes.byref(params._c_struct()), spec, sc,
                 bptr, s, _stream(x))
         elif isinstance(params, int) and not isinstance(params, bool):
             st = _lib.lib.lof_virtual_round_mant_f32(
@@ -162,7 +162,7 @@ def virtual_mx_round(input: torch.Tensor, block_size: int, element_format: Float
         raise ValueError("virtual_mx_round: out must be a contiguous float32 tensor")
     mode = _mode(round_mode)
     bptr, keep = _bits_ptr(rand_bits, x, "virtual_mx_round")
-    ef, sf = element_format.c_format(), scale_format.c_format()
+    ef, sf = element_format._c_struct(), scale_format._c_struct()
     with _on_device(x):
         st = _lib.lib.lof_virtual_mx_round_f32(
             x.data_ptr(), y.data_ptr(), x.numel(),
@@ -205,7 +205,7 @@ class AccumSpec:
         spec = _lib.RoundSpec(int(self.mode), 0, 0)
         if self.fmt is None:
             return _lib.Accum(0, int(self.mant_bits), _NO_FORMAT, spec, int(self.chunk))
-        return _lib.Accum(1, 0, self.fmt.c_format(), spec, int(self.chunk))
+        return _lib.Accum(1, 0, self.fmt._c_struct(), spec, int(self.chunk))
 
 
 def _mat_view(t: torch.Tensor, what: str):

@@ -41,7 +41,7 @@ def pack_format(params: FloatFormatDescriptor, unsigned_behavior: int = 0) -> _l
     1 NegtoNaN)."""
     if not 1 <= params.total_bits <= 16:
         raise NotImplementedError(f"pack codec: bitwidth {params.total_bits} outside [1, 16]")
-    return _lib.PackFormat(params.c_format(), int(unsigned_behavior),
+    return _lib.PackFormat(params._c_struct(), int(unsigned_behavior),
                            _checker(params.is_inf_checker, "Inf"),
                            _checker(params.is_nan_checker, "NaN"))
 

@@ -1,4 +1,4 @@
-"""Format descriptors as objects: copies and pickles."""
+"""Format descriptors as objects: copies, pickles and their C struct."""
 import copy
 import pickle
 
@@ -31,3 +31,10 @@ def test_copies_keep_a_subclasss_attributes(clone, used):
     assert type(g) is Named and g.as_tuple() == f.as_tuple()
     assert (g.family, g.note) == ("e4m3", "weights")
     assert bytes(g.c_format()) == bytes(f.c_format())
+
+
+def test_a_changed_c_struct_changes_no_format():
+    f = _named()
+    for c in (f.c_format(), lof.AccumSpec(fmt=f).c_accum().fmt):
+        c.bias = 3
+    assert f.bias == f.c_format().bias == lof.AccumSpec(fmt=f).c_accum().fmt.bias == 7
