@@ -178,14 +178,6 @@ def _lof_gemm_2d(A, B, accum_mant_bits, gemm_round_mode, stochastic_rounding_bit
     return out.reshape(*batch, M, N)
 
 
-def _alpha(scale_a: float, scale_b: float) -> float:
-    if scale_a == 1.0 and scale_b == 1.0:
-        return 1.0
-    import numpy as np
-    denom = np.float32(scale_a) * np.float32(scale_b)
-    return 1.0 if denom == 0 else float(np.float32(1.0) / denom)
-
-
 class LinearGradSpec:
     """How LoF_Linear's backward rounds grad_out before the dgrad / wgrad GEMMs."""
 
@@ -392,7 +384,7 @@ class LoF_Linear(_LoFLayer):
         x_q = STERound.apply(x, self._act_fid, self._round_mode_int, self.act_scale_factor)
         w_q = STERound.apply(self.weight, self._weight_fid, self._round_mode_int,
                              self.w_scale_factor)
-        return x_q, w_q, _alpha(self.act_scale_factor, self.w_scale_factor)
+        return x_q, w_q, ops._alpha(self.act_scale_factor, self.w_scale_factor)
 
     def forward(self, x):
         x_q, w_q, alpha = self.quantized_operands(x)
@@ -544,7 +536,7 @@ class LoF_Conv2d(_LoFLayer):
             denom = float(self.w_scale_factor) * float(self.act_scale_factor)
             alpha = 1.0 if denom == 0.0 else float(np.float32(1.0 / denom))
         else:                           # lof_gemm's run_scaled, in float
-            alpha = _alpha(self.w_scale_factor, self.act_scale_factor)
+            alpha = ops._alpha(self.w_scale_factor, self.act_scale_factor)
         kw = dict(stride=self.stride, padding=self.padding, dilation=self.dilation, alpha=alpha)
         if self.groups == 1:
             out = ops.conv2d(x_q.detach(), w_q.detach(), spec, **kw)

@@ -127,7 +127,8 @@ def virtual_round(input: torch.Tensor, params, round_mode=RoundingMode.RoundToNe
     bptr, keep = _bits_ptr(rand_bits, x, "virtual_round")
     spec = _lib.RoundSpec(mode, 0, int(stoch_len))
     s = _seed_for(mode, seed)
-    sc = float(scale)  # the C float argument is static_cast<float>(scale)
+    # the C float argument is static_cast<float>(scale); the general form takes all that numpy does
+    sc = scale if type(scale) is float else float(np.float32(scale))
     with _on_device(x):
         if isinstance(params, FloatFormatDescriptor):
             st = _lib.lib.lof_virtual_round_f32(
@@ -264,6 +265,14 @@ def gemm(A: torch.Tensor, B: torch.Tensor, accum: AccumSpec, alpha: float = 1.0,
     return D
 
 
+def _alpha(scale_a, scale_b) -> float:
+    """run_scaled's 1 / (scale_a * scale_b) (cutlass_gemms.cuh:1777-1787), all in float."""
+    if type(scale_a) is float and type(scale_b) is float and scale_a == 1.0 and scale_b == 1.0:
+        return 1.0
+    denom = np.float32(scale_a) * np.float32(scale_b)
+    return 1.0 if denom == 0 else float(np.float32(1.0) / denom)
+
+
 def lof_gemm(A: torch.Tensor, B: torch.Tensor, accum_mant_bits: int,
              round_mode=RoundingMode.RoundToNearestEven, stochastic_rounding_bits: int = 0,
              scale_a: float = 1.0, scale_b: float = 1.0) -> torch.Tensor:
@@ -272,11 +281,7 @@ def lof_gemm(A: torch.Tensor, B: torch.Tensor, accum_mant_bits: int,
     reference kernel, the accumulator always rounds to nearest even: ``round_mode`` and
     ``stochastic_rounding_bits`` are accepted and ignored (cutlass_gemms.cuh:122)."""
     RoundingMode(int(round_mode))
-    if scale_a == 1.0 and scale_b == 1.0:
-        alpha = 1.0
-    else:   # run_scaled (cutlass_gemms.cuh:1777-1787), all in float
-        denom = np.float32(scale_a) * np.float32(scale_b)
-        alpha = 1.0 if denom == 0 else float(np.float32(1.0) / denom)
+    alpha = _alpha(scale_a, scale_b)
     return gemm(A, B, AccumSpec(mant_bits=int(accum_mant_bits), chunk=1), alpha=alpha)
 
 
