@@ -192,6 +192,8 @@ typedef struct lof_gemm_desc {
  *           (v_fma_mixlo_f16, one rounding of the exact sum: at chunk 1 on lanes whose
  *           products or sums are inexact in FP32, and for every chunk sum of a slice that
  *           fails the exact-sum test).
+ *   0x40000 on its own changes no leaf: like any bit above it runs the product on the wave tile
+ *           where the chunk-sum kernels would take it.
  * Chunk sums run on MFMA only where every partial sum of the chunk is exact in FP32 (chunks of
  * 8 to 32 on the bf16 MFMAs, where the slice's values are all bfloat16 values; chunks of 2
  * and 4 on the f32 MFMA), and the

@@ -137,7 +137,7 @@ LOF_API lof_status lof_conv2d_f32(const lof_conv2d_desc* desc, int32_t config,
     // testing bits as in lof_gemm_f32: 0x100 general leaf path, 0x200 every chunk on VALU,
     // 0x800 / 0x1000 / 0x2000 / 0x4000 / 0x8000 / 0x20000 the exact-sum / RTO /
     // binary16-held / packed binary16 / directed-rounding / mixed-precision FMA leaves off,
-    // 0x10000 the bf16 MFMA chunk sums off
+    // 0x10000 the bf16 MFMA chunk sums off, 0x40000 none of them
     if (config >= 0) {
         if (config & ~0xFF) g.chain = -1;   // these paths are the tiles' below
         if (config & 0x800) g.sum_off |= 1;

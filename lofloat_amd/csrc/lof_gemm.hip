@@ -415,7 +415,8 @@ LOF_API lof_status lof_gemm_f32(const lof_gemm_desc* desc, int32_t config, lof_s
     // exact-sum leaves off, 0x1000 its RTO leaves, 0x2000 its binary16-held chunk-1 leaves,
     // 0x4000 only their packed binary16 form, 0x8000 the directed-rounding chunk-1 leaves,
     // 0x10000 the bf16 MFMA chunk sums (exact chunks of 8 to 32 then use the VALU chain)
-    // -- any of them on the tiles below, which hold those paths, instead of the chunk-sum kernels
+    // -- any of them, and 0x40000 alone, on the tiles below, which hold those paths, instead of the
+    // chunk-sum kernels
     if (config >= 0 && (config & ~0xFF)) g.chain = -1;
     if (config >= 0 && (config & 0x800)) g.sum_off |= 1;
     if (config >= 0 && (config & 0x1000)) g.sum_off |= 2;
