@@ -175,17 +175,15 @@ typedef struct lof_gemm_desc {
  * < lof_gemm_num_configs() that is valid for the chunk (lof_gemm_config_valid).  Testing
  * bits OR-ed into config:
  *   0x100   forces the literal (general) leaf path;
- *   0x200   makes an MFMA config compute every chunk sum with the VALU fmaf chain;
+ *   0x200   makes a wave tile (an mfma config) compute every chunk sum with the VALU fmaf chain;
  *   0x400   makes it compute every chunk sum on MFMA without the exactness test (this one
  *           can change results);
- *   0x800   turns the MFMA configs' exact-sum leaves off;
- *   0x1000  turns their RTO leaves off;
- *   0x2000  turns their binary16-held chunk-1 leaves off;
+ *   0x800   turns its exact-sum leaves off;
+ *   0x1000  turns its RTO leaves off;
+ *   0x2000  turns its binary16-held chunk-1 leaves off;
  *   0x4000  turns off only the packed binary16 form of those leaves;
  *   0x8000  turns off the directed-rounding leaves (round-to-odd from the sum rounded down
- *           and up, for mantissa-only and binary16-shaped accumulators at chunk 1, and on
- *           the 64x64 and 64x128 wave tiles for the sums of chunks 8 to 32 into
- *           mantissa-only accumulators of 20 or more bits);
+ *           and up, for mantissa-only and binary16-shaped accumulators at chunk 1);
  *   0x10000 turns off the bf16 MFMA chunk sums (exact chunks of 8 to 32 then sum on the
  *           VALU chain; chunks of 2 and 4 always use the f32 MFMA);
  *   0x20000 turns off the mixed-precision FMA leaves of binary16-shaped accumulators
@@ -194,11 +192,13 @@ typedef struct lof_gemm_desc {
  *           fails the exact-sum test).
  *   0x40000 on its own changes no leaf: like any bit above it runs the product on the wave tile
  *           where the chunk-sum kernels would take it.
- * Chunk sums run on MFMA only where every partial sum of the chunk is exact in FP32 (chunks of
+ * Round-to-nearest-even into a mantissa-only accumulator of 1 to 23 bits or a binary16-shaped
+ * format runs on the chunk-sum kernels, whose f32 MFMAs are the fmaf chain.  On the wave tiles
+ * chunk sums run on MFMA only where every partial sum of the chunk is exact in FP32 (chunks of
  * 8 to 32 on the bf16 MFMAs, where the slice's values are all bfloat16 values; chunks of 2
- * and 4 on the f32 MFMA), and the
- * short leaves only where they provably equal the reference leaf, both checked per tile and
- * k-slice at run time, so all configs give bit-identical results.  Replaces lo_float::LoF_gemm
+ * and 4 on the f32 MFMA).  Both take the short leaves only where they provably equal the
+ * reference leaf, checked per tile and k-slice at run time, so all configs give bit-identical
+ * results.  Replaces lo_float::LoF_gemm
  * (Lof_kernel.cu:96-154) and lo_float::Gemm::operator() (cutlass_gemms.cuh:1789-1822;
  * alpha = 1/(scale_a*scale_b) per run_scaled, 1777-1787, is the caller's job). */
 LOF_API lof_status lof_gemm_f32(const lof_gemm_desc* desc, int32_t config, lof_stream_t stream);
@@ -211,11 +211,12 @@ LOF_API int32_t lof_gemm_config_valid(int32_t config, int32_t chunk);
 /* Writes a short "BMxBN/TMxTN" style name of the tile (mfma21: a wave tile of 128 x 64); returns
  * LOF_ERR_INVALID_ARGUMENT if out of range.  The short tiles mfma32x32, mfma16x64, mfma64x16 and
  * mfma16x16 exist for round-to-nearest-even mantissa-only accumulators of 1 to 23 bits and
- * binary16-shaped formats; other products, and the first three at chunk 2, run 64 x 64 instead. */
+ * binary16-shaped formats; other products, and the first three at chunk 2, run 64 x 64 instead,
+ * and mfma16x16 runs 32 x 32 for fewer than 4 k or 4 rows of an operand stored k-major. */
 LOF_API lof_status lof_gemm_config_name(int32_t config, char* buf, int32_t buflen);
 
-/* Autotuner: times the candidate tile configs on this problem -- the wave tiles for chunks
- * they take, else the VALU tiles -- (desc->D is overwritten; C and beta are
+/* Autotuner: times the candidate tile configs on this problem -- the chunk-sum kernels' tiles
+ * where they run, else the wave tiles for chunks they take, else the VALU tiles -- (desc->D is overwritten; C and beta are
  * not used, and a C that overlaps D is rejected with LOF_ERR_INVALID_ARGUMENT), records the
  * winner for problems of the same shape class and accumulator (kind, mantissa bits, format
  * bias, chunk) and returns it.  The operands' values are not part of the key. */
@@ -233,8 +234,8 @@ LOF_API lof_status lof_gemm_autotune(const lof_gemm_desc* desc, int32_t iters,
  *   LOF_CONV_NHWC: x N x H x W x C, w K x R x S x C (KRSC), y and c N x P x Q x K; the
  *     reduction index is (r, s, c) with c fastest.
  * Each output is the ascending-k leaf chain of lof_gemm_f32 over its reduction.  Convolutions
- * run on two wave tiles, configs 7 (64 x 64) and 6 (128 x 64) (others return
- * LOF_ERR_UNSUPPORTED), with chunk in {1, 2, 4, 8, 16, 32}; x must have fewer than 2^30
+ * take configs 7 (64 x 64, on the chunk-sum kernels where they run, else a wave tile) and 6 (the
+ * 128 x 64 wave tile) (others return LOF_ERR_UNSUPPORTED), with chunk in {1, 2, 4, 8, 16, 32}; x must have fewer than 2^30
  * elements.
  * ------------------------------------------------------------------------------- */
 enum { LOF_CONV_NCHW = 0, LOF_CONV_NHWC = 1 };
@@ -253,7 +254,7 @@ typedef struct lof_conv2d_desc {
     float beta;
 } lof_conv2d_desc;
 
-/* y = alpha * conv(x, w) [+ beta * c].  config: -1 for the default wave tile, else 6 or 7,
+/* y = alpha * conv(x, w) [+ beta * c].  config: -1 for the default tile, else 6 or 7,
  * with lof_gemm_f32's testing bits.  Replaces lo_float::LoF_conv2d
  * (Lof_kernel.cu:156-228; NCHW/OIHW, alpha = 1 / (weight_scale * input_scale), beta = 0)
  * and lo_float::Conv2d::operator() (cutlass_conv.cuh:118-181; NHWC/KRSC).  The reference's
@@ -294,7 +295,8 @@ typedef struct lof_group_item {
 typedef struct lof_grouped lof_grouped;
 
 /* Validate the items and upload the work list.  config: -1 = default (or the tuned
- * choice from lof_grouped_autotune), else < lof_grouped_num_configs().  A GEMM item with
+ * choice from lof_grouped_autotune, unless it is the chunk-sum kernels' and the list has chunk sums
+ * that they do not take), else < lof_grouped_num_configs().  A GEMM item with
  * at least as many tiles as the persistent grid has workgroups fills the device by itself:
  * lof_grouped_run launches it through the single-GEMM kernel (whose tile is faster than
  * the combined kernel's) ahead of the persistent launch that runs every other item.  The

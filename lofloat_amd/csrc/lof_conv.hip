@@ -33,8 +33,7 @@ void k_conv_mfma(GemmArgs g) {
 
 using ConvKernel = void (*)(GemmArgs);
 
-// [tile][log2 chunk][subn]: tile 0 = 64 x 64 (mfma11), tile 1 = 128 x 64 (mfma21), the two
-// wave tiles the GEMM's default choice uses.
+// [tile][log2 chunk][subn]: tile 0 = 64 x 64 (mfma11), tile 1 = 128 x 64 (mfma21)
 #define LOF_CONV_PAIR(WMB, C) {k_conv_mfma<WMB, 1, C, false>, k_conv_mfma<WMB, 1, C, true>}
 #define LOF_CONV_TILE(WMB)                                                                 \
     {LOF_CONV_PAIR(WMB, 1), LOF_CONV_PAIR(WMB, 2), LOF_CONV_PAIR(WMB, 4),                  \
@@ -122,7 +121,7 @@ LOF_API lof_status lof_conv2d_f32(const lof_conv2d_desc* desc, int32_t config,
                          "{1, 2, 4, 8, 16, 32} (got %d)", what, g.chunk);
     int tile;   // 0: 64 x 64, 1: 128 x 64
     const int cfg = config >= 0 ? (config & 0xFF) : -1;
-    if (cfg < 0) {   // the GEMM's default rule: 128 x 64 for long chunks with >= 384 tiles
+    if (cfg < 0) {   // 128 x 64 for long chunks with >= 384 tiles
         const int64_t tiles_128x64 = ((int64_t)c.K + 127) / 128 * ((Ncols + 63) / 64);
         tile = (g.chunk >= 16 && tiles_128x64 >= 384) ? 1 : 0;
     } else if (cfg == kCfgMfma11) {

@@ -62,7 +62,8 @@ enum ChainKind : int { kChainMant = 0, kChainMant23 = 1, kChainHalf = 2, kChainM
 // start PAD floats apart, the row swizzled by k.  An MFMA operand read takes KI consecutive k of
 // 64 / KI consecutive rows each; the swizzle puts them in different banks (64 banks of 4
 // bytes), and PAD spreads the transposing stores of a row-major operand, whose lanes hold
-// consecutive groups of four k.  (Rows of R + 4 floats: every operand read had two-way conflicts.)
+// consecutive groups of four k, to two-way conflicts.  (Rows of R + 4 floats: every operand read had
+// them.  4096^3, chunk 32, both operands row-major: 67 M conflict cycles of 268 M LDS ones, two a store.)
 template <int R, int BK, int KI>
 struct ChainLds {
     static constexpr int PAD = R >= 64 && KI == 2 ? 8 : 4;
@@ -791,7 +792,8 @@ __device__ __forceinline__ void gemm_tile_chain(const GemmArgs& g, int tile_m, i
 #pragma unroll
                 for (int it = 0; it < NV; ++it) *(float4*)(d + it * (256 / R) * L::GROUP) = v[it];
             } else {      // 4 k of a row, 1024 / BK (at most 32) rows further each time
-                // MFMA kinds' rows lie at least 32 apart, past the swizzle
+                // The thread's own row, below that step, shares no bit with it or with the swizzle
+                // (a multiple of 32 where the step is 32 rows, of 16 where it is 16 or 8): it is added.
                 float* d = S + (tid % (BK / 4)) * L::GROUP + (kPack ? 0 : tid / (BK / 4));
 #pragma unroll
                 for (int it = 0; it < NV; ++it) {

@@ -24,6 +24,11 @@
 // A[l % 32][l / 32] and B[l / 32][l % 32]; result register r of lane l is
 // D[8 * (r / 4) + 4 * (l / 32) + r % 4][l % 32].
 //
+// What runs here: accumulators and modes that the chunk-sum kernels (lof_gemm_chain.hpp) do not take;
+// mantissa-only ones at chunk 1, 10 and 23 bits aside, in large products; the grouped launch's configs
+// 0 to 7; and, for the accumulators that those kernels do take, configs mfma21 and mfma12 (mfma22 at
+// chunk 1), testing bits, and rows more than 2^25 floats apart.
+//
 // Pipelining: the next K slice is loaded from HBM into registers while the current slice
 // computes from one LDS buffer, then stored to the other (one barrier per slice); interior
 // slices use float4 loads.  The chunk length is a template parameter so a chunk's LDS reads
@@ -394,7 +399,6 @@ __device__ __forceinline__ void rto_fma16(const float* a, float b, float* acc) {
 // virtual_round, lo_float.h:2716-2756) or, F16, the binary16 conversion (a binary16-shaped
 // format, for sums the caller has bounded below 2^15).  M23: a 23-bit accumulator, whose round()
 // keeps every float: RTO24 alone, 4 instructions a leaf against 7.
-// (Forward and both gradients of a 2048 x 1024 -> 4096 layer on FP32 operands: 6.64 -> 3.26 ms.)
 template <bool F16, bool M23 = false>
 __device__ __forceinline__ void leaves_dr16(const float (&a)[16], float b, float (&acc)[16],
                                             const GemmArgs& g) {
